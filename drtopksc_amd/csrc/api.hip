@@ -72,6 +72,13 @@ struct Plan {
     u64 npart, o_part;  // beta path: per-workgroup records of the concatenation
     u64 o_dvals, o_doff, o_sel, o_skeys, o_sidx, total;
     u64 npad1, npad2, o_bufA, o_bufB, o_dsel;  // bitonic family
+    bool own_config;   // the library's choice of alpha with the reference's final options
+};
+
+// The short pipeline's parameters and layout inside a workspace of the plan's size.
+struct ShortPlan {
+    int alpha, f1, f2;
+    u64 o_dvals, o_sup1, o_sup2, o_sel, o_hist, o_cnt, o_max, o_skeys, o_sidx;
 };
 
 #include "single_tuning.inc"
@@ -154,6 +161,8 @@ drtopk_status resolve(drtopk_algo algo, drtopk_dtype dtype, u64 n, u64 k, const 
     pl->n = n; pl->k = k;
     pl->alpha = alpha; pl->beta = beta; pl->path = path; pl->nb = nb; pl->B = p->num_buckets;
     pl->flags = p->flags;
+    pl->own_config = p->alpha < 0 && nb == 8 && p->num_buckets == 256 && p->beta == 2 &&
+                     (p->flags & ~DRTOPK_FLAG_TIMING) == DRTOPK_FLAGS_DEFAULT;
     pl->L = 1ull << alpha;
     pl->S = alpha ? cdiv(n, pl->L) : 0;
     pl->D = (u64)beta * pl->S;
@@ -199,6 +208,64 @@ drtopk_status resolve(drtopk_algo algo, drtopk_dtype dtype, u64 n, u64 k, const 
     pl->o_dsel = o; o = align_up(o + (bit && path ? 8ull * k : 0), 256);
     pl->total = o;
     return DRTOPK_OK;
+}
+
+// Whether the short pipeline (short.hip) serves this call, and with which subranges.  Calls that
+// set alpha, beta, digits, buckets or options ask for that very pipeline, and so do calls with
+// stats (they report the general pipeline's intermediate results): those keep it.
+//  - Subranges: the first top-k reads its delegates with one workgroup while the concatenation's
+//    reads spread over the chip, so alpha is as large as leaves 4 delegates per selected one
+//    (the threshold then lets 1.15 k random keys through; 1.39 k with 2) and at least 4096.
+//  - The concatenation holds up to k << alpha keys; alpha is lowered until the layout fits the
+//    workspace that drtopk_workspace_size returns.
+//  - More delegates than one selection holds are selected in two or three levels, their maxima
+//    over ranges first: the levels that cost the fewest cycles, about 0.6 per value and 9000 per
+//    level measured, twice that when their lists do not fit LDS.  A level
+//    needs 2k ranges for the same reason as the delegates.
+bool short_plan(const Plan& pl, ShortPlan* sp) {
+    if (!pl.own_config || pl.algo == DRTOPK_ALGO_BITONIC || pl.n <= SMALL_N || pl.k > SHORT_KMAX) return false;
+    const u64 k = pl.k;
+    int a0 = std::min(16, floor_log2(pl.n / std::max<u64>(4 * k, 4096)));
+    if (cdiv(pl.n, 1ull << a0) > SMALL_N && cdiv(pl.n, 2ull << a0) >= 2 * k) ++a0;  // one level is quicker
+    for (int a = a0; a >= 2; --a) {
+        const u64 S = cdiv(pl.n, 1ull << a), V = k << a;
+        if (S < 2 * k || short_segments(V) > SHORT_SEGS) continue;
+        int f1 = 0, f2 = 0;
+        if (S > SMALL_N) {
+            double best = 0;
+            for (int x = 2; x <= 8; ++x)
+                for (int y = 0; x + y <= 8; y = y ? y + 1 : 2) {
+                    const u64 top = cdiv(S, 1ull << (x + y));
+                    if (top > SMALL_N || top < 2 * k || (k << x) > SMALL_N || (k << y) > SMALL_N) continue;
+                    const bool lds = std::max(top, std::max(k << x, y ? k << y : 0)) <= SHORT_LISTED && k <= SHORT_LISTED / 5;
+                    const double c = 0.6 * (double)(top + (k << x) + (y ? k << y : 0)) + (lds ? 9000.0 : 18000.0) * (y ? 3 : 2);
+                    if (!f1 || c < best) {
+                        best = c;
+                        f1 = x;
+                        f2 = y;
+                    }
+                }
+            if (!f1) continue;
+        }
+        const u64 ns = short_segments(V), S1 = cdiv(S, 1ull << f1);
+        sp->alpha = a;
+        sp->f1 = f1;
+        sp->f2 = f2;
+        u64 o = align_up(sizeof(Ctrl), 256);
+        sp->o_dvals = o; o = align_up(o + 4 * S, 256);
+        sp->o_sel = o; o = align_up(o + 4 * k, 256);
+        sp->o_hist = o; o = align_up(o + 4 * 2048, 256);
+        sp->o_cnt = o; o = align_up(o + 4 * ns, 256);
+        sp->o_max = o; o = align_up(o + 4 * ns, 256);
+        sp->o_skeys = o; o = align_up(o + 4 * 4096 * ns, 256);
+        sp->o_sidx = o; o = align_up(o + 4 * 4096 * ns, 256);
+        // the maxima are dead once the concatenation is written: they share its indices' area
+        sp->o_sup1 = sp->o_sidx;
+        sp->o_sup2 = align_up(sp->o_sup1 + (f1 ? 4 * S1 : 0), 256);
+        o = std::max(o, align_up(sp->o_sup2 + (f2 ? 4 * cdiv(S1, 1ull << f2) : 0), 256));
+        if (o <= pl.total) return true;
+    }
+    return false;
 }
 
 SelState make_sel(int mode, u64 m, u64 k, int nb, int B, int stop_digit, int stop_on_one, int max_passes) {
@@ -264,6 +331,32 @@ drtopk_status select_impl(const Plan& pl, const void* d_keys, void* d_workspace,
     hipStream_t st = (hipStream_t)stream;
     char* ws = (char*)d_workspace;
     Ctrl* ctrl = (Ctrl*)(ws + pl.o_ctrl);
+    if (!h_stats && pl.own_config && pl.algo != DRTOPK_ALGO_BITONIC &&
+        g_test_segcap.load(std::memory_order_relaxed) == 0) {
+        ShortArgs sa{};
+        sa.keys = (const u32*)d_keys;
+        sa.n = pl.n; sa.k = pl.k; sa.f32 = pl.f32; sa.ctrl = ctrl;
+        sa.out_keys = d_topk_keys; sa.out_idx = (i64*)d_topk_idx; sa.d_kth = d_kth;
+        if (pl.n <= SMALL_N) {
+            HIPCHK(launch_small(sa, st));
+            return DRTOPK_OK;
+        }
+        ShortPlan sp;
+        if (short_plan(pl, &sp)) {
+            sa.alpha = sp.alpha; sa.f1 = sp.f1; sa.f2 = sp.f2;
+            sa.dvals = (u32*)(ws + sp.o_dvals);
+            sa.sup1 = (u32*)(ws + sp.o_sup1);
+            sa.sup2 = (u32*)(ws + sp.o_sup2);
+            sa.sel_ids = (u32*)(ws + sp.o_sel);
+            sa.ghist = (u32*)(ws + sp.o_hist);
+            sa.cnt = (u32*)(ws + sp.o_cnt);
+            sa.segmax = (u32*)(ws + sp.o_max);
+            sa.skeys = (u32*)(ws + sp.o_skeys);
+            sa.sidx = (u32*)(ws + sp.o_sidx);
+            HIPCHK(launch_short(sa, st));
+            return DRTOPK_OK;
+        }
+    }
     u32* hist = (u32*)(ws + pl.o_hist);
     u64* rcnt = (u64*)(ws + pl.o_rcnt);
     u64* roff = (u64*)(ws + pl.o_roff);

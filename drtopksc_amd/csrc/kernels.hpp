@@ -148,6 +148,37 @@ constexpr u64 DIRECT_TILE = 16384;
 hipError_t launch_extract(const ExtractArgs& a, hipStream_t st);
 hipError_t launch_finalize(SelState* sel, Ctrl* ctrl, int f32, void* d_kth, u64 k, hipStream_t st);
 
+// short.hip ---------------------------------------------------------------------------
+// One-workgroup selections: the whole top-k (launch_small, n <= SMALL_N), or delegate pass ->
+// first top-k -> concatenation -> second top-k and outputs in four or five launches.
+constexpr u32 SMALL_N = 36864;     // keys, or values of one selection, that one workgroup holds in LDS
+constexpr u32 SHORT_KMAX = 8192;   // largest k of launch_short
+constexpr u32 SHORT_LISTED = 20480;  // values a level may have for its lists to stay in LDS, with k <= 4096
+constexpr u32 SHORT_SEGS = 4096;   // most concatenation segments it reads
+struct ShortArgs {
+    const u32* keys;   // 16-byte aligned
+    u64 n, k;
+    int alpha, f32;    // alpha >= 2
+    int f1, f2;        // log2 of the delegates per range of the first top-k's second level, and of
+                       // those ranges per range of the third (0: no such level; f1 + f2 <= 8)
+    Ctrl* ctrl;
+    u32* dvals;        // [S] delegates, padded to 16 bytes
+    u32* sup1;         // maxima of every 2^f1 delegates, padded to 16 bytes
+    u32* sup2;         // maxima of every 2^f2 of those
+    u32* sel_ids;      // [k]
+    u32* ghist;        // [2048]
+    u32* skeys;        // concatenation: short_segments x 4096 keys
+    u32* sidx;         // and indices
+    u32* cnt;          // [short_segments]
+    u32* segmax;       // [short_segments]
+    void* out_keys;
+    i64* out_idx;
+    void* d_kth;
+};
+hipError_t launch_small(const ShortArgs& a, hipStream_t st);
+hipError_t launch_short(const ShortArgs& a, hipStream_t st);
+u32 short_segments(u64 V);         // concatenation segments of V = k << alpha slots
+
 // bitonic.hip ---------------------------------------------------------------------------
 // Bitonic family: first top-k over the delegates, whole-subrange concatenation, second
 // top-k, index-ordered outputs.  alpha == 0: one top-k over V.
