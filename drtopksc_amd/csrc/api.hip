@@ -268,6 +268,84 @@ bool short_plan(const Plan& pl, ShortPlan* sp) {
     return false;
 }
 
+// Whether the filter pipeline (filter.hip) serves a call that the short pipeline leaves: k large
+// enough that a sample places it.  m samples hold r = k m / n of the top k keys on average; rank
+// r + 7 sqrt(r) + 12 bounds the k-th key from below with a probability of failure below 1e-12, and
+// r >= 30 keeps it below the largest sample with the same certainty.  m is the smallest of 2^15, 2^17,
+// 2^19 that does; from 2^27 keys on at least 2^17, so that the k-th key's class (about n / m keys)
+// stays small; 2^13 below 2^26 keys where that holds 30, as one workgroup selects from the sample
+// (2^15: 18 us, 2^13: 12 us) and the keys kept in vain cost less.
+//  Where the lines lie (general pipeline -> this one, us, uniform uint32 / normal float32):
+//  below k = n / 16384 the delegates' bound is the better one (2^30, 2^14: 748 -> about 760);
+//  2^30: k 2^16 793 -> 753 / 790 -> 759, 2^20 949 -> 788, 2^22 1020 -> 862, 2^28 5450 -> 3780;
+//  2^26: k 2^18 123 -> 105 / 134 -> 111;  2^24: k 2^16 67 -> 63 / 78 -> 66, 2^22 131 -> 130;
+//  2^22: k n/8 63 -> 58, n/4 75 -> 76;  2^20: k n/16 55 -> 47 / 67 -> 49, n/4 60 -> 62, hence n / 8 there.
+//  Clustered keys gain more, as the passes over them here don't depend on the distribution:
+//  2^24 lognormal keys, k 2^16: 148 -> 50.
+//  Kept keys: about n r' / m.  Each wave of the pass has a segment of its own, and a pool takes the
+// units that find it full (clustered keys); both have to fit the workspace.
+bool filter_plan(const Plan& pl, FilterArgs* fa, char* ws) {
+    const u64 n = pl.n, k = pl.k;
+    if (!pl.own_config || pl.algo == DRTOPK_ALGO_BITONIC || n <= SMALL_N ||
+        k > n / (n < (1ull << 24) ? 8 : 4) || filter_units(n) > F_RANGES * F_RUNITS)
+        return false;
+    for (int lm = n >= (1ull << 27) ? 17 : 15; lm <= 19 && (n >> lm) >= 1; lm += 2) {
+        double r = (double)k * (double)(1ull << lm) / (double)n;
+        if (r < 30) continue;
+        if (lm == 15 && r >= 120 && n < (1ull << 26)) {
+            lm = 13;
+            r /= 4;
+        }
+        if (lm == 17 && r > 8192) {  // too many samples above the bound for one workgroup's list
+            lm = 15;
+            r /= 4;
+        }
+        const double d = 4 * std::sqrt(r) + 4;
+        const u32 rp = (u32)std::ceil(r + 7 * std::sqrt(r) + 12), rhi = (u32)std::ceil(r + d);
+        const u32 rlo = r > d ? (u32)(r - d) : 0u;
+        const double per = (double)n / (double)(1ull << lm);  // keys per sample
+        const u64 kept = (u64)(per * rp), units = filter_units(n);
+        const u64 cls = (u64)(per * std::max(1.0, (rhi - rlo) / 254.0)) + 1;
+        const u64 lcap = std::min<u64>(std::max<u64>(4096, cls) + 2048, 64 + 4 * cls + n / 512);
+        u64 o = align_up(sizeof(Ctrl), 256);
+        auto take = [&](u64 bytes) {
+            const u64 at = o;
+            o = align_up(o + bytes, 256);
+            return ws + at;
+        };
+        fa->state = take(filter_state_bytes());
+        fa->cnt = (u32*)take(4 * units);
+        fa->base = (u32*)take(4 * units);
+        fa->rg = (u32*)take(4 * F_RANGES);
+        fa->rq = (u32*)take(4 * F_RANGES);
+        fa->lkey = (u32*)take(4 * 64 * lcap);
+        fa->lrange = (u32*)take(4 * 64 * lcap);
+        if (o + 4096 > pl.total) return false;
+        // a wave's segment holds what its units keep; in a workspace with a slot per key, all of them
+        const u64 room = (pl.total - o) / 8 & ~3ull, waves = 4 * filter_grid(n).grid;
+        const u64 most = cdiv(cdiv(units, 4), filter_grid(n).grid) * F_UNIT + 8 * F_UNIT;  // keys of a wave
+        u64 pool = 0;
+        if (room < waves * most) {
+            pool = (u64)(1.6 * (double)kept) + 8 * F_UNIT;
+            if (pool > room || (room - pool) / waves < kept * 3 / 2 / waves + 64) return false;
+        }
+        fa->wcap = (u32)std::min<u64>(most, (room - pool) / waves);
+        fa->pool_cap = (u32)pool;
+        if (room < (1ull << lm) + (1ull << 14)) return false;
+        fa->skeys = (u32*)(ws + o);
+        fa->sidx = fa->skeys + room;
+        fa->sample = fa->skeys;  // dead once the keys are filtered
+        fa->lm = lm;
+        fa->kept = kept;
+        fa->rp = rp;
+        fa->rlo = rlo;
+        fa->rhi = rhi;
+        fa->lcap = (u32)lcap;
+        return true;
+    }
+    return false;
+}
+
 SelState make_sel(int mode, u64 m, u64 k, int nb, int B, int stop_digit, int stop_on_one, int max_passes) {
     SelState s;
     std::memset(&s, 0, sizeof(s));
@@ -354,6 +432,13 @@ drtopk_status select_impl(const Plan& pl, const void* d_keys, void* d_workspace,
             sa.skeys = (u32*)(ws + sp.o_skeys);
             sa.sidx = (u32*)(ws + sp.o_sidx);
             HIPCHK(launch_short(sa, st));
+            return DRTOPK_OK;
+        }
+        FilterArgs fa{};
+        if (filter_plan(pl, &fa, ws)) {
+            fa.keys = sa.keys; fa.n = pl.n; fa.k = pl.k; fa.f32 = pl.f32; fa.ctrl = ctrl;
+            fa.out_keys = d_topk_keys; fa.out_idx = (i64*)d_topk_idx; fa.d_kth = d_kth;
+            HIPCHK(launch_filter(fa, st));
             return DRTOPK_OK;
         }
     }

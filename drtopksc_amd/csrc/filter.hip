@@ -1,0 +1,967 @@
+// filter.hip -- top-k of one vector for large k in six launches: a sample bounds the k-th key from
+// below, one pass over the keys keeps those above the bound, and the selection runs on them.
+//
+// The delegate scheme pays for large k twice: its delegate stores (0.4 GB beside 4 GB of keys at
+// 2^30, k = 2^24) and a concatenation that reads most subranges again.  Here the keys are read
+// once and about 1.1 .. 2.6 k of them written.
+//
+//  k_fsample  m pseudo-random keys, one from each of m equal strata.
+//  k_fsplit   t, the r'-th largest sample, with r' = r + 7 sqrt(r) + 12 above the expected rank
+//             r = k m / n: fewer than k keys reach t with a probability below 1e-12 (the positions
+//             do not depend on the keys).  Up to 254 samples of ranks r -+ (4 sqrt(r) + 4)
+//             become splitters.
+//  k_filter   keys > t with their indices, in index order, per unit of 2048 keys; how many
+//             equal t (counted, never stored: any number of ties at t costs nothing); and the
+//             exact counts between and at the splitters.
+//  k_fpick    the kept keys of the k-th key's class, and per range of units how many lie above it.
+//  k_fkth     the k-th key, and where each range's outputs start.
+//  k_fwrite   the outputs in index order; ties at t are read from the keys again.
+//
+// At 2^30 keys, k = 2^22, the six take 7 + 34 + 765 + 38 + 35 + 48 us (1028 us for the general
+// pipeline, 862 for the call); the read alone takes 630.  At 2^24 keys, k = 2^16: 3 + 9 + 21 + 8 + 14 + 5 us
+// (67 and 63 for the calls): there the launches, and the chains of round trips in the two
+// one-workgroup kernels, are most of it.
+//
+// Should the bound fail after all, or a buffer not hold what it was sized for, k_fkth selects from
+// the keys themselves with its one workgroup: slow, but exact.
+#include <algorithm>
+
+#include "common.hpp"
+#include "kernels.hpp"
+#include "wgselect.hpp"
+
+namespace drtopk {
+
+constexpr int FS_NT = 1024;
+constexpr u32 F_CLASSES = 512;  // 2b: between splitters b-1 and b; 2b+1: equal to splitter b; 511: above the window
+constexpr u32 F_ABOVE = F_CLASSES - 1;
+constexpr u32 F_SPLIT = 254;  // so that no splitter's class is 511
+constexpr int F_REPS = 4;         // replicas of the class counters
+constexpr u32 F_SORT = 512;       // samples above the bound that are put in order at once
+constexpr u32 F_STAGE = 512;    // kept keys a wave stages in LDS
+constexpr u32 F_LISTS = 64;     // sublists of the class, so that their cursors do not serialise
+constexpr u32 F_BATCH = WG * 8; // kept keys a workgroup takes at a time in k_fpick and k_fwrite
+
+enum : u32 { F_CLASS = 0, F_AT_T = 1, F_DONE = 2 };
+
+struct FilterState {
+    u32 t, up, q;      // bound, upper end of the window, splitters
+    u32 pool;          // entries taken from the spill pool
+    u32 fail;          // a buffer was too small
+    u32 K, gt, ties;   // the k-th key, keys above it, ties taken
+    u32 kind;          // F_CLASS, F_AT_T (K == t), F_DONE (outputs written by k_fkth)
+    u32 pad[7];
+    u32 lcount[F_LISTS];
+    u32 split[256];    // ascending, 0xFFFFFFFF past q
+};
+size_t filter_state_bytes() { return sizeof(FilterState) + 4ull * F_REPS * F_CLASSES; }
+
+// ---------------------------------------------------------------- sample
+// Sample i is a key of stratum [i n / m, (i + 1) n / m).
+__host__ __device__ __forceinline__ u32 sample_pos(u32 i, u64 n, int lm) {
+    const u32 b = (u32)(((u64)i * n) >> lm), e = (u32)(((u64)(i + 1) * n) >> lm);
+    u32 h = i * 0x9E3779B1u;
+    h ^= h >> 15;
+    h *= 0x85EBCA77u;
+    h ^= h >> 13;
+    h *= 0xC2B2AE3Du;
+    h ^= h >> 16;
+    return b + (u32)(((u64)h * (e - b)) >> 32);
+}
+
+template <class K>
+__global__ __launch_bounds__(WG) void k_fsample(const u32* __restrict__ keys, u64 n, int lm, u32* __restrict__ sample,
+                                                u32* __restrict__ sup, Ctrl* ctrl, FilterState* st,
+                                                u32* __restrict__ cls) {
+    const u32 g = blockIdx.x * WG + threadIdx.x;  // 2^lm / 4 threads, at least 2048
+    u32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = keys[sample_pos(4 * g + j, n, lm)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = K::to_ord(v[j]);
+    *(u32x4*)(sample + 4 * g) = v;
+    if (lm > 15) {  // the maxima of every 8 (2^17 samples) or 32 (2^19) of them
+        const int lanes = lm == 17 ? 2 : 8;
+        const u32 m = row_max_u32(max4(v), lanes);
+        if ((threadIdx.x & (lanes - 1)) == 0) sup[g / lanes] = m;
+    }
+    static_assert(F_REPS * F_CLASSES <= 2048 && sizeof(FilterState) / 4 <= 2048, "one counter per thread");
+    if (g < F_REPS * F_CLASSES) cls[g] = 0;
+    if (g < sizeof(FilterState) / 4) ((u32*)st)[g] = 0;
+    if (g == 0) ws_head_begin(&ctrl->head);
+}
+
+// ---------------------------------------------------------------- bound and splitters
+// LM 13, 15: the 2^LM samples in LDS.  Otherwise LG = LM - 14: 2^14 maxima of 2^LG samples each: their r'-th largest T0 is
+// a lower bound of the samples', and those above it, 1.1 .. 1.4 r' for random samples, are all in
+// ranges whose maximum exceeds T0.  The samples above T0 are listed in LDS and the bounds taken there.
+template <int LM>
+__global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample, const u32* __restrict__ sup, u32 rp,
+                                                  u32 rlo, u32 rhi, FilterState* st) {
+    constexpr int LG = LM > 15 ? LM - 14 : 0;
+    constexpr u32 HELD = LG ? 16384 : 1u << LM;
+    __shared__ WgSel<FS_NT> L;
+    __shared__ __align__(16) u32 el[wg_words<FS_NT>(HELD)];
+    __shared__ __align__(16) u32 own_list[LG ? F_LIST_LDS : 1];
+    __shared__ __align__(16) u32 srt[F_SORT];
+    u32* list = LG ? own_list : el;
+    const int t = threadIdx.x;
+    wg_init<FS_NT>(L);
+    constexpr int ni = HELD / (4 * FS_NT);
+    wg_stage<FS_NT>(el, ni, [&](u32 e) { return *(const u32x4*)((LG ? sup : sample) + e); });
+    u32 gt;
+    const u32 T0 = wg_kth<FS_NT>([&](auto&& f) { wg_each(el, ni, f); }, rp, L, &gt);
+    u32 hi = L.hi;
+    if (t == 0) L.misc[8] = 0;
+    __syncthreads();
+    if constexpr (LG == 0) {  // from the samples again: the list takes their place in LDS
+#pragma unroll 8
+        for (u32 e = 4 * t; e < HELD; e += 4 * FS_NT) {
+            const u32x4 x = *(const u32x4*)(sample + e);
+            if (max4(x) > T0) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (x[j] > T0) list[atomicAdd(&L.misc[8], 1u)] = x[j];
+            }
+        }
+    } else {
+        u32 e = t * ni * 4;
+        wg_each(el, ni, [&](const u32x4& m) {
+#pragma unroll
+            for (u32 j = 0; j < 4; ++j) {
+                if (m[j] <= T0) continue;
+                u32x4 x[(1 << LG) / 4];
+#pragma unroll
+                for (int i = 0; i < (1 << LG) / 4; ++i) x[i] = *(const u32x4*)(sample + ((e + j) << LG) + 4 * i);
+#pragma unroll
+                for (int i = 0; i < (1 << LG); ++i)
+                    if (x[i / 4][i % 4] > T0) {
+                        const u32 p = atomicAdd(&L.misc[8], 1u);
+                        if (p < F_LIST_LDS) list[p] = x[i / 4][i % 4];
+                    }
+            }
+            e += 4;
+        });
+    }
+    __syncthreads();
+    const u32 nl = LG ? min(L.misc[8], F_LIST_LDS) : L.misc[8];
+    const bool all = nl == L.misc[8];  // else (tied or clustered samples) T0 is the bound, and any listed sample a splitter
+    auto each = [&](auto&& f) {
+        for (u32 i = t; i < nl; i += FS_NT) f(u32x4{list[i], 0, 0, 0});
+    };
+    if (all && nl <= F_SORT) {
+        // few: all in descending order, two threads comparing one of them with half of the others.  At
+        // 2^15 samples and 220 in the list this takes the place of two selections and a sort.
+        if (t < 4 && nl + t < F_SORT) list[nl + t] = 0;
+        if (t == 0) {
+            L.misc[9] = 1;
+            L.misc[10] = 0;
+        }
+        __syncthreads();
+        const u32 c = (u32)t >> 1, x = c < nl ? list[c] : 0u;
+        u32 rank = 0;
+        for (u32 j = 4 * ((u32)t & 1); j < nl; j += 8) {
+            const u32x4 y = *(const u32x4*)(list + j);
+#pragma unroll
+            for (u32 i = 0; i < 4; ++i) rank += j + i < nl && (y[i] > x || (y[i] == x && j + i < c)) ? 1u : 0u;
+        }
+        rank += (u32)__builtin_amdgcn_mov_dpp((int)rank, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
+        if ((t & 1) == 0 && c < nl) srt[rank] = x;
+        __syncthreads();
+        const u32 T = nl >= rp ? srt[rp - 1] : T0, tw = nl >= rhi ? srt[rhi - 1] : T;
+        const u32 up = rlo >= 1 && nl >= rlo ? srt[rlo - 1] : hi;
+        // the window's samples are consecutive: [misc 9, misc 10)
+        if ((u32)t < nl) {
+            auto in = [&](u32 y) { return y > T && y >= tw && y <= up; };
+            if (in(srt[t]) && (t == 0 || !in(srt[t - 1]))) L.misc[9] = t + 1;
+            if (in(srt[t]) && ((u32)t + 1 == nl || !in(srt[t + 1]))) L.misc[10] = t + 1;
+        }
+        __syncthreads();
+        const u32 first = L.misc[9] - 1, q = min(L.misc[10] > first ? L.misc[10] - first : 0u, F_SPLIT);
+        if (t < 256) st->split[t] = (u32)t < q ? srt[first + q - 1 - t] : 0xFFFFFFFFu;
+        if (t == 0) {
+            st->t = T;
+            st->up = up;
+            st->q = q;
+        }
+        return;
+    }
+    __syncthreads();
+    // the bound t; the window (tw, up] that almost surely holds the k-th key, where the splitters lie
+    u32 T = T0, tw = T0, up = hi;
+    if (all && nl >= rp) T = tw = wg_kth_between<FS_NT>(each, T0, hi, rp, L, &gt);
+    __syncthreads();
+    if (all && nl >= rhi) tw = wg_kth_between<FS_NT>(each, T, hi, rhi, L, &gt);
+    __syncthreads();
+    if (all && rlo >= 1 && nl >= rlo) up = wg_kth_between<FS_NT>(each, tw, hi, rlo, L, &gt);
+    __syncthreads();
+    // splitters: the samples of the window (any 254 of them), in order
+    if (t == 0) L.misc[8] = 0;
+    __syncthreads();
+    for (u32 i = t; i < nl; i += FS_NT) {
+        const u32 x = list[i];
+        if (x > T && x >= tw && x <= up) {
+            const u32 p = atomicAdd(&L.misc[8], 1u);
+            if (p < F_SPLIT) L.cand[p] = x;
+        }
+    }
+    __syncthreads();
+    const u32 q = min(L.misc[8], F_SPLIT);
+    {  // the rank of each, four threads comparing it with a quarter of the others
+        const u32 c = (u32)t >> 2, x = L.cand[c];
+        u32 rank = 0;
+        for (u32 j = 4 * ((u32)t & 3); j < q; j += 16) {
+            const u32x4 y = *(const u32x4*)(L.cand + j);
+#pragma unroll
+            for (u32 i = 0; i < 4; ++i) rank += j + i < q && (y[i] < x || (y[i] == x && j + i < c)) ? 1u : 0u;
+        }
+        rank += (u32)__builtin_amdgcn_mov_dpp((int)rank, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
+        rank += (u32)__builtin_amdgcn_mov_dpp((int)rank, 0x4E, 0xF, 0xF, false);  // quad_perm 2,3,0,1
+        if ((t & 3) == 0) st->split[c < q ? rank : c] = c < q ? x : 0xFFFFFFFFu;
+    }
+    if (t == 0) {
+        st->t = T;
+        st->up = up;
+        st->q = q;
+    }
+}
+
+// ---------------------------------------------------------------- filter
+// Class of a kept key x <= up: splitters below it, and whether it equals the next one.
+__device__ __forceinline__ u32 class_of(const u32* sp, u32 x) {
+    u32 lo = 0;
+#pragma unroll
+    for (u32 step = 128; step; step >>= 1)
+        if (sp[lo + step - 1] < x) lo += step;
+    return 2 * lo + (sp[lo] == x ? 1u : 0u);  // sp[255] is 0xFFFFFFFF, lo <= q
+}
+
+// The compare domain of a raw key: unsigned for uint32.  A float32's bits compare as a signed integer
+// against a bound that is not negative, whatever the key; below that the negative keys' low bits
+// are flipped first.
+template <class K>
+struct FDomain;
+template <>
+struct FDomain<KeyU32> {
+    using T = u32;
+    static __device__ __forceinline__ T bound(u32 ord) { return ord; }
+    static __device__ __forceinline__ u32 to_domain(u32 raw) { return raw; }
+    static __device__ __forceinline__ bool converts(T) { return false; }
+    static __device__ __forceinline__ u32 ordered(u32 x, bool) { return x; }
+};
+template <>
+struct FDomain<KeyF32> {
+    using T = int;
+    static __device__ __forceinline__ T bound(u32 ord) { return (int)(ord ^ 0x80000000u); }
+    static __device__ __forceinline__ u32 to_domain(u32 raw) { return raw ^ ((u32)((int)raw >> 31) & 0x7FFFFFFFu); }
+    static __device__ __forceinline__ bool converts(T t) { return t < 0; }
+    static __device__ __forceinline__ u32 ordered(u32 x, bool converted) {
+        return converted ? x ^ 0x80000000u : KeyF32::to_ord(x);
+    }
+};
+
+// Bound by the read stream where few keys are kept: a wave takes 2048 keys at a time (eight 16-byte
+// loads per lane), and a 256-key load that holds none above t costs four instructions a lane.
+// The others are counted with one ballot per key, placed in index order with one mask count per
+// key and staged in the wave's LDS.  They leave, with their classes counted, when that is full:
+// on this part a load is waited for together with the stores issued before it, so a wave that
+// stored after every unit waited for a write's round trip each time (2^30 keys, 172 K kept: 694 us).
+// Waves work alone, without a barrier in the loop.
+template <class K>
+__global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, u32 n, u32 nunits, int rounds, u32 wcap,
+                                               u32 pool_at, u32 pool_cap, FilterState* st, u32* __restrict__ skeys,
+                                               u32* __restrict__ sidx, u32* __restrict__ cnt, u32* __restrict__ base_of,
+                                               u32* __restrict__ cls) {
+    using D = FDomain<K>;
+    using DT = typename D::T;
+    __shared__ u32 sp[256], lh[F_CLASSES], sk[WG / WAVE][F_STAGE], si[WG / WAVE][F_STAGE];
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    sp[threadIdx.x] = st->split[threadIdx.x];
+    lh[threadIdx.x] = 0;
+    lh[WG + threadIdx.x] = 0;
+    const u32 t_ord = st->t, up = st->up;
+    const DT t = D::bound(t_ord);
+    const bool conv = D::converts(t);  // uniform
+    u32 above = 0;
+    __syncthreads();
+    auto count_class = [&](u32 v) {
+        if (v > up) ++above;
+        else atomicAdd(&lh[class_of(sp, v)], 1u);
+    };
+    // the wave's share of the segments, filled from its start; what its units kept and where, one unit
+    // per lane until 64 of them are written
+    const u32 gbase = (blockIdx.x * (WG / WAVE) + w) * wcap;
+    u32 gpos = 0, fill = 0, nrec = 0, my_unit = 0, my_cnt = 0, my_base = 0;
+    auto flush = [&]() {  // the staged keys are the last `fill` of the wave's share
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own LDS writes
+        __builtin_amdgcn_wave_barrier();
+        for (u32 i = lane; i < fill; i += WAVE) {
+            const u32 v = sk[w][i], at = gbase + gpos - fill + i;
+            skeys[at] = v;
+            sidx[at] = si[w][i];
+            count_class(v);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        fill = 0;
+    };
+    auto write_units = [&]() {
+        if ((u32)lane < nrec) {
+            cnt[my_unit] = my_cnt;
+            base_of[my_unit] = my_base;
+        }
+        nrec = 0;
+    };
+    // a workgroup step is 4 * rounds consecutive units, the waves taking every fourth
+    const u32 per = (u32)rounds * (WG / WAVE);
+    for (u32 step = blockIdx.x; step * per < nunits; step += gridDim.x)
+        for (int rd = 0; rd < rounds; ++rd) {
+            const u32 unit = step * per + rd * (WG / WAVE) + w;
+            if (unit >= nunits) break;  // uniform over the wave; no barrier in the loop
+            if (nrec == WAVE) write_units();
+            const u32 k0 = unit * F_UNIT;
+            u32x4 x[8];
+            u32 pads = 0;
+            if (k0 + F_UNIT <= n) {  // uniform
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+                    x[b] = __builtin_nontemporal_load((const u32x4*)(keys + k0) + b * WAVE + lane);
+            } else {
+                pads = k0 + F_UNIT - n;
+#pragma unroll
+                for (int b = 0; b < 8; ++b) {
+                    const u32 e = k0 + 4 * (b * WAVE + lane);
+                    if (e + 4 <= n) x[b] = *(const u32x4*)(keys + e);
+                    else
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) x[b][j] = e + j < n ? keys[e + j] : K::from_ord(0);  // the lowest key
+                }
+            }
+            if (conv) {
+#pragma unroll
+                for (int b = 0; b < 8; ++b)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) x[b][j] = D::to_domain(x[b][j]);
+            }
+            u32 c[8], kept = 0, eq = 0;
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                c[b] = 0;
+                const DT m = max(max((DT)x[b][0], (DT)x[b][1]), max((DT)x[b][2], (DT)x[b][3]));
+                if (__ballot(m >= t)) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        c[b] += (u32)__popcll(__ballot((DT)x[b][j] > t));
+                        eq += (DT)x[b][j] == t ? 1u : 0u;
+                    }
+                    kept += c[b];
+                }
+            }
+            if (__ballot(eq)) {
+                eq = (u32)__builtin_amdgcn_readlane((int)wave_incl_scan_u32(eq), WAVE - 1);
+                if (t_ord == 0) eq -= pads;
+            } else {
+                eq = 0;
+            }
+            const bool spill = gpos + kept > wcap;  // rare: clustered keys go to the pool
+            if (fill + kept > F_STAGE || spill) flush();
+            bool staged = kept <= F_STAGE && !spill;
+            u32 base = gbase + gpos;
+            if (spill) {
+                u32 at = 0;
+                if (lane == 0) at = atomicAdd(&st->pool, kept);
+                at = (u32)__builtin_amdgcn_readfirstlane((int)at);
+                base = pool_at + at;
+                if (at > pool_cap || kept > pool_cap - at) {
+                    if (lane == 0) st->fail = 1;
+                    kept = 0;
+                }
+            } else {
+                gpos += kept;
+            }
+            if ((u32)lane == nrec) {
+                my_unit = unit;
+                my_cnt = kept | (eq << 16);
+                my_base = kept ? base : 0u;
+            }
+            ++nrec;
+            if (kept == 0) continue;
+            u32 at = staged ? fill : base;
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                if (c[b] == 0) continue;
+                u32 pos = at;  // this lane's first: the granule's kept keys of the lanes below
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const u64 m = __ballot((DT)x[b][j] > t);
+                    pos = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, pos));
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if ((DT)x[b][j] > t) {
+                        const u32 v = D::ordered(x[b][j], conv), id = k0 + 4 * (b * WAVE + lane) + j;
+                        if (staged) {
+                            sk[w][pos] = v;
+                            si[w][pos] = id;
+                        } else {
+                            skeys[pos] = v;
+                            sidx[pos] = id;
+                            count_class(v);
+                        }
+                        ++pos;
+                    }
+                at += c[b];
+            }
+            if (staged) fill += kept;
+        }
+    flush();
+    write_units();
+    above = wave_incl_scan_u32(above);
+    if (lane == WAVE - 1 && above) atomicAdd(&lh[F_ABOVE], above);
+    __syncthreads();
+    u32* g = cls + (blockIdx.x % F_REPS) * F_CLASSES;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const u32 c = lh[j * WG + threadIdx.x];
+        if (c) atomicAdd(&g[j * WG + threadIdx.x], c);
+    }
+}
+
+// ---------------------------------------------------------------- the k-th key's class
+struct FClass {
+    u32 kept;      // all kept keys
+    u32 lo, hi;    // kept < k: K == t.  Otherwise the k-th key lies in (lo, hi], hi == lo + 1 once it is known
+    u32 above, kk; // keys above hi, rank of the k-th key among those in (lo, hi]
+    u32 in;        // keys in (lo, hi]
+};
+// Every thread of an NT-thread block; `lds` holds 8 words, `scratch` NT/64.  Ends with a barrier.
+template <int NT>
+__device__ __forceinline__ FClass find_class(const FilterState* st, const u32* __restrict__ cls, u32 k, u32* lds,
+                                             u32* scratch) {
+    constexpr int PER = NT >= 512 ? 1 : (int)F_CLASSES / NT;
+    u32 c[PER], s = 0, tot;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        c[j] = 0;
+        const int b = (int)F_CLASSES - 1 - ((int)threadIdx.x * PER + j);
+        if (b >= 0) {
+            u32 r[F_REPS];
+#pragma unroll
+            for (int i = 0; i < F_REPS; ++i) r[i] = cls[i * F_CLASSES + b];
+#pragma unroll
+            for (int i = 0; i < F_REPS; ++i) c[j] += r[i];
+        }
+        s += c[j];
+    }
+    u32 run = wg_excl_scan<NT>(s, scratch, &tot);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        if (run < k && run + c[j] >= k) {
+            lds[0] = (u32)((int)F_CLASSES - 1 - ((int)threadIdx.x * PER + j));
+            lds[1] = run;
+            lds[2] = c[j];
+        }
+        run += c[j];
+    }
+    __syncthreads();
+    FClass f;
+    f.kept = tot;
+    f.lo = f.hi = st->t;
+    f.above = f.kk = f.in = 0;
+    if (tot >= k) {
+        const u32 b = lds[0], i = b >> 1;
+        f.above = lds[1];
+        f.in = lds[2];
+        f.kk = k - f.above;
+        if (b == F_ABOVE) {
+            f.lo = st->up;
+            f.hi = 0xFFFFFFFFu;
+        } else if (b & 1) {
+            f.hi = st->split[i];
+            f.lo = f.hi - 1;
+        } else {
+            f.lo = i ? st->split[i - 1] : st->t;
+            f.hi = i < st->q ? st->split[i] - 1 : st->up;
+        }
+    }
+    return f;
+}
+
+// The kept keys of units [u0, u1) of a range, laid end to end (at most F_RUNITS units).
+struct RangeLds {
+    u32 pref[F_RUNITS + 1], base[F_RUNITS], eqp[F_RUNITS + 1];
+    u32 scratch[WG / WAVE], lds[8];
+};
+// Fills the table; returns the keys kept (every thread).  Contains barriers.
+__device__ __forceinline__ u32 range_open(RangeLds& R, const u32* __restrict__ cnt, const u32* __restrict__ base_of, u32 u0,
+                                          u32 u1, u32* eq_out) {
+    static_assert(F_RUNITS <= WG, "one unit per thread");
+    const u32 u = u0 + threadIdx.x;
+    const u32 c = u < u1 ? cnt[u] : 0u;
+    if (threadIdx.x < F_RUNITS) R.base[threadIdx.x] = u < u1 ? base_of[u] : 0u;
+    u32 tot, eq;
+    const u32 ex = wg_excl_scan<WG>(c & 0xFFFFu, R.scratch, &tot);
+    const u32 eqx = wg_excl_scan<WG>(c >> 16, R.scratch, &eq);
+    if (threadIdx.x < F_RUNITS) {
+        R.pref[threadIdx.x] = ex;
+        R.eqp[threadIdx.x] = eqx;
+    }
+    if (threadIdx.x == 0) {
+        R.pref[F_RUNITS] = tot;
+        R.eqp[F_RUNITS] = eq;
+    }
+    __syncthreads();
+    *eq_out = eq;
+    return tot;
+}
+// Slots of the eight consecutive kept keys from e on (valid ones only below `tot`).
+__device__ __forceinline__ void range_slots(const RangeLds& R, u32 e, u32 tot, u32 (&at)[8]) {
+    u32 s = 0;
+#pragma unroll
+    for (u32 step = F_RUNITS / 2; step; step >>= 1)
+        if (R.pref[s + step] <= e) s += step;
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) {
+        const bool ok = e + j < tot;
+        while (ok && R.pref[s + 1] <= e + j) ++s;
+        at[j] = ok ? R.base[s] + (e + j - R.pref[s]) : 0u;
+    }
+}
+
+__global__ __launch_bounds__(WG) void k_fpick(FilterState* st, const u32* __restrict__ cls, u32 k, u32 nunits, u32 upr,
+                                              const u32* __restrict__ cnt, const u32* __restrict__ base_of,
+                                              const u32* __restrict__ skeys, u32* __restrict__ rg, u32* __restrict__ rq,
+                                              u32 lcap, u32* __restrict__ lkey, u32* __restrict__ lrange) {
+    __shared__ RangeLds R;
+    const FClass f = find_class<WG>(st, cls, k, R.lds, R.scratch);
+    const u32 r = blockIdx.x, u0 = r * upr, u1 = min(u0 + upr, nunits);
+    u32 eq;
+    const u32 tot = range_open(R, cnt, base_of, u0, u1, &eq);
+    if (f.kept < k) {  // K == t, or the bound failed
+        if (threadIdx.x == 0) {
+            rg[r] = tot;
+            rq[r] = eq;
+        }
+        return;
+    }
+    const bool known = f.hi - f.lo == 1;  // one value: counted, not listed
+    u32 g = 0, q = 0;
+    for (u32 e0 = 0; e0 < tot; e0 += F_BATCH) {
+        u32 at[8], x[8], in = 0;
+        range_slots(R, e0 + 8 * threadIdx.x, tot, at);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = skeys[at[j]];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (e0 + 8 * threadIdx.x + j >= tot) x[j] = 0;
+            g += x[j] > f.hi ? 1u : 0u;
+            in += x[j] > f.lo && x[j] <= f.hi ? 1u : 0u;
+        }
+        q += in;
+        if (known) continue;
+        u32 n;
+        const u32 ex = wg_excl_scan<WG>(in, R.scratch, &n);
+        if (n == 0) continue;  // uniform
+        const u32 list = (r + e0 / F_BATCH) % F_LISTS;
+        if (threadIdx.x == 0) R.lds[4] = atomicAdd(&st->lcount[list], n);
+        __syncthreads();
+        u32 to = R.lds[4] + ex;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (x[j] > f.lo && x[j] <= f.hi) {
+                if (to < lcap) {
+                    lkey[list * lcap + to] = x[j];
+                    lrange[list * lcap + to] = r;
+                }
+                ++to;
+            }
+        __syncthreads();
+    }
+    u32 gs, qs;
+    wg_excl_scan<WG>(g, R.scratch, &gs);
+    wg_excl_scan<WG>(q, R.scratch, &qs);
+    if (threadIdx.x == 0) {
+        rg[r] = gs;
+        rq[r] = known ? qs : 0u;
+    }
+}
+
+// ---------------------------------------------------------------- k-th key and range offsets
+template <class K>
+__global__ __launch_bounds__(FS_NT) void k_fkth(FilterState* st, const u32* __restrict__ cls, u32 k, u32 nranges,
+                                                u32* __restrict__ rg, u32* __restrict__ rq, u32 lcap,
+                                                const u32* __restrict__ lkey, const u32* __restrict__ lrange,
+                                                const u32* __restrict__ keys, u32 n, u32* __restrict__ out_keys,
+                                                i64* __restrict__ out_idx, u32* __restrict__ d_kth) {
+    __shared__ WgSel<FS_NT> L;
+    __shared__ __align__(16) u32 el[wg_words<FS_NT>(32768)];
+    __shared__ u32 lpref[F_LISTS + 1], lds[8];
+    const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE;
+    wg_init<FS_NT>(L);
+    constexpr int RPT = F_RANGES / FS_NT;
+    static_assert(32768 + 2 * F_RANGES <= wg_words<FS_NT>(32768), "the ranges' counts behind the list");
+    u32 g[RPT], q[RPT];  // loaded with the class counters: one round trip
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+        const u32 r = t * RPT + j;
+        g[j] = r < nranges ? rg[r] : 0u;
+        q[j] = r < nranges ? rq[r] : 0u;
+    }
+    const u32 in_list = t < (int)F_LISTS ? st->lcount[t] : 0u;
+    const FClass f = find_class<FS_NT>(st, cls, k, lds, L.a);
+    u32 qs = 0, eqs;
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) qs += q[j];
+    wg_excl_scan<FS_NT>(qs, L.b, &eqs);
+    u32 Kk = f.hi, gt = f.above, kind = F_CLASS;
+    bool ok = st->fail == 0;
+    if (f.kept < k) {
+        kind = F_AT_T;
+        gt = f.kept;
+        ok = ok && (u64)f.kept + eqs >= k;
+    } else if (f.hi - f.lo > 1) {
+        if (t < (int)WAVE) {
+            const u32 inc = wave_incl_scan_u32(in_list);
+            lpref[t + 1] = inc;
+            if (t == 0) lpref[0] = 0;
+            lds[4 + 0] = 0;
+        }
+        __syncthreads();
+        if (t < (int)F_LISTS && lpref[t + 1] - lpref[t] > lcap) lds[4] = 1;
+        __syncthreads();
+        const u32 m = lpref[F_LISTS];
+        ok = ok && lds[4] == 0 && m == f.in;
+        if (ok) {
+            // f(i, slot, key) for every entry of the lists laid end to end, a wave per list, eight loads
+            // in flight
+            auto each_entry = [&](auto&& fn) {
+                for (u32 l = w; l < F_LISTS; l += FS_NT / WAVE) {
+                    const u32 c = lpref[l + 1] - lpref[l];
+                    for (u32 i0 = 0; i0 < c; i0 += 8 * WAVE) {
+                        u32 x[8];
+#pragma unroll
+                        for (u32 u = 0; u < 8; ++u) x[u] = lkey[l * lcap + min(i0 + u * WAVE + lane, c - 1)];
+#pragma unroll
+                        for (u32 u = 0; u < 8; ++u) {
+                            const u32 i = i0 + u * WAVE + lane;
+                            if (i < c) fn(lpref[l] + i, l * lcap + i, x[u]);
+                        }
+                    }
+                }
+            };
+            const bool held = m <= 32768;
+            if (held) {
+                each_entry([&](u32 i, u32, u32 x) { el[i] = x; });
+                __syncthreads();
+            }
+            Kk = wg_kth_between<FS_NT>(
+                [&](auto&& fn) {
+                    if (held)
+                        for (u32 i = t; i < m; i += FS_NT) fn(u32x4{el[i], f.lo, f.lo, f.lo});
+                    else
+                        each_entry([&](u32, u32, u32 x) { fn(u32x4{x, f.lo, f.lo, f.lo}); });
+                },
+                f.lo + 1, f.hi, f.kk, L, &gt);
+            gt += f.above;
+            // the class's keys above K and equal to it, back to their ranges
+            u32* add = el + 32768;
+            for (u32 i = t; i < 2 * F_RANGES; i += FS_NT) add[i] = 0;
+            __syncthreads();
+            each_entry([&](u32, u32 s, u32 x) {
+                if (x >= Kk) atomicAdd(&add[(x > Kk ? 0u : F_RANGES) + lrange[s]], 1u);
+            });
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                g[j] += add[t * RPT + j];
+                q[j] += add[F_RANGES + t * RPT + j];
+            }
+        }
+    }
+    if (ok) {
+        u32 gs = 0, tot;
+        qs = 0;
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            gs += g[j];
+            qs += q[j];
+        }
+        __syncthreads();
+        u32 gr = wg_excl_scan<FS_NT>(gs, L.a, &tot), qr = wg_excl_scan<FS_NT>(qs, L.b, &tot);
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+            const u32 r = t * RPT + j;
+            if (r < nranges) {
+                rg[r] = gr;
+                rq[r] = qr;
+            }
+            gr += g[j];
+            qr += q[j];
+        }
+        if (t == 0) {
+            st->K = Kk;
+            st->gt = gt;
+            st->ties = k - gt;
+            st->kind = kind;
+            if (d_kth) *d_kth = K::from_ord(Kk);
+        }
+        return;
+    }
+    // last resort: this workgroup selects from the keys, a wave per contiguous share of them
+    __syncthreads();
+    wg_init<FS_NT>(L);
+    __syncthreads();
+    const u32 share = (((n + FS_NT / WAVE - 1) / (FS_NT / WAVE)) + 255u) & ~255u;
+    const u32 b0 = min(n, w * share), b1 = min(n, b0 + share);
+    auto load = [&](u32 e) {  // a lane's four keys (0 past the share: its last granule may be partial)
+        u32x4 x = {0, 0, 0, 0};
+        if (e + 4 <= b1) {
+            x = *(const u32x4*)(keys + e);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = K::to_ord(x[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (e + j < b1) x[j] = K::to_ord(keys[e + j]);
+        }
+        return x;
+    };
+    Kk = wg_kth<FS_NT>(
+        [&](auto&& fn) {
+#pragma unroll 8
+            for (u32 e = b0 + 4 * lane; e < b1; e += 4 * WAVE) fn(load(e));
+        },
+        k, L, &gt);
+    if (t == 0) {
+        st->kind = F_DONE;
+        if (d_kth) *d_kth = K::from_ord(Kk);
+    }
+    if (!out_keys && !out_idx) return;
+    u32 cg = 0, cq = 0;
+    for (u32 e = b0 + 4 * lane; e < b1; e += 4 * WAVE) {
+        const u32x4 x = load(e);
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j) {
+            cg += x[j] > Kk ? 1u : 0u;
+            cq += e + j < b1 && x[j] == Kk ? 1u : 0u;
+        }
+    }
+    cg = wave_incl_scan_u32(cg);
+    cq = wave_incl_scan_u32(cq);
+    __syncthreads();
+    if (lane == WAVE - 1) {
+        L.a[w] = cg;
+        L.b[w] = cq;
+    }
+    __syncthreads();
+    u32 tot;
+    u32 gr = wave_totals_prefix<FS_NT>(L.a, &tot), qr = wave_totals_prefix<FS_NT>(L.b, &tot);
+    const u32 ties = k - gt;
+    for (u32 e0 = b0; e0 < b1; e0 += 4 * WAVE) {
+        const u32 e = e0 + 4 * lane;
+        const u32x4 x = load(e);
+        u32 mg = 0, mq = 0;
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j) {
+            mg += x[j] > Kk ? 1u : 0u;
+            mq += e + j < b1 && x[j] == Kk ? 1u : 0u;
+        }
+        const u32 mine = (mg << 16) | mq, inc = wave_incl_scan_u32(mine);
+        u32 gb = gr + ((inc - mine) >> 16), qb = qr + ((inc - mine) & 0xFFFFu);
+#pragma unroll
+        for (u32 j = 0; j < 4; ++j) {
+            const bool isg = x[j] > Kk, isq = e + j < b1 && x[j] == Kk;
+            if (isg || (isq && qb < ties)) {
+                const u32 p = gb + min(qb, ties);
+                if (out_keys) out_keys[p] = K::from_ord(x[j]);
+                if (out_idx) out_idx[p] = (i64)(e + j);
+            }
+            gb += isg ? 1u : 0u;
+            qb += isq ? 1u : 0u;
+        }
+        const u32 all = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+        gr += all >> 16;
+        qr += all & 0xFFFFu;
+    }
+}
+
+// ---------------------------------------------------------------- outputs
+template <class K>
+__global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nunits, u32 upr, const u32* __restrict__ cnt,
+                                               const u32* __restrict__ base_of, const u32* __restrict__ skeys,
+                                               const u32* __restrict__ sidx, const u32* __restrict__ rg,
+                                               const u32* __restrict__ rq, const u32* __restrict__ keys, u32 n, u32 k,
+                                               u32* __restrict__ out_keys, i64* __restrict__ out_idx) {
+    __shared__ RangeLds R;
+    __shared__ u32 sk[F_BATCH], si[F_BATCH];
+    const u32 kind = st->kind, K0 = st->K, ties = st->ties;
+    if (kind == F_DONE) return;
+    u32 r = blockIdx.x, sub = 0, subs = 1;
+    if (kind == F_AT_T) {
+        // Only the ranges with outputs, several workgroups to each where they are few: ties at the
+        // bound may all be taken from the first of the ranges.
+        __shared__ u16 act[F_RANGES];
+        constexpr u32 RPT = F_RANGES / WG;
+        const u32 nr = gridDim.x, r0 = threadIdx.x * RPT;
+        u32 on = 0, na;
+#pragma unroll
+        for (u32 j = 0; j < RPT; ++j)
+            if (r0 + j < nr) {
+                const u32 at = r0 + j, nx = at + 1;
+                if (nx == nr || rg[nx] != rg[at] || (rq[at] < ties && rq[nx] != rq[at])) on |= 1u << j;
+            }
+        u32 to = wg_excl_scan<WG>((u32)__popc(on), R.scratch, &na);
+#pragma unroll
+        for (u32 j = 0; j < RPT; ++j)
+            if (on >> j & 1) act[to++] = (u16)(r0 + j);
+        __syncthreads();
+        subs = max(nr / na, 1u);  // na >= 1: the last range is in
+        if (r >= na * subs) return;
+        sub = r % subs;
+        r = act[r / subs];
+    }
+    const u32 u0 = r * upr, u1 = min(u0 + upr, nunits);
+    u32 g = rg[r], q = rq[r], eq;  // outputs before the next batch: above K0, and ties
+    const u32 tot = range_open(R, cnt, base_of, u0, u1, &eq);
+    if (kind == F_AT_T) {
+        // Each unit by a wave alone.  Ties at the bound were counted, not kept: a unit that gives some
+        // is read again; of the others all that was kept goes out.  (The workgroup in batches of 2048
+        // keys, three barriers each, a range per workgroup: 23 us for 65536 ties among the first
+        // 475 K of 2^24 keys.)
+        const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+        for (u32 i = sub * (WG / WAVE) + w; i < u1 - u0; i += subs * (WG / WAVE)) {
+            u32 gu = g + R.pref[i], qu = q + R.eqp[i];
+            if (qu >= ties || R.eqp[i + 1] == R.eqp[i]) {
+                const u32 c = R.pref[i + 1] - R.pref[i], to = gu + min(qu, ties), from = R.base[i];
+                for (u32 j = lane; j < c && to + j < k; j += WAVE) {
+                    if (out_keys) out_keys[to + j] = K::from_ord(skeys[from + j]);
+                    if (out_idx) out_idx[to + j] = (i64)sidx[from + j];
+                }
+                continue;
+            }
+            const u32 k0 = (u0 + i) * F_UNIT + 4 * lane;
+            u32x4 x[8];
+#pragma unroll
+            for (u32 b = 0; b < 8; ++b) {
+                const u32 e = k0 + b * 4 * WAVE;
+                if (e + 4 <= n) x[b] = *(const u32x4*)(keys + e);
+                else
+#pragma unroll
+                    for (u32 j = 0; j < 4; ++j) x[b][j] = e + j < n ? keys[e + j] : 0u;
+            }
+#pragma unroll
+            for (u32 b = 0; b < 8; ++b) {
+                u32 mine = 0;  // above << 16 | ties
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j) {
+                    const u32 v = K::to_ord(x[b][j]);
+                    mine += k0 + b * 4 * WAVE + j < n ? (v > K0 ? 0x10000u : (v == K0 ? 1u : 0u)) : 0u;
+                }
+                const u32 inc = wave_incl_scan_u32(mine);
+                u32 gb = gu + ((inc - mine) >> 16), qb = qu + ((inc - mine) & 0xFFFFu);
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j) {
+                    const u32 v = K::to_ord(x[b][j]), e = k0 + b * 4 * WAVE + j;
+                    const bool isg = e < n && v > K0, isq = e < n && v == K0;
+                    if (isg || (isq && qb < ties)) {
+                        const u32 p = gb + min(qb, ties);
+                        if (p < k) {
+                            if (out_keys) out_keys[p] = x[b][j];
+                            if (out_idx) out_idx[p] = (i64)e;
+                        }
+                    }
+                    gb += isg ? 1u : 0u;
+                    qb += isq ? 1u : 0u;
+                }
+                const u32 all = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+                gu += all >> 16;
+                qu += all & 0xFFFFu;
+            }
+        }
+        return;
+    }
+    q = min(q, ties);
+    // a batch of 8 keys per thread in index order: those above K0 and the ties still to take
+    auto emit = [&](const u32 (&x)[8], const u32 (&id)[8], u32 nv) {
+        u32 c = 0;  // above << 16 | ties, among the thread's first nv keys
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) c += j < nv ? (x[j] > K0 ? 0x10000u : (x[j] == K0 ? 1u : 0u)) : 0u;
+        u32 all;
+        const u32 ex = wg_excl_scan<WG>(c, R.scratch, &all);
+        const u32 rem = min(ties - q, F_BATCH);  // ties left for this batch
+        u32 lg = ex >> 16, lq = ex & 0xFFFFu;
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) {
+            if (j >= nv || x[j] < K0) continue;
+            if (x[j] > K0 || lq < rem) {
+                const u32 s = lg + min(lq, rem);
+                sk[s] = K::from_ord(x[j]);
+                si[s] = id[j];
+            }
+            lg += x[j] > K0 ? 1u : 0u;
+            lq += x[j] == K0 ? 1u : 0u;
+        }
+        __syncthreads();
+        const u32 took = min(all & 0xFFFFu, rem), m = (all >> 16) + took, to = g + q;
+        for (u32 i = threadIdx.x; i < m && to + i < k; i += WG) {
+            if (out_keys) out_keys[to + i] = sk[i];
+            if (out_idx) out_idx[to + i] = (i64)si[i];
+        }
+        g += all >> 16;
+        q += took;
+        __syncthreads();
+    };
+    for (u32 e0 = 0; e0 < tot; e0 += F_BATCH) {
+        const u32 e = e0 + 8 * threadIdx.x;
+        u32 at[8], x[8], id[8];
+        range_slots(R, e, tot, at);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            x[j] = skeys[at[j]];
+            id[j] = sidx[at[j]];
+        }
+        emit(x, id, e < tot ? min(tot - e, 8u) : 0u);
+    }
+}
+
+hipError_t launch_filter(const FilterArgs& a, hipStream_t st) {
+    FilterState* fs = (FilterState*)a.state;
+    u32* cls = (u32*)(fs + 1);
+    const u32 n = (u32)a.n, k = (u32)a.k;
+    const u32 nunits = filter_units(a.n);
+    // units per range: about half a batch of kept keys, in 512 .. F_RANGES ranges
+    const u64 half = (u64)F_BATCH / 2 * nunits / std::max<u64>(a.kept, 1);
+    const u64 most = std::min<u64>((nunits + 511) / 512, F_RUNITS);
+    const u32 upr = (u32)std::max<u64>((nunits + F_RANGES - 1) / F_RANGES, std::min(most, half));
+    const u32 nranges = (nunits + upr - 1) / upr;
+    if (upr > F_RUNITS || (a.lm != 13 && a.lm != 15 && a.lm != 17 && a.lm != 19)) return hipErrorInvalidValue;
+    const FilterGrid fg = filter_grid(a.n);
+#define F_SPLIT_LAUNCH(LM)                                                                                          \
+    hipLaunchKernelGGL((k_fsplit<LM>), dim3(1), dim3(FS_NT), 0, st, a.sample, a.sample + (1u << a.lm), a.rp, a.rlo, \
+                       a.rhi, fs)
+#define F_LAUNCH(K)                                                                                                     \
+    do {                                                                                                                \
+        hipLaunchKernelGGL((k_fsample<K>), dim3((1u << a.lm) / 4 / WG), dim3(WG), 0, st, a.keys, a.n, a.lm, a.sample,  \
+                           a.sample + (1u << a.lm), a.ctrl, fs, cls);                                                   \
+        if (a.lm == 13) F_SPLIT_LAUNCH(13);                                                                            \
+        else if (a.lm == 15) F_SPLIT_LAUNCH(15);                                                                       \
+        else if (a.lm == 17) F_SPLIT_LAUNCH(17);                                                                       \
+        else F_SPLIT_LAUNCH(19);                                                                                       \
+        hipLaunchKernelGGL((k_filter<K>), dim3(fg.grid), dim3(WG), 0, st, a.keys, n, nunits, fg.rounds, a.wcap,        \
+                           fg.grid * 4 * a.wcap, a.pool_cap, fs, a.skeys, a.sidx, a.cnt, a.base, cls);                        \
+        hipLaunchKernelGGL(k_fpick, dim3(nranges), dim3(WG), 0, st, fs, cls, k, nunits, upr, a.cnt, a.base, a.skeys,   \
+                           a.rg, a.rq, a.lcap, a.lkey, a.lrange);                                                      \
+        hipLaunchKernelGGL((k_fkth<K>), dim3(1), dim3(FS_NT), 0, st, fs, cls, k, nranges, a.rg, a.rq, a.lcap, a.lkey,  \
+                           a.lrange, a.keys, n, (u32*)a.out_keys, a.out_idx, (u32*)a.d_kth);                           \
+        if (a.out_keys || a.out_idx)                                                                                   \
+            hipLaunchKernelGGL((k_fwrite<K>), dim3(nranges), dim3(WG), 0, st, fs, nunits, upr, a.cnt, a.base, a.skeys, \
+                               a.sidx, a.rg, a.rq, a.keys, n, k, (u32*)a.out_keys, a.out_idx);                         \
+    } while (0)
+    if (a.f32) F_LAUNCH(KeyF32);
+    else F_LAUNCH(KeyU32);
+#undef F_LAUNCH
+#undef F_SPLIT_LAUNCH
+    return hipGetLastError();
+}
+
+}  // namespace drtopk

@@ -179,6 +179,53 @@ hipError_t launch_small(const ShortArgs& a, hipStream_t st);
 hipError_t launch_short(const ShortArgs& a, hipStream_t st);
 u32 short_segments(u64 V);         // concatenation segments of V = k << alpha slots
 
+// filter.hip --------------------------------------------------------------------------
+// Large k: a sampled lower bound of the k-th key, one filter pass, selection of what it keeps.
+constexpr u32 F_UNIT = 2048;     // keys per unit: one segment of kept keys
+constexpr u32 F_RANGES = 2048;   // most ranges of units (workgroups of the passes over kept keys)
+constexpr u32 F_RUNITS = 256;    // most units per range (n <= 2^30)
+constexpr u32 F_LIST_LDS = 17408;  // samples above the first bound of 2^17 or 2^19
+inline u32 filter_units(u64 n) { return (u32)((n + F_UNIT - 1) / F_UNIT); }
+// Workgroups of the filter pass and the consecutive 8192-key rounds each takes per step.  2^30 keys, no
+// key kept: 693 us with 1 round, 633 with 4, 619 with 8 (8192 workgroups); small inputs need the
+// workgroups more.
+struct FilterGrid {
+    u32 grid;
+    int rounds;
+};
+inline FilterGrid filter_grid(u64 n) {
+    const u32 units = filter_units(n);
+    u32 r = units / (4 * 2048);
+    r = r < 1 ? 1 : (r > 8 ? 8 : r);
+    const u32 steps = (units + 4 * r - 1) / (4 * r);
+    return {steps < 8192 ? steps : 8192, (int)r};
+}
+size_t filter_state_bytes();
+struct FilterArgs {
+    const u32* keys;   // 16-byte aligned, n >= 2^15
+    u64 n, k;
+    int f32;
+    int lm;            // log2 of the samples: 15, 17 or 19; n >= 2^lm
+    u32 rp;            // sample rank bounding the k-th key from below
+    u32 rlo, rhi;      // sample ranks between which the k-th key almost surely lies (rlo 0: the largest)
+    u64 kept;          // keys expected above the bound
+    u32 wcap;          // kept keys a wave's own segment holds
+    u32 pool_cap;      // and the pool behind the segments, for units that find it full
+    u32 lcap;          // entries of each of the 64 sublists of the k-th key's class
+    Ctrl* ctrl;
+    void* state;       // filter_state_bytes()
+    u32* sample;       // [2^lm + 2^14]
+    u32* cnt;          // [units] kept | equal to the bound << 16
+    u32* base;         // [units] first slot of the unit's kept keys
+    u32 *rg, *rq;      // [F_RANGES]
+    u32 *lkey, *lrange;  // [64 * lcap]
+    u32 *skeys, *sidx;   // [4 * workgroups * wcap + pool_cap]
+    void* out_keys;
+    i64* out_idx;
+    void* d_kth;
+};
+hipError_t launch_filter(const FilterArgs& a, hipStream_t st);
+
 // bitonic.hip ---------------------------------------------------------------------------
 // Bitonic family: first top-k over the delegates, whole-subrange concatenation, second
 // top-k, index-ordered outputs.  alpha == 0: one top-k over V.
