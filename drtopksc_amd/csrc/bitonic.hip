@@ -8,12 +8,17 @@
 // and the result does not depend on how the network is scheduled.
 //
 // Scheduling on gfx950 (160 KB of LDS per CU):
-//  - k <= T/2: one workgroup reduces an LDS tile of T composites to its own top-k (sort into
-//    k-runs, then log2(T/k) merge+rebuild rounds entirely in LDS); tiles are reduced level by
-//    level until one tile remains.  T = 8192 (64 KB, two workgroups per CU) for k <= 2048 and
-//    T = 16384 (128 KB, one 1024-thread workgroup per CU) above, so k up to 8192 stays in LDS
-//    and each level shrinks the data by T/k >= 2.  The reference instead halves once per launch
-//    (bitonic_com.cuh:648-657).
+//  - k <= 4096: a workgroup reduces a tile in LDS to its own top-k (sort into k-runs, then
+//    merge + rebuild rounds); tiles are reduced level by level until one remains.  A compare step costs
+//    an LDS round trip and a barrier, so a thread takes eight composites through three steps at once in
+//    registers.  Unsorted input comes in tiles of 2048 (the 55 steps of k = 1024 on many CUs), sorted runs
+//    in tiles of 8192 (few levels).  The first level builds its composites from the delegates or the
+//    concatenation, the last one writes the results: in index order, after one more sort of the k
+//    survivors.  The reference halves once per launch (bitonic_com.cuh:648-657).
+//    2^26 keys, k = 1024: the 131072 delegates take 36 us and the 524288 concatenated keys with the results
+//    56 (one step per round trip in tiles of 8192, with launches of their own for the composites, the
+//    copy of the delegates and the sort by index: 270 in all).
+//  - k = 8192: tiles of 16384 composites, one compare step per round trip.
 //  - k > 8192 (the reference's largerK global-scratch variant): the network runs over a global
 //    buffer; strides >= 16384 are global passes, all smaller strides of a stage are fused into
 //    one LDS pass per 16384-composite tile.
@@ -24,8 +29,7 @@
 
 namespace drtopk {
 
-constexpr u32 BT_SMALL = 8192;   // LDS tile of composites for k <= 2048 (64 KB)
-constexpr int BTT_SMALL = 512;
+constexpr u32 BT_KMAX = 4096;    // largest k of the eight-at-once tiles
 constexpr u32 BT = 16384;        // LDS tile for larger k and the global network (128 KB)
 constexpr int BTT = 1024;
 
@@ -50,7 +54,239 @@ __device__ __forceinline__ void lds_steps(u64* A, u32 T, u64 base, u64 len, u64 
     }
 }
 
-// ---------------------------------------------------------------- tile reduction (k <= TILE/2)
+// ---------------------------------------------------------------- eight composites at once (k <= 4096)
+struct BtArgs {
+    u64 n;             // the level's input (a power of two); n of the last level may be below 8
+    u32 kk, k;         // run length max(k, 8); results k
+    int src;           // BT_RUNS: sorted runs of kk in A; BT_DELEG: dvals; BT_KEYS: V, or its subranges in D
+    int fin;           // BT_LEVEL: tile top-kk to out; BT_FIRST: top-k delegates to out; BT_LAST: results
+    const u64* A;
+    const u32* dvals;
+    u64 S;
+    const u32* keys;
+    u64 nkeys, nv;
+    int alpha, f32;
+    const u64* D;
+    u64* out;
+    u32* out_keys;
+    i64* out_idx;
+    u32* d_kth;
+    Ctrl* ctrl;
+};
+enum { BT_RUNS, BT_DELEG, BT_KEYS };
+enum { BT_LEVEL, BT_FIRST, BT_LAST };
+
+// Word of element i: one word of padding per eight, so that neither eight consecutive elements per
+// thread nor elements at a stride meet in the banks.
+__device__ __forceinline__ u32 bt_at(u32 i) { return i + (i >> 3); }
+
+__device__ __forceinline__ void bt_cx(u64& a, u64& b, bool up) {
+    const bool sw = up == (a > b);
+    const u64 x = sw ? b : a, y = sw ? a : b;
+    a = x;
+    b = y;
+}
+// Compare steps at distances d, d/2, .. 1 (d = 1, 2 or 4, uniform).
+__device__ __forceinline__ void bt_steps(u64 (&x)[8], u32 d, bool up) {
+    if (d >= 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bt_cx(x[j], x[j + 4], up);
+    }
+    if (d >= 2) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+            bt_cx(x[j], x[j + 2], up);
+            bt_cx(x[j + 1], x[j + 3], up);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) bt_cx(x[j], x[j + 1], up);
+}
+// Strides top .. 1 of stage `len` over the T elements of S, up to three per round trip.  Ends with a
+// barrier.
+__device__ __forceinline__ void bt_stage(u64* S, u32 T, u32 top, u32 len) {
+    for (; top; top >>= 3) {
+        const u32 b = top >= 4 ? 29 - __clz((int)top) : 0;  // unit 2^b = top / 4
+        const u32 t = threadIdx.x;
+        if (t < T / 8) {
+            const u32 i0 = ((t >> b) << (b + 3)) | (t & ((1u << b) - 1));
+            u64 x[8];
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) x[j] = S[bt_at(i0 + (j << b))];
+            bt_steps(x, top >> b, (i0 & (2 * len)) == 0);
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) S[bt_at(i0 + (j << b))] = x[j];
+        }
+        __syncthreads();
+    }
+}
+// Sorts the T elements, eight consecutive ones in each thread's x, into alternating runs of kk (or
+// one ascending run where T == kk) in S.  Ends with a barrier.
+__device__ __forceinline__ void bt_sort_runs(u64* S, u64 (&x)[8], u32 T, u32 kk) {
+    const u32 t = threadIdx.x;
+    if (t < T / 8) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) bt_cx(x[j], x[j + 1], (j & 2) == 0);
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+            bt_cx(x[j], x[j + 2], j == 0);
+            bt_cx(x[j + 1], x[j + 3], j == 0);
+            bt_cx(x[j], x[j + 1], j == 0);
+            bt_cx(x[j + 2], x[j + 3], j == 0);
+        }
+        bt_steps(x, 4, ((8 * t) & 8) == 0);
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) S[bt_at(8 * t + j)] = x[j];
+    }
+    __syncthreads();
+    for (u32 len = 8; len < kk; len <<= 1) bt_stage(S, T, len, len);
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT) void k_bt_tile(const BtArgs a) {
+    constexpr u32 TILE = NT * 8;
+    __shared__ u64 S[TILE + TILE / 8];
+    __shared__ u32 cnt;
+    const u32 t = threadIdx.x, kk = a.kk;
+    const u32 T = (u32)(a.n < 8 ? 8 : (a.n < TILE ? a.n : TILE));
+    const u64 base = (u64)blockIdx.x * TILE;
+    if (t == 0) cnt = 0;
+    // eight consecutive composites per thread
+    u64 x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = 0;
+    if (a.src == BT_RUNS) {
+        if (t < T / 8) {  // odd runs reversed: alternating runs without sorting again
+            const u32 i = 8 * t, r0 = i & ~(kk - 1);
+            const bool rev = i & kk;
+            const u64* p = a.A + base + (rev ? r0 + (kk - 8 - (i - r0)) : i);
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) S[bt_at(rev ? i + 7 - j : i + j)] = p[j];
+        }
+        __syncthreads();
+    } else {
+        u32 valid = 0;
+        const u64 v0 = base + 8 * t;
+        if (t < T / 8) {
+            if (a.src == BT_DELEG) {
+#pragma unroll
+                for (u32 j = 0; j < 8; ++j)
+                    if (v0 + j < a.S) x[j] = ((u64)a.dvals[v0 + j] << 32) | (u64)(0xFFFFFFFFu - (u32)(v0 + j));
+            } else {
+                u64 g0 = v0;
+                if (a.D && a.alpha >= 3 && v0 < a.nv)  // the eight lie in one subrange
+                    g0 = ((u64)(0xFFFFFFFFu - (u32)a.D[v0 >> a.alpha]) << a.alpha) + (v0 & ((1ull << a.alpha) - 1));
+#pragma unroll
+                for (u32 j = 0; j < 8; ++j) {
+                    u64 g = g0 + j;
+                    if (a.D && a.alpha < 3 && v0 + j < a.nv)
+                        g = ((u64)(0xFFFFFFFFu - (u32)a.D[(v0 + j) >> a.alpha]) << a.alpha) +
+                            ((v0 + j) & ((1ull << a.alpha) - 1));
+                    if (v0 + j < a.nv && g < a.nkeys) {
+                        const u32 key = a.keys[g];
+                        x[j] = ((u64)(a.f32 ? KeyF32::to_ord(key) : key) << 32) | (u64)(0xFFFFFFFFu - (u32)g);
+                        ++valid;
+                    }
+                }
+            }
+        }
+        if (a.src == BT_KEYS) {  // the concatenation's size, a statistic
+            valid = wave_incl_scan_u32(valid);
+            __syncthreads();
+            if ((t & (WAVE - 1)) == WAVE - 1 && valid) atomicAdd(&cnt, valid);
+            __syncthreads();
+            if (t == 0 && cnt) atomicAdd((unsigned long long*)&a.ctrl->concat_size, (unsigned long long)cnt);
+        }
+        bt_sort_runs(S, x, T, kk);
+    }
+    for (u32 cur = T / 2; cur >= kk; cur >>= 1) {
+        // merge: element t of the halved tile = max of the pair (i, i + kk) of runs 2r, 2r + 1; and the
+        // first three strides of the runs' rebuild
+        const u32 b = 28 - __clz((int)kk);  // unit kk / 8
+        const u32 i0 = ((t >> b) << (b + 3)) | (t & ((1u << b) - 1));
+        if (t < cur / 8) {
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) {
+                const u32 m = i0 + (j << b), i = 2 * m - (m & (kk - 1));
+                const u64 p = S[bt_at(i)], q = S[bt_at(i + kk)];
+                x[j] = p > q ? p : q;
+            }
+            bt_steps(x, 4, (i0 & kk) == 0);
+        }
+        __syncthreads();
+        if (t < cur / 8) {
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) S[bt_at(i0 + (j << b))] = x[j];
+        }
+        __syncthreads();
+        bt_stage(S, cur, kk >> 4, kk >> 1);
+    }
+    const u32 skip = kk - a.k;  // S[0..kk) ascending
+    if (a.fin == BT_LEVEL) {
+        for (u32 i = t; i < kk; i += NT) a.out[(u64)blockIdx.x * kk + i] = S[bt_at(i)];
+        return;
+    }
+    const u32 K0 = (u32)(S[bt_at(skip)] >> 32);
+    if (a.fin == BT_FIRST) {
+        for (u32 i = t; i < a.k; i += NT) a.out[i] = S[bt_at(skip + i)];
+        if (t == 0) {
+            a.ctrl->first.result = K0;
+            a.ctrl->first.done = 1;
+            a.ctrl->selected = a.k;
+        }
+        return;
+    }
+    // results: (index << 32 | key) of the k survivors, sorted
+    u32 gt = 0;
+    if (t < kk / 8) {
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) {
+            const u32 i = 8 * t + j;
+            const u64 c = S[bt_at(i)];
+            x[j] = i >= skip ? ((u64)(0xFFFFFFFFu - (u32)c) << 32) | (c >> 32) : ~0ull;  // the rest sorts last
+            gt += i >= skip && (u32)(c >> 32) > K0 ? 1u : 0u;
+        }
+    }
+    gt = wave_incl_scan_u32(gt);
+    if (t == 0) cnt = 0;
+    __syncthreads();
+    if ((t & (WAVE - 1)) == WAVE - 1 && gt) atomicAdd(&cnt, gt);
+    bt_sort_runs(S, x, kk, kk);
+    for (u32 i = t; i < a.k; i += NT) {
+        const u64 p = S[bt_at(i)];
+        if (a.out_keys) a.out_keys[i] = a.f32 ? KeyF32::from_ord((u32)p) : (u32)p;
+        if (a.out_idx) a.out_idx[i] = (i64)(p >> 32);
+    }
+    if (t == 0) {
+        a.ctrl->count_gt = cnt;
+        a.ctrl->ties = a.k - cnt;
+        a.ctrl->kth = K0;
+        a.ctrl->second.result = K0;
+        a.ctrl->second.done = 1;
+        if (a.d_kth) *a.d_kth = a.f32 ? KeyF32::from_ord(K0) : K0;
+    }
+}
+
+// All levels of one top-k: a.n composites of a.src to a.fin; B0 and B1 take the levels' runs.
+void bt_levels(BtArgs a, u64* B0, u64* B1, hipStream_t st) {
+    const int fin = a.fin;
+    u64* const result = a.out;
+    for (;;) {
+        const bool small = a.n <= 2048 ? a.kk <= 2048 : (a.src != BT_RUNS && 2 * a.kk <= 2048);
+        const u64 tile = small ? 2048 : 8192, tiles = a.n > tile ? a.n / tile : 1;
+        a.fin = tiles == 1 ? fin : BT_LEVEL;
+        a.out = tiles == 1 ? result : B0;
+        if (small) hipLaunchKernelGGL((k_bt_tile<256>), dim3((unsigned)tiles), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_bt_tile<1024>), dim3((unsigned)tiles), dim3(1024), 0, st, a);
+        if (tiles == 1) return;
+        a.n = tiles * a.kk;
+        a.src = BT_RUNS;
+        a.A = B0;
+        std::swap(B0, B1);
+    }
+}
+
+// ---------------------------------------------------------------- tile reduction (k == 8192)
 // Reduces tile b of A (T <= TILE elements) to its top-k, sorted ascending, at out[b*k, b*k + k).
 // presorted: A holds runs of k each sorted ascending (a previous level's output); odd runs are
 // loaded reversed, which gives the alternating k-runs the merge needs without sorting again.
@@ -165,7 +401,6 @@ u64* tile_levels(u64* A, u64* B, u64 n, u64 k, hipStream_t st) {
 // Top-k (ascending, at A[0..k)) of the n composites in A (n a power of two, n >= k, k a power
 // of two); B is scratch of n elements.  Returns the buffer holding the result.
 u64* bitonic_topk(u64* A, u64* B, u64 n, u64 k, hipStream_t st) {
-    if (k <= BT_SMALL / 4) return tile_levels<BT_SMALL, BTT_SMALL>(A, B, n, k, st);
     if (k <= BT / 2) return tile_levels<BT, BTT>(A, B, n, k, st);
     // global network
     hipLaunchKernelGGL(k_bt_sort_lds, dim3((unsigned)(n / BT)), dim3(BTT), 0, st, A, (u64)(BT / 2));
@@ -293,6 +528,23 @@ hipError_t launch_bitonic(const BitonicArgs& a, hipStream_t st) {
     const u64 k = a.k;
     u64* A = a.bufA;
     u64* B = a.bufB;
+    if (k <= BT_KMAX) {
+        BtArgs t = {};
+        t.k = (u32)k;
+        t.kk = (u32)std::max<u64>(k, 8);
+        t.dvals = a.dvals; t.S = a.S; t.keys = a.keys; t.nkeys = a.n; t.alpha = a.alpha; t.f32 = a.f32; t.ctrl = a.ctrl;
+        t.nv = a.n;
+        if (a.alpha > 0) {
+            t.n = a.npad1; t.src = BT_DELEG; t.fin = BT_FIRST; t.out = a.dsel;
+            bt_levels(t, A, B, st);
+            t.D = a.dsel;
+            t.nv = k << a.alpha;
+        }
+        t.n = a.npad2; t.src = BT_KEYS; t.fin = BT_LAST; t.out = nullptr;
+        t.out_keys = (u32*)a.out_keys; t.out_idx = a.out_idx; t.d_kth = (u32*)a.d_kth;
+        bt_levels(t, A, B, st);
+        return hipGetLastError();
+    }
     const u64* top = nullptr;  // top-k delegate composites
     u64 nv, npad;
     if (a.alpha > 0) {
