@@ -1,4 +1,4 @@
-"""Autotuner of the batched form: picks alpha, digit width and delegate-pass tile per
+"""Autotuner of the batched form: picks alpha and the delegate-pass tile per
 (ceil log2 n, ceil log2 k) cell and writes the table drtopk_batch_plan takes.
 
     python -m drtopksc_amd.autotune --out drtopksc_amd/tuning/mi355x.json
@@ -8,8 +8,8 @@ whose keys spread differently over the radix digits) and every cell in the batch
 range (n 2^12..2^22, k 1..4096) it builds a batch of `rows` rows of that type whose n and k fall
 in that cell, times drtopk_select_batched (HIP events on the launch stream, median of `reps`)
 for each candidate, checks that every candidate returns the same outputs, and keeps the fastest.
-Candidates: alpha in policy-2 .. policy+2 (the planner lowers invalid ones), 4- or 8-bit
-digits, tiles of 2^13 or 2^15 keys.  Rows of one cell share a batch, so a cell's time is its
+Candidates: alpha in policy-2 .. policy+2 (the planner lowers invalid ones), tiles of 2^13 or
+2^15 keys (the digit width no longer matters to the batched kernels and stays 8).  Rows of one cell share a batch, so a cell's time is its
 throughput when batched with its own kind.
 
 The result is JSON: {"device": ..., "cells": [[dtype, log2n, log2k, alpha, digit_bits, tile_log2], ...]};
@@ -249,7 +249,7 @@ def main(argv=None):
                 best = None
                 ref = None
                 for a in range(max(0, a0 - 2), a0 + 3):
-                    for nb in (4, 8):
+                    for nb in (8,):  # no kernel of the batched form depends on it
                         for tl in (13, 15):
                             if a > tl:
                                 continue

@@ -10,8 +10,8 @@
 //             fixed-size tiles of all rows, 16-byte loads, eight in flight per lane.
 //             It is the only kernel that reads all keys.
 //  k_brows    one workgroup per row (persistent, rows taken largest-first from a queue):
-//             first top-k over the row's delegates (exact k-th largest delegate by radix
-//             digits), range selection (every subrange whose delegate is greater, then the
+//             first top-k over the row's delegates (exact k-th largest delegate), range
+//             selection (every subrange whose delegate is greater, then the
 //             lowest-ID ties up to k, radixselect.cuh:413-427 / :603-618), filtered
 //             concatenation of those subranges (keys >= threshold, radixselect.cuh:1575-1607)
 //             into LDS, second top-k over it and the index-ordered extraction of the
@@ -34,6 +34,7 @@
 #include "../../include/drtopk.h"
 #include "common.hpp"
 #include "host_util.hpp"
+#include "wgselect.hpp"
 
 namespace drtopk {
 namespace {
@@ -66,7 +67,7 @@ struct BatchRow {
                     // and as many row indices
     u32 S;          // subranges (0 when alpha == 0)
     u32 chunk_begin, nchunks;
-    u8 alpha, f32, nb, tile_log2;
+    u8 alpha, f32, nb, tile_log2;  // nb: as tuned, no kernel depends on it
 };
 static_assert(sizeof(BatchRow) == 64, "row layout");
 
@@ -103,8 +104,6 @@ __device__ __forceinline__ u32 group_max_last(u32 m, int g) {
     if (g >= 64) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x143, 0xC, 0xF, false));  // row_bcast:31
     return m;
 }
-
-__device__ __forceinline__ u32 max4(const u32x4& v) { return max(max(v[0], v[1]), max(v[2], v[3])); }
 
 constexpr u32 BS_WKEYS = BS_UNR * WAVE * 4;  // keys per wave per batch (2048)
 constexpr u32 BS_BATCH = BS_WKEYS * (BS_NT / WAVE);  // keys per workgroup per batch (8192)
@@ -240,8 +239,13 @@ __global__ __launch_bounds__(BS_NT) void k_bsample(const unsigned char* __restri
 // ---------------------------------------------------------------- per-row workgroup
 constexpr int BR_NT = 512;
 constexpr int BR_W = BR_NT / WAVE;
-constexpr u32 REG_WORDS = 12288;       // 48 KB: candidate list or concatenation cache
-constexpr u32 CONCAT_CAP = REG_WORDS / 2;  // keys + row indices
+// 56 KB: a row's delegates, then its concatenation (keys and row indices).  With the rest of RowLds two
+// workgroups fit a CU.
+constexpr u32 REG_WORDS = wg_words<BR_NT>(14336);
+constexpr u32 STAGE_CAP = 14336;  // delegates (or keys of a row without them) selected in LDS
+constexpr u32 CONCAT_CAP = 6144;  // keys + row indices; an odd number of granules per thread
+static_assert(2 * CONCAT_CAP <= REG_WORDS && wg_words<BR_NT>(CONCAT_CAP) == CONCAT_CAP, "concatenation in LDS");
+constexpr u32 SEL_CAP = 4096;  // selected subranges listed in LDS (ids below STAGE_CAP)
 
 // Sources: a sequence of E slots read four at a time (e a multiple of 4); each slot yields
 // an ordered key, its row index (or element index) and a valid bit.
@@ -316,15 +320,17 @@ struct SrcV {
     const u32* row;
     u64 n;
     const u32* sel;
+    const u16* lsel;  // the list in LDS, or null
     int alpha;
     int f32;
     u32 lo;
     u64 E;  // slots (alpha == 1 reads the id list slot by slot and must stop at E)
+    __device__ __forceinline__ u64 id(u64 i) const { return lsel ? (u32)lsel[i] : sel[i]; }
     __device__ __forceinline__ u32 cvt(u32 b) const { return f32 ? KeyF32::to_ord(b) : b; }
     __device__ __forceinline__ u32 load4(u64 e, u32* x, u32* ix) const {
         u32 v = 0;
         if (alpha != 1) {
-            const u64 base = alpha == 0 ? e : (((u64)sel[e >> alpha] << alpha) | (e & ((1ull << alpha) - 1)));
+            const u64 base = alpha == 0 ? e : ((id(e >> alpha) << alpha) | (e & ((1ull << alpha) - 1)));
             if (base + 4 <= n) {
                 const u32x4 q = *(const u32x4*)(row + base);
                 x[0] = q[0]; x[1] = q[1]; x[2] = q[2]; x[3] = q[3];
@@ -343,7 +349,7 @@ struct SrcV {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const u64 ee = e + j;
-                const u64 base = ee < E ? (((u64)sel[ee >> 1] << 1) | (ee & 1)) : n;
+                const u64 base = ee < E ? ((id(ee >> 1) << 1) | (ee & 1)) : n;
                 const bool ok = base < n;
                 x[j] = ok ? row[base] : 0u;
                 ix[j] = (u32)base;
@@ -366,7 +372,7 @@ struct SrcV {
     // per-lane condition (such a load is waited for where the branches join); only a granule
     // that runs past the row's end (its last subrange) is re-read key by key.
     __device__ __forceinline__ u32 load4_fast(u64 e, u32* x, u32* ix) const {
-        const u64 base = alpha == 0 ? e : (((u64)sel[e >> alpha] << alpha) | (e & ((1ull << alpha) - 1)));
+        const u64 base = alpha == 0 ? e : ((id(e >> alpha) << alpha) | (e & ((1ull << alpha) - 1)));
         const u64 bc = base + 4 <= n ? base : ((n - 4) & ~3ull);
         const u32x4 q = *(const u32x4*)(row + bc);
         x[0] = q[0]; x[1] = q[1]; x[2] = q[2]; x[3] = q[3];
@@ -396,262 +402,290 @@ constexpr int BR_U = 4;
 constexpr u64 BR_STEP = (u64)BR_NT * 4 * BR_U;
 
 struct RowLds {
-    u32 hist[BR_W * 256];
-    u64 scan[BR_W + 1];
-    u32 misc[16];
+    WgSel<BR_NT> sel;
+    u32 scan[BR_W];
+    u32 queue;
+    u16 ids[SEL_CAP];
 };
 
-// One granule of a digit pass: its valid keys under the prefix counted in the wave's histogram
-// (and, with gather, listed as candidates).
-__device__ __forceinline__ void hist_step(const u32 (&x)[4], u32 v, u32 mask, u32 prefix, int shift, int R, u32* wh,
-                                          bool gather, u32* cand, u32 cap, RowLds& L) {
+// The slots [0, E) of src, each wave a contiguous share of whole 256-slot rows, four rows in flight:
+// f(x, ix, valid bits) for every four slots, every lane of the wave at once, with no barrier.
+template <class Src, class F>
+__device__ __forceinline__ void src_each(const Src& src, u64 E, F&& f) {
+    constexpr u32 ROW = 4 * WAVE;
+    const u32 lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    const u64 per = (E + BR_W * ROW - 1) / (BR_W * ROW) * ROW;
+    u64 e = min(E, w * per);
+    const u64 e1 = min(E, e + per), eb = min(e1, src.bulk_end(E, 4));
+    for (; e + BR_U * ROW <= eb; e += BR_U * ROW) {
+        u32 x[BR_U][4], ix[BR_U][4], v[BR_U];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const bool act = ((v >> j) & 1u) && (x[j] & mask) == prefix;
-        wave_hist_add(wh, act, (x[j] >> shift) & (R - 1));
-        if (gather && act) {
-            const u32 p = atomicAdd(&L.misc[0], 1u);
-            if (p < cap) cand[p] = x[j];
-        }
+        for (u32 u = 0; u < BR_U; ++u) v[u] = src.load4_fast(e + u * ROW + 4 * lane, x[u], ix[u]);
+#pragma unroll
+        for (u32 u = 0; u < BR_U; ++u) f(x[u], ix[u], v[u]);
+    }
+    for (; e < e1; e += ROW) {
+        u32 x[4] = {0, 0, 0, 0}, ix[4];
+        const u32 v = e + 4 * lane < e1 ? src.load4(e + 4 * lane, x, ix) : 0u;
+        f(x, ix, v);
     }
 }
 
-// k-th largest (ascending rank m-k) of the valid slots of src by radix digits of nb bits,
-// most significant first.  With `gather`, once the candidates of the current prefix fit in
-// cand[0..cap) the next pass copies them there and the remaining digits run on LDS.
-// Returns the key; *gt = valid slots strictly greater.
-template <class Src>
-__device__ __forceinline__ u32 wg_kth(const Src& src, u64 E, u64 k, int nb, bool gather_ok, u32* cand, u32 cap, RowLds& L,
-                      u64* gt_out) {
-    const int t = threadIdx.x, w = t / WAVE, lane = t & (WAVE - 1);
-    const int R = 1 << nb;
-    u32 prefix = 0, mask = 0;
-    u64 kk = k, gt = 0;
-    bool in_cand = false, gather = gather_ok && E <= cap;
-    u32 mc = 0;
-    if (t == 0) L.misc[0] = 0;  // gather counter
-    for (int shift = 32 - nb; shift >= 0; shift -= nb) {
-        for (int i = t; i < BR_W * R; i += BR_NT) L.hist[(i / R) * 256 + (i % R)] = 0;
-        __syncthreads();
-        u32* wh = L.hist + w * 256;
-        if (in_cand) {
-            for (u32 i0 = 0; i0 < mc; i0 += BR_NT) {
-                const u32 i = i0 + t;
-                const u32 x = i < mc ? cand[i] : 0u;
-                wave_hist_add(wh, i < mc && (x & mask) == prefix, (x >> shift) & (R - 1));
-            }
-        } else {
-            const u64 Eb = src.bulk_end(E, BR_STEP);
-            for (u64 e0 = 0; e0 < Eb; e0 += BR_STEP) {  // whole steps: every load issued before use
-                u32 x[BR_U][4], ix[BR_U][4], v[BR_U];
-#pragma unroll
-                for (int u = 0; u < BR_U; ++u) v[u] = src.load4_fast(e0 + ((u64)u * BR_NT + t) * 4, x[u], ix[u]);
-#pragma unroll
-                for (int u = 0; u < BR_U; ++u) hist_step(x[u], v[u], mask, prefix, shift, R, wh, gather, cand, cap, L);
-            }
-            for (u64 e0 = Eb; e0 < E; e0 += (u64)BR_NT * 4) {
-                const u64 e = e0 + (u64)t * 4;
-                u32 x[4], ix[4];
-                const u32 v = e < E ? src.load4(e, x, ix) : 0u;
-                hist_step(x, v, mask, prefix, shift, R, wh, gather, cand, cap, L);
-            }
-        }
-        __syncthreads();
-        if (gather) {
-            in_cand = true;
-            gather = false;
-            mc = min(L.misc[0], cap);
-        }
-        if (t < R) {
-            u32 s = 0;
-            for (int q = 0; q < BR_W; ++q) s += L.hist[q * 256 + t];
-            L.hist[t] = s;
-        }
-        __syncthreads();
-        if (w == 0) {
-            // bins from the top: lane l holds bins R-1-l*bpl ... R-(l+1)*bpl
-            const int bpl = R >= WAVE ? R / WAVE : 1;
-            u32 c[4] = {0, 0, 0, 0};
-            u64 s = 0;
-            for (int j = 0; j < bpl; ++j) {
-                const int b = R - 1 - lane * bpl - j;
-                c[j] = b >= 0 ? L.hist[b] : 0u;
-                s += c[j];
-            }
-            const u64 inc = wave_incl_scan_u64(s);
-            const u64 bal = __ballot(inc >= kk);
-            const int fl = bal ? __ffsll((unsigned long long)bal) - 1 : 0;
-            if (lane == fl) {
-                u64 above = inc - s;
-                int bin = R - 1 - lane * bpl - (bpl - 1);
-                u32 cnt = c[bpl - 1];
-                for (int j = 0; j < bpl; ++j) {
-                    if (above + c[j] >= kk) {
-                        bin = R - 1 - lane * bpl - j;
-                        cnt = c[j];
-                        break;
-                    }
-                    above += c[j];
-                }
-                L.misc[2] = (u32)bin;
-                L.misc[3] = cnt;
-                L.misc[4] = (u32)above;
-                L.misc[5] = (u32)(above >> 32);
-            }
-        }
-        __syncthreads();
-        const u32 bin = L.misc[2], cnt = L.misc[3];
-        const u64 above = (u64)L.misc[4] | ((u64)L.misc[5] << 32);
-        prefix |= bin << shift;
-        mask |= (u32)(R - 1) << shift;
-        kk -= above;
-        gt += above;
-        if (!in_cand && gather_ok && cnt <= cap && shift > 0) gather = true;
-    }
-    *gt_out = gt;
-    return prefix;
-}
-
-// Ordered pass: calls emit(pos, key, index) for every valid slot with key > K and for the
-// first `ties` valid slots with key == K (ALL: every valid slot), pos = rank among those
-// emitted, in slot order.  Returns the number of valid slots > K (ALL: valid slots).
-// One step of wg_ordered: thread t holds granules t*U .. t*U+U-1 of the step, so one block scan
-// ranks all of them in slot order.
-template <bool ALL, int U, class F>
-__device__ __forceinline__ void ordered_step(const u32 (&x)[U][4], const u32 (&ix)[U][4], const u32 (&v)[U], u32 K,
-                                             u64 ties, RowLds& L, u64& gt_run, u64& eq_run, F& emit) {
+// Top-k of an array that LDS does not hold: the k-th largest valid slot K of src, then emit(pos, key,
+// index) for those above it and the first ties, pos = rank among the emitted in slot order.
+template <class Src, class F>
+__device__ __forceinline__ u32 src_topk(const Src& src, u64 E, u32 k, RowLds& L, F emit) {
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    u32 gt;
+    const u32 K = wg_kth<BR_NT>(
+        [&](auto&& f) {
+            src_each(src, E, [&](const u32 (&x)[4], const u32 (&)[4], u32 v) {
+                f(u32x4{v & 1 ? x[0] : 0u, v & 2 ? x[1] : 0u, v & 4 ? x[2] : 0u, v & 8 ? x[3] : 0u});
+            });
+        },
+        k, L.sel, &gt);
     u32 g = 0, q = 0;
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const bool ok = (v[u] >> j) & 1u;
-            g += (ok && (ALL || x[u][j] > K)) ? 1u : 0u;
-            q += (!ALL && ok && x[u][j] == K) ? 1u : 0u;
-        }
-    u64 tot;
-    const u64 ex = block_excl_scan_u64<BR_NT>(((u64)q << 32) | g, L.scan, &tot);
-    u64 gb = gt_run + (u32)ex, qb = eq_run + (ex >> 32);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
+    src_each(src, E, [&](const u32 (&x)[4], const u32 (&)[4], u32 v) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            if (!((v[u] >> j) & 1u)) continue;
-            if (ALL || x[u][j] > K) {
-                emit(gb + min(qb, ties), x[u][j], ix[u][j]);
-                ++gb;
-            } else if (x[u][j] == K) {
-                if (qb < ties) emit(gb + qb, x[u][j], ix[u][j]);
-                ++qb;
-            }
+            g += (v >> j & 1) && x[j] > K ? 1u : 0u;
+            q += (v >> j & 1) && x[j] == K ? 1u : 0u;
         }
-    gt_run += (u32)tot;
-    eq_run += tot >> 32;
+    });
+    g = wave_incl_scan_u32(g);
+    q = wave_incl_scan_u32(q);
+    __syncthreads();
+    if (lane == WAVE - 1) {
+        L.sel.a[w] = g;
+        L.sel.b[w] = q;
+    }
+    __syncthreads();
+    const u32 ties = k - gt;
+    u32 tot;
+    g = wave_totals_prefix<BR_NT>(L.sel.a, &tot);
+    q = wave_totals_prefix<BR_NT>(L.sel.b, &tot);
+    src_each(src, E, [&](const u32 (&x)[4], const u32 (&ix)[4], u32 v) {
+        u32 mine = 0;  // above << 16 | ties
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mine += (v >> j & 1) ? (x[j] > K ? 0x10000u : (x[j] == K ? 1u : 0u)) : 0u;
+        if (__ballot(mine != 0) == 0) return;
+        const u32 inc = wave_incl_scan_u32(mine);
+        u32 gb = g + ((inc - mine) >> 16), qb = q + ((inc - mine) & 0xFFFFu);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const bool isg = (v >> j & 1) && x[j] > K, isq = (v >> j & 1) && x[j] == K;
+            if (isg || (isq && qb < ties)) emit(gb + min(qb, ties), x[j], ix[j]);
+            gb += isg ? 1u : 0u;
+            qb += isq ? 1u : 0u;
+        }
+        const u32 all = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+        g += all >> 16;
+        q += all & 0xFFFFu;
+    });
+    return K;
 }
 
-template <bool ALL, class Src, class F>
-__device__ __forceinline__ u64 wg_ordered(const Src& src, u64 E, u32 K, u64 ties, RowLds& L, F emit) {
+// Ordered pass: emit(pos, key, index) for every valid slot, pos = its rank in slot order.  Returns
+// their number.  In a step thread t holds granules t*BR_U .. t*BR_U+BR_U-1, so one block scan ranks them all.
+template <int U, class F>
+__device__ __forceinline__ void ordered_step(const u32 (&x)[U][4], const u32 (&ix)[U][4], const u32 (&v)[U], RowLds& L,
+                                             u32& run, F& emit) {
+    u32 c = 0, tot;
+#pragma unroll
+    for (int u = 0; u < U; ++u) c += __popc(v[u]);
+    u32 p = run + wg_excl_scan<BR_NT>(c, L.scan, &tot);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if ((v[u] >> j) & 1u) emit(p++, x[u][j], ix[u][j]);
+    run += tot;
+}
+
+template <class Src, class F>
+__device__ __forceinline__ u32 wg_ordered(const Src& src, u64 E, RowLds& L, F emit) {
     const int t = threadIdx.x;
-    u64 gt_run = 0, eq_run = 0;
+    u32 run = 0;
     const u64 Eb = src.bulk_end(E, BR_STEP);
     for (u64 e0 = 0; e0 < Eb; e0 += BR_STEP) {
         u32 x[BR_U][4], ix[BR_U][4], v[BR_U];
 #pragma unroll
         for (int u = 0; u < BR_U; ++u) v[u] = src.load4_fast(e0 + ((u64)t * BR_U + u) * 4, x[u], ix[u]);
-        ordered_step<ALL, BR_U>(x, ix, v, K, ties, L, gt_run, eq_run, emit);
+        ordered_step<BR_U>(x, ix, v, L, run, emit);
     }
     for (u64 e0 = Eb; e0 < E; e0 += (u64)BR_NT * 4) {
         const u64 e = e0 + (u64)t * 4;
         u32 x[1][4], ix[1][4], v[1];
         v[0] = e < E ? src.load4(e, x[0], ix[0]) : 0u;
-        ordered_step<ALL, 1>(x, ix, v, K, ties, L, gt_run, eq_run, emit);
+        ordered_step<1>(x, ix, v, L, run, emit);
     }
-    return gt_run;
+    return run;
 }
 
-// One row of k_brows (its index q in the processing order).  SPILL (alpha > 0 and k larger than
+// The plan's rule for a row's concatenation region (it reserves the room).
+__host__ __device__ __forceinline__ bool row_spills(int alpha, u64 k) { return alpha > 0 && k > CONCAT_CAP; }
+
+// One row of k_brows (its index q in the processing order).  `spill` (alpha > 0 and k larger than
 // the LDS concatenation cache, so the filtered concatenation of C >= k keys cannot fit it): the
 // keys that overflow the cache go to the row's workspace region after its selected ids, then the
 // cached part, and the second top-k streams those C keys instead of gathering the k << alpha
 // slots through the id list twice more.  Rows with k within the cache keep the LDS path (and,
-// when the concatenation does overflow, the re-gather), without the extra code in their loops.
-template <bool SPILL>
+// when the concatenation does overflow, the re-gather).
+//  A row is a chain of barriers, LDS round trips and about ten trips to memory, one workgroup deep, so
+// what counts is how short the chain is.  Delegates, the concatenation, and a short row itself, are
+// selected in LDS by wgselect.hpp's linear buckets (two passes where 8-bit digits took four, one scan
+// per emission); arrays that LDS does not hold are read from memory on each pass, the waves alone.  64 rows of 2^17
+// keys: 29 -> 11 us; one row of 2^22 keys, k = 4096 (65536 delegates, 2^18 concatenated slots): 98 -> 50;
+// 4096 rows of 2^12 .. 2^22 keys, two rows to a CU: 400 -> 195.
 __device__ __forceinline__ void brow(const BatchRow* rp, u32 q, const u32* __restrict__ keys, BatchWs* wsh,
                                      const u32* __restrict__ deleg, u32* __restrict__ selws,
                                      u32* __restrict__ kth_out, u32* __restrict__ out_keys, i64* __restrict__ out_idx,
                                      RowLds& L, u32* reg) {
     const int t = threadIdx.x;
     const u64 n = rp->n, k = rp->k, out_off = rp->out_off;
-    const int a = rp->alpha, nb = rp->nb, f32 = rp->f32;
+    const int a = rp->alpha, f32 = rp->f32;
     const u32* row = keys + rp->key_off;
     u32* sel = selws + rp->sel_off;
-
-    // first top-k over the delegates and range selection
-    u32 T = 0;
-    u64 E = n;
-    if (a > 0) {
-        const SrcG dg{deleg + rp->deleg_off, rp->S};
-        u64 g = 0;
-        T = wg_kth(dg, rp->S, k, nb, true, reg, REG_WORDS, L, &g);
-        const u64 ties = k - g;
-        wg_ordered<false>(dg, rp->S, T, ties, L, [&](u64 p, u32, u32 id) {
-            if (p < k) sel[p] = id;
+    auto emit_out = [&](u32 p, u32 x, u32 ix) {
+        if (p < k) {
+            if (out_keys) out_keys[out_off + p] = f32 ? KeyF32::from_ord(x) : x;
+            if (out_idx) out_idx[out_off + p] = (i64)ix;
+        }
+    };
+    auto each = [&](int ni) { return [=](auto&& f) { wg_each(reg, ni, f); }; };
+    // m words from p (16-byte aligned) into reg, 0 past them
+    auto stage = [&](const u32* p, u32 m, bool conv) {
+        const int ni = wg_granules<BR_NT>(m);
+        wg_stage<BR_NT>(reg, ni, [&](u32 e) {
+            u32x4 x = {0, 0, 0, 0};
+            if (e + 4 <= m) {
+                x = *(const u32x4*)(p + e);
+                if (conv)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) x[j] = KeyF32::to_ord(x[j]);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (e + j < m) x[j] = conv ? KeyF32::to_ord(p[e + j]) : p[e + j];
+            }
+            return x;
         });
+        return ni;
+    };
+
+    u32 T = 0, gt32;
+    u64 E = n;
+    const u16* lsel = nullptr;
+    wg_init<BR_NT>(L.sel);
+    const bool spill = row_spills(a, k);
+    if (a == 0 && n <= STAGE_CAP) {  // no delegates: the keys themselves
+        const int ni = stage(row, (u32)n, f32);
+        const u32 K = wg_kth<BR_NT>(each(ni), (u32)k, L.sel, &gt32);
+        wg_emit<BR_NT>(reg, ni, K, gt32, (u32)k - gt32, L.sel, [&](u32 p, u32 e, u32 x) { emit_out(p, x, e); });
+        if (t == 0 && kth_out) kth_out[q] = f32 ? KeyF32::from_ord(K) : K;
+        return;
+    }
+    // first top-k over the delegates and range selection
+    if (a > 0) {
+        const u32* dg = deleg + rp->deleg_off;
+        const u32 S = rp->S;
+        if (S <= STAGE_CAP) {
+            const int ni = stage(dg, S, false);
+            T = wg_kth<BR_NT>(each(ni), (u32)k, L.sel, &gt32);
+            const bool held = k <= SEL_CAP;
+            wg_emit<BR_NT>(reg, ni, T, gt32, (u32)k - gt32, L.sel, [&](u32 p, u32 e, u32) {
+                if (p < k) {
+                    if (held) L.ids[p] = (u16)e;
+                    else sel[p] = e;
+                }
+            });
+            if (held) lsel = L.ids;
+        } else {
+            T = src_topk(SrcG{dg, S}, S, (u32)k, L, [&](u32 p, u32, u32 id) {
+                if (p < k) sel[p] = id;
+            });
+        }
         __syncthreads();
         E = k << a;
     }
     // filtered concatenation, cached in LDS when it fits
-    const SrcV vs{row, n, sel, a, f32, T, E};
+    const SrcV vs{row, n, sel, lsel, a, f32, T, E};
     u32* ckey = reg;
     u32* cidx = reg + CONCAT_CAP;
-    u32* gck = sel + ((k + 3) & ~3ull);  // SPILL: room for E keys, then E indices
+    u32* gck = sel + ((k + 3) & ~3ull);  // spill: room for E keys, then E indices
     u32* gci = gck + ((E + 3) & ~3ull);
-    const u64 C = wg_ordered<true>(vs, E, 0u, 0, L, [&](u64 p, u32 x, u32 ix) {
-        if (p < CONCAT_CAP) {
-            ckey[p] = x;
-            cidx[p] = ix;
-        } else if (SPILL) {  // p < C <= E
-            gck[p] = x;
-            gci[p] = ix;
+    u32 C = 0;
+    int ni = 0;
+    if (!spill && T > 0 && E > BR_STEP) {
+        // Long (more than one step of the ordered pass) and sparse: each wave lists what it finds in its share of the slots in a segment of its
+        // own, with no barrier between loads, and zeros fill the segments (no key here is 0).
+        constexpr u32 SEG = CONCAT_CAP / BR_W;
+        const u32 lane = t & (WAVE - 1), w = t / WAVE;
+        for (u32 i = t; i < CONCAT_CAP; i += BR_NT) ckey[i] = 0;
+        __syncthreads();
+        u32 fill = 0;
+        src_each(vs, E, [&](const u32 (&x)[4], const u32 (&ix)[4], u32 v) {
+            if (__ballot(v != 0) == 0) return;
+            const u32 c = __popc(v), inc = wave_incl_scan_u32(c);
+            u32 p = fill + inc - c;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (v >> j & 1) {
+                    if (p < SEG) {
+                        ckey[w * SEG + p] = x[j];
+                        cidx[w * SEG + p] = ix[j];
+                    }
+                    ++p;
+                }
+            fill += (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+        });
+        if (lane == 0) L.scan[w] = fill;
+        __syncthreads();
+        const u32 mine = L.scan[lane & (BR_W - 1)];
+        if (__ballot(mine > SEG) == 0) {
+            wave_totals_prefix<BR_NT>(L.scan, &C);
+            ni = wg_granules<BR_NT>(CONCAT_CAP);
         }
-    });
-    __syncthreads();
+        __syncthreads();
+    }
+    if (ni == 0) {
+        C = wg_ordered(vs, E, L, [&](u32 p, u32 x, u32 ix) {
+            if (p < CONCAT_CAP) {
+                ckey[p] = x;
+                cidx[p] = ix;
+            } else if (spill) {  // p < C <= E
+                gck[p] = x;
+                gci[p] = ix;
+            }
+        });
+        if (C <= CONCAT_CAP) {
+            ni = wg_granules<BR_NT>(C) | 1;  // odd: the threads' shares lie end to end
+            for (u32 i = C + t; i < (u32)ni * 4 * BR_NT; i += BR_NT) ckey[i] = 0;
+        }
+        __syncthreads();
+    }
     // every key of the top-k set is >= T, so the concatenation holds at least k keys
     if (C < k) {
         if (t == 0) ws_fail(&wsh->head, ERR_CONCAT_SHORT);
         return;
     }
     // second top-k and extraction
-    u64 gt = 0;
     u32 K;
-    auto emit_out = [&](u64 p, u32 x, u32 ix) {
-        if (p < k) {
-            if (out_keys) out_keys[out_off + p] = f32 ? KeyF32::from_ord(x) : x;
-            if (out_idx) out_idx[out_off + p] = (i64)ix;
-        }
-    };
-    if (C <= CONCAT_CAP) {
-        const SrcL ls{ckey, cidx, C};
-        K = wg_kth(ls, C, k, nb, false, nullptr, 0, L, &gt);
-        wg_ordered<false>(ls, C, K, k - gt, L, emit_out);
-    } else if (SPILL) {
+    if (ni) {
+        K = wg_kth<BR_NT>(each(ni), (u32)k, L.sel, &gt32);
+        wg_emit<BR_NT>(reg, ni, K, gt32, (u32)k - gt32, L.sel, [&](u32 p, u32 e, u32 x) { emit_out(p, x, cidx[e]); });
+    } else if (spill) {
         for (u32 i = t; i < CONCAT_CAP; i += BR_NT) {
             gck[i] = ckey[i];
             gci[i] = cidx[i];
         }
-        __syncthreads();  // the LDS cache is free again: it takes the digit passes' candidates
-        const SrcL gs{gck, gci, C};
-        K = wg_kth(gs, C, k, nb, true, reg, REG_WORDS, L, &gt);
-        wg_ordered<false>(gs, C, K, k - gt, L, emit_out);
+        __syncthreads();
+        K = src_topk(SrcL{gck, gci, C}, C, (u32)k, L, emit_out);
     } else {
-        K = wg_kth(vs, E, k, nb, true, reg, REG_WORDS, L, &gt);
-        wg_ordered<false>(vs, E, K, k - gt, L, emit_out);
+        K = src_topk(vs, E, (u32)k, L, emit_out);
     }
     if (t == 0 && kth_out) kth_out[q] = f32 ? KeyF32::from_ord(K) : K;
 }
-
-// The plan's rule for a row's concatenation region (it reserves the room).
-__host__ __device__ __forceinline__ bool row_spills(int alpha, u64 k) { return alpha > 0 && k > CONCAT_CAP; }
 
 // Four waves per SIMD (two workgroups per CU): the row body needs a few more registers than that
 // allows unbounded, and halving the resident rows costs more than the bound does.
@@ -668,15 +702,12 @@ __global__ __launch_bounds__(BR_NT, 4) void k_brows(const unsigned char* __restr
     const int t = threadIdx.x;
     for (;;) {
         __syncthreads();
-        if (t == 0) L.misc[15] = atomicAdd(&wsh->queue, 1u);
+        if (t == 0) L.queue = atomicAdd(&wsh->queue, 1u);
         __syncthreads();
-        const u32 q = L.misc[15];
+        const u32 q = L.queue;
         if (q >= nrows) break;
         const BatchRow* rp = rows + order[q];
-        if (row_spills(rp->alpha, rp->k))
-            brow<true>(rp, order[q], keys, wsh, deleg, selws, kth_out, out_keys, out_idx, L, reg);
-        else
-            brow<false>(rp, order[q], keys, wsh, deleg, selws, kth_out, out_keys, out_idx, L, reg);
+        brow(rp, order[q], keys, wsh, deleg, selws, kth_out, out_keys, out_idx, L, reg);
     }
 }
 
