@@ -518,16 +518,18 @@ drtopk_status drtopk_server_submit(drtopk_server* s, const drtopk_query* q, uint
     if (need == ~0ull || align_up(need, 256) + ob > s->cfg.budget_bytes)
         return fail(DRTOPK_ERR_BUDGET, "request needs %llu bytes, the arena holds %llu",
                     (unsigned long long)(need + ob), (unsigned long long)s->cfg.budget_bytes);
-    std::lock_guard<std::mutex> lk(s->mu);
-    const u64 t = s->next_ticket++;
     Req r;
     r.q = *q;
     r.need = align_up(need, 256) + ob;
-    r.t_submit = now_ns();
-    s->reqs.emplace(t, r);
-    s->queue.push_back(t);
-    *ticket = t;
-    s->cv_work.notify_one();
+    {
+        std::lock_guard<std::mutex> lk(s->mu);
+        const u64 t = s->next_ticket++;
+        r.t_submit = now_ns();
+        s->reqs.emplace(t, r);
+        s->queue.push_back(t);
+        *ticket = t;
+    }
+    s->cv_work.notify_one();  // without the lock, which the woken worker takes at once
     return DRTOPK_OK;
 }
 
