@@ -47,7 +47,9 @@ REF_ABLATION_2P29_K2P24_MS = {  # baseline{,+filter,+filter+shuffle}/U_OptimumFI
 
 
 def bytes_build(st: dict, n: int, k: int) -> int:
-    """This build's algorithmic bytes for one top-k: what each pass must move at least.
+    """The general pipeline's algorithmic bytes for one top-k: what each pass must move at least.  (The
+    statistics are that pipeline's; a timed call asks for none and may take a shorter pipeline, which
+    moves fewer bytes for the same result.)
     - 4n: the delegate pass reads V once;
     - 4D: the delegate write;
     - 4D per first-top-k pass that reads the delegates (digit passes after the first, whose
