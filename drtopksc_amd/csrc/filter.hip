@@ -37,10 +37,15 @@ constexpr u32 F_CLASSES = 512;  // 2b: between splitters b-1 and b; 2b+1: equal 
 constexpr u32 F_ABOVE = F_CLASSES - 1;
 constexpr u32 F_SPLIT = 254;  // so that no splitter's class is 511
 constexpr int F_REPS = 4;         // replicas of the class counters
+constexpr u32 F_BATCH = WG * 8; // kept keys a workgroup takes at a time in k_fpick and k_fwrite
+// Whether a range's units go to waves that work alone instead of to the workgroup in batches: sorted or
+// clustered keys fill the units of few ranges (2^26 ascending keys, k = 2^16: k_fpick 161 -> 24 us, k_fwrite
+// 238 -> 67).  A unit with few kept keys is not worth a wave (2^28 keys, the top ones 1 in 256 of a
+// sixteenth: 380 us for the call, 219 in batches).
+__device__ __forceinline__ bool range_dense(u32 tot, u32 units) { return tot > max(2 * F_BATCH, 256 * units); }
 constexpr u32 F_SORT = 512;       // samples above the bound that are put in order at once
 constexpr u32 F_STAGE = 512;    // kept keys a wave stages in LDS
 constexpr u32 F_LISTS = 64;     // sublists of the class, so that their cursors do not serialise
-constexpr u32 F_BATCH = WG * 8; // kept keys a workgroup takes at a time in k_fpick and k_fwrite
 
 enum : u32 { F_CLASS = 0, F_AT_T = 1, F_DONE = 2 };
 
@@ -69,6 +74,11 @@ __host__ __device__ __forceinline__ u32 sample_pos(u32 i, u64 n, int lm) {
     return b + (u32)(((u64)h * (e - b)) >> 32);
 }
 
+// The stratum of the sample at slot s: those whose maximum is taken together lie far apart, as keys in a
+// sorted or clustered vector are large together (2^28 ascending keys, k = 2^24: the list of k_fsplit took
+// eight samples for each it needed and overflowed).
+__device__ __forceinline__ u32 sample_stratum(u32 s, int lm) { return (s * 0x9E3779B1u) & ((1u << lm) - 1); }
+
 template <class K>
 __global__ __launch_bounds__(WG) void k_fsample(const u32* __restrict__ keys, u64 n, int lm, u32* __restrict__ sample,
                                                 u32* __restrict__ sup, Ctrl* ctrl, FilterState* st,
@@ -76,7 +86,7 @@ __global__ __launch_bounds__(WG) void k_fsample(const u32* __restrict__ keys, u6
     const u32 g = blockIdx.x * WG + threadIdx.x;  // 2^lm / 4 threads, at least 2048
     u32x4 v;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = keys[sample_pos(4 * g + j, n, lm)];
+    for (int j = 0; j < 4; ++j) v[j] = keys[sample_pos(sample_stratum(4 * g + j, lm), n, lm)];
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = K::to_ord(v[j]);
     *(u32x4*)(sample + 4 * g) = v;
@@ -546,7 +556,42 @@ __global__ __launch_bounds__(WG) void k_fpick(FilterState* st, const u32* __rest
     }
     const bool known = f.hi - f.lo == 1;  // one value: counted, not listed
     u32 g = 0, q = 0;
-    for (u32 e0 = 0; e0 < tot; e0 += F_BATCH) {
+    const bool dense = range_dense(tot, u1 - u0);
+    if (dense) {  // uniform; each unit by a wave alone
+        const u32 lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+        for (u32 i = w; i < u1 - u0; i += WG / WAVE) {
+            const u32 c = R.pref[i + 1] - R.pref[i], from = R.base[i];
+            for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
+                u32 x[8], in = 0;
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u) x[u] = skeys[from + min(j0 + u * WAVE + lane, c - 1)];
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u) {
+                    if (j0 + u * WAVE + lane >= c) x[u] = 0;  // neither above nor in the class
+                    g += x[u] > f.hi ? 1u : 0u;
+                    in += x[u] > f.lo && x[u] <= f.hi ? 1u : 0u;
+                }
+                q += in;
+                if (known) continue;
+                const u32 inc = wave_incl_scan_u32(in), n = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+                if (n == 0) continue;  // uniform over the wave
+                const u32 list = (r + 4 * i + j0 / (8 * WAVE)) % F_LISTS;
+                u32 b = 0;
+                if (lane == 0) b = atomicAdd(&st->lcount[list], n);
+                u32 to = (u32)__builtin_amdgcn_readfirstlane((int)b) + inc - in;
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u)
+                    if (x[u] > f.lo && x[u] <= f.hi) {
+                        if (to < lcap) {
+                            lkey[list * lcap + to] = x[u];
+                            lrange[list * lcap + to] = r;
+                        }
+                        ++to;
+                    }
+            }
+        }
+    }
+    for (u32 e0 = dense ? tot : 0; e0 < tot; e0 += F_BATCH) {
         u32 at[8], x[8], in = 0;
         range_slots(R, e0 + 8 * threadIdx.x, tot, at);
 #pragma unroll
@@ -880,6 +925,62 @@ __global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nunits
         }
         return;
     }
+    if (range_dense(tot, u1 - u0)) {  // each unit by a wave alone: counted, then written
+        const u32 lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+        for (u32 i = w; i < u1 - u0; i += WG / WAVE) {
+            const u32 c = R.pref[i + 1] - R.pref[i], from = R.base[i];
+            u32 m = 0;  // above << 16 | ties
+            for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
+                u32 x[8];
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u) x[u] = skeys[from + min(j0 + u * WAVE + lane, c - 1)];
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u)
+                    m += j0 + u * WAVE + lane < c ? (x[u] > K0 ? 0x10000u : (x[u] == K0 ? 1u : 0u)) : 0u;
+            }
+            m = wave_incl_scan_u32(m);
+            if (lane == WAVE - 1) sk[i] = m;
+        }
+        __syncthreads();
+        const u32 m = threadIdx.x < u1 - u0 ? sk[threadIdx.x] : 0u;
+        u32 all;
+        const u32 gx = wg_excl_scan<WG>(m >> 16, R.scratch, &all), qx = wg_excl_scan<WG>(m & 0xFFFFu, R.scratch, &all);
+        if (threadIdx.x < F_RUNITS) {
+            sk[threadIdx.x] = g + gx;
+            si[threadIdx.x] = q + qx;
+        }
+        __syncthreads();
+        for (u32 i = w; i < u1 - u0; i += WG / WAVE) {
+            const u32 c = R.pref[i + 1] - R.pref[i], from = R.base[i];
+            u32 gu = sk[i], qu = si[i];
+            for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
+                u32 x[8], id[8];
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u) {
+                    const u32 at = from + min(j0 + u * WAVE + lane, c - 1);
+                    x[u] = skeys[at];
+                    id[u] = sidx[at];
+                }
+#pragma unroll
+                for (u32 u = 0; u < 8; ++u) {
+                    const bool ok = j0 + u * WAVE + lane < c, isg = ok && x[u] > K0, isq = ok && x[u] == K0;
+                    const unsigned long long mg = __ballot(isg), mq = __ballot(isq);
+                    const u32 gb = gu + __builtin_amdgcn_mbcnt_hi((u32)(mg >> 32), __builtin_amdgcn_mbcnt_lo((u32)mg, 0));
+                    const u32 qb = qu + __builtin_amdgcn_mbcnt_hi((u32)(mq >> 32), __builtin_amdgcn_mbcnt_lo((u32)mq, 0));
+                    if (isg || (isq && qb < ties)) {
+                        const u32 p = gb + min(qb, ties);
+                        if (p < k) {
+                            if (out_keys) out_keys[p] = K::from_ord(x[u]);
+                            if (out_idx) out_idx[p] = (i64)id[u];
+                        }
+                    }
+                    gu += (u32)__popcll(mg);
+                    qu += (u32)__popcll(mq);
+                }
+            }
+        }
+        return;
+    }
     q = min(q, ties);
     // a batch of 8 keys per thread in index order: those above K0 and the ties still to take
     auto emit = [&](const u32 (&x)[8], const u32 (&id)[8], u32 nv) {
@@ -929,9 +1030,12 @@ hipError_t launch_filter(const FilterArgs& a, hipStream_t st) {
     u32* cls = (u32*)(fs + 1);
     const u32 n = (u32)a.n, k = (u32)a.k;
     const u32 nunits = filter_units(a.n);
-    // units per range: about half a batch of kept keys, in 512 .. F_RANGES ranges
+    // Units per range: about half a batch of kept keys, in 512 .. F_RANGES ranges (2^24 random keys, k = 2^16:
+    // 61.6 us with 512, 64.1 with 1024; ascending ones 98 and 78), from 2^26 keys 1024 .. F_RANGES (95.6 and
+    // 96.3; ascending 281 and 222).
     const u64 half = (u64)F_BATCH / 2 * nunits / std::max<u64>(a.kept, 1);
-    const u64 most = std::min<u64>((nunits + 511) / 512, F_RUNITS);
+    const u64 fewest = nunits < (1u << 15) ? 512 : 1024;
+    const u64 most = std::min<u64>((nunits + fewest - 1) / fewest, F_RUNITS);
     const u32 upr = (u32)std::max<u64>((nunits + F_RANGES - 1) / F_RANGES, std::min(most, half));
     const u32 nranges = (nunits + upr - 1) / upr;
     if (upr > F_RUNITS || (a.lm != 13 && a.lm != 15 && a.lm != 17 && a.lm != 19)) return hipErrorInvalidValue;

@@ -108,6 +108,21 @@ def test_large_k_partial_outputs_and_graph(orc, dt):  # noqa: F811
         assert np.array_equal(out[2].cpu().numpy(), idx)
 
 
+@pytest.mark.parametrize("n,k", [((1 << 26) + 3, 70_000), (1 << 26, (1 << 21) + 1)])
+@pytest.mark.parametrize("dist", ["ascending", "block", "runs"])
+def test_dense_units(orc, dt, dist, n, k):  # noqa: F811
+    """Kept keys that fill their units: sorted keys, one block of large ones, long runs of equal ones."""
+    if dist == "block":
+        v = make(orc, "uniform", n, 47)[0] >> np.uint32(4)
+        v[n // 5:n // 5 + k + 1000] |= np.uint32(1 << 31)
+    elif dist == "runs":
+        v = (np.arange(n, dtype=np.uint64) // 5000 * 2654435761 % (1 << 32)).astype(np.uint32)
+    else:
+        v = make(orc, "ascending", n, 47)[0]
+    print(f"[case] filter dense {dist} n={n} k={k}", flush=True)
+    check(orc, dt, v, False, k, dt.ALGO_RADIX)
+
+
 def test_longest_ranges(orc, dt):  # noqa: F811
     """2^29 keys with few kept: ranges of as many units as one holds; the same call with stats takes the
     general pipeline."""
