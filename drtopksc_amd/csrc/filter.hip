@@ -17,8 +17,8 @@
 //  k_fkth     the k-th key, and where each range's outputs start.
 //  k_fwrite   the outputs in index order; ties at t are read from the keys again.
 //
-// At 2^30 keys, k = 2^22, the six take 7 + 34 + 765 + 38 + 35 + 48 us (1028 us for the general
-// pipeline, 862 for the call); the read alone takes 630.  At 2^24 keys, k = 2^16: 3 + 9 + 21 + 8 + 14 + 5 us
+// At 2^30 keys, k = 2^22, the six take 6 + 30 + 738 + 25 + 17 + 29 us (1028 us for the general
+// pipeline, 856 for the call); the read alone takes 630.  At 2^24 keys, k = 2^16: 3 + 9 + 21 + 8 + 14 + 5 us
 // (67 and 63 for the calls): there the launches, and the chains of round trips in the two
 // one-workgroup kernels, are most of it.
 //

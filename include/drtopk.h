@@ -218,7 +218,8 @@ typedef struct drtopk_row {
  * whose keys are distributed differently (float32: sign and exponent in the top digits).
  * DRTOPK_TUNE_DEFAULT in a cell keeps the library's built-in choice.  alpha 0 = no delegates (the
  * row is selected directly); the planner lowers an alpha that leaves fewer than k subranges or
- * exceeds the tile.  digit_bits 4 or 8; tile_log2 10..15 is log2 of the keys one workgroup of
+ * exceeds the tile.  digit_bits 4 or 8 (checked and kept in the plan; results and kernels do not
+ * depend on it); tile_log2 10..15 is log2 of the keys one workgroup of
  * the delegate pass streams per work unit. */
 typedef struct drtopk_tuning {
     uint8_t alpha[2][32][32];
