@@ -68,6 +68,7 @@ __global__ __launch_bounds__(SH_NT) void k_small(const u32* __restrict__ keys, u
     if (t == 0 && d_kth) *d_kth = K::from_ord(K0);
     if (!out_keys && !out_idx) return;
     wg_emit<SH_NT>(el, ni, K0, gt, k - gt, L, [&](u32 p, u32 e, u32 x) {
+        if (p >= k) return;
         if (out_keys) out_keys[p] = K::from_ord(x);
         if (out_idx) out_idx[p] = (i64)e;
     });
@@ -428,10 +429,11 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
         if (span == 0) {
             K0 = base;
             gt = above;
-        } else if (held && in_bin <= WgSel<SH_NT>::CAND) {
+        } else if (held && in_bin <= WgSel<SH_NT>::CAND && base) {
+            // (a bucket that starts at 0 would take in the zeros past the concatenation, which its count
+            // doesn't cover: below, they count as keys of their own)
 #pragma unroll 1
-            for (int i = 0; i < ni; ++i)
-                wg_collect(*(const u32x4*)(el + own + 4 * i), base, span, &L.misc[8], L.cand);
+            for (int i = 0; i < ni; ++i) wg_collect<SH_NT>(*(const u32x4*)(el + own + 4 * i), base, span, L);
             __syncthreads();
             u32 g;
             K0 = wg_rank<SH_NT>(in_bin, kk, L, &g);
@@ -473,6 +475,7 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
     if (held) {
         __syncthreads();
         wg_emit<SH_NT>(el, ni, K0, gt, ties, L, [&](u32 p, u32 e, u32 x) {
+            if (p >= k) return;
             if (out_keys) out_keys[p] = K::from_ord(x);
             if (out_idx) out_idx[p] = (i64)ix[own + (e - 4 * (u32)(t * ni))];
         });
@@ -549,8 +552,8 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
                 if (j >= m || x[j] < K0) continue;
                 if (x[j] > K0 || qb < ties) {
                     const u32 p = gb + min(qb, ties);
-                    if (out_keys) out_keys[p] = K::from_ord(x[j]);
-                    if (out_idx) out_idx[p] = (i64)si[i + j];
+                    if (out_keys && p < k) out_keys[p] = K::from_ord(x[j]);
+                    if (out_idx && p < k) out_idx[p] = (i64)si[i + j];
                 }
                 gb += x[j] > K0 ? 1u : 0u;
                 qb += x[j] == K0 ? 1u : 0u;

@@ -151,13 +151,17 @@ __device__ __forceinline__ u32 wg_rank(u32 cnt, u32 kk, WgSel<NT>& L, u32* above
     return L.misc[9];
 }
 
-// Appends the keys of x in [base, base + span] to list (room for all of them is the caller's matter):
-// one test for the four, as few granules hold any.
-__device__ __forceinline__ void wg_collect(const u32x4& x, u32 base, u32 span, u32* count, u32* list) {
+// Appends the keys of x in [base, base + span] to the candidates (no more than fit; the caller has
+// counted them): one test for the four, as few granules hold any.
+template <int NT>
+__device__ __forceinline__ void wg_collect(const u32x4& x, u32 base, u32 span, WgSel<NT>& L) {
     if (min(min(x[0] - base, x[1] - base), min(x[2] - base, x[3] - base)) <= span) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (x[j] - base <= span) list[atomicAdd(count, 1u)] = x[j];
+            if (x[j] - base <= span) {
+                const u32 p = atomicAdd(&L.misc[8], 1u);
+                if (p < WgSel<NT>::CAND) L.cand[p] = x[j];
+            }
     }
 }
 
@@ -210,7 +214,7 @@ __device__ __forceinline__ u32 wg_kth_between(It&& it, u32 lo, u32 hi, u32 k, Wg
         base += M[0] << sh;
         span = min((1u << sh) - 1u, hi - base);  // a top bin past 2^32 must not wrap round to low keys
         if (span && cnt <= WgSel<NT>::CAND) {
-            it([&](const u32x4& x) { wg_collect(x, base, span, &L.misc[8], L.cand); });
+            it([&](const u32x4& x) { wg_collect<NT>(x, base, span, L); });
             __syncthreads();
             u32 g;
             base = wg_rank<NT>(cnt, kk, L, &g);

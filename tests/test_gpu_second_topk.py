@@ -1,0 +1,34 @@
+"""GPU test of the short pipeline's second top-k on inputs that single out one branch of it each: sparse
+keys, whose k-th key lies in the bucket that starts at the lowest key of all.  Outputs must equal the
+oracle's and the general pipeline's (the same call with stats) bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_short import check, dt  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def as_keys(orc, ordered, f32):
+    """The key bits of ordered values."""
+    if not f32:
+        return ordered
+    return np.where(ordered >> 31 != 0, ordered ^ np.uint32(1 << 31), ~ordered).astype(np.uint32)
+
+
+@pytest.mark.parametrize("alpha", [-1, -2])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,k", [(65_537, 9), (70_000, 12), (100_003, 17), (131_073, 5), (140_000, 5), (200_001, 8),
+                                 (262_147, 33), (300_001, 2), (600_000, 20), (1 << 20, 64), ((1 << 20) + 3, 8)])
+def test_sparse_keys(orc, dt, alpha, f32, n, k):  # noqa: F811
+    """The lowest key everywhere but in 1 .. k-1 subranges of 32, one key far above the rest: the threshold
+    is the lowest key, and so is the start of the k-th key's bucket."""
+    rng = np.random.default_rng(n + k)
+    for live in sorted({1, k // 2, k - 1} - {0}):
+        v = np.zeros(n, np.uint32)
+        for i, s in enumerate(rng.choice(n // 32, live, replace=False)):
+            v[32 * s:32 * s + 32] = np.arange(32) if i else np.concatenate(([1 << 31], np.arange(1, 32)))
+        print(f"[case] sparse n={n} k={k} alpha={alpha} f32={f32} live={live}", flush=True)
+        check(orc, dt, as_keys(orc, v, f32), f32, k, dt.ALGO_RADIX, alpha=alpha)
