@@ -303,6 +303,8 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
         if (t == 0) ctrl_fail(ctrl, ERR_CONCAT_SHORT);
         return;
     }
+    const u32 kth_bin = L.misc[0], above = L.misc[1], in_bin = L.misc[2];
+    __syncthreads();  // the selection below reuses misc, and no barrier need come before it
     // concatenation element e: its segment is the last one starting at or before e (an empty
     // segment shares its start with the next one, which is the one found)
     auto seg_of = [&](u32 e) {
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
         gt = C - Q;
     } else {
         // the k-th key's bucket, then its rank among the bucket's keys
-        const u32 base = T + (L.misc[0] << sh), above = L.misc[1], in_bin = L.misc[2], kk = k - above;
+        const u32 base = T + (kth_bin << sh), kk = k - above;
         const u32 span = min((1u << sh) - 1u, hi - base);
         if (!held && above + in_bin <= FIN_CAP) {
             // clustered keys: the concatenation exceeds LDS, but the keys from the bucket up fit.  The

@@ -1,5 +1,6 @@
 """GPU test of the short pipeline's second top-k on inputs that single out one branch of it each: sparse
-keys, whose k-th key lies in the bucket that starts at the lowest key of all.  Outputs must equal the
+keys, whose k-th key lies in the bucket that starts at the lowest key of all, and ties that fill the k-th
+key's bucket of a concatenation held in LDS.  Outputs must equal the
 oracle's and the general pipeline's (the same call with stats) bit for bit."""
 import numpy as np
 import pytest
@@ -32,3 +33,19 @@ def test_sparse_keys(orc, dt, alpha, f32, n, k):  # noqa: F811
             v[32 * s:32 * s + 32] = np.arange(32) if i else np.concatenate(([1 << 31], np.arange(1, 32)))
         print(f"[case] sparse n={n} k={k} alpha={alpha} f32={f32} live={live}", flush=True)
         check(orc, dt, as_keys(orc, v, f32), f32, k, dt.ALGO_RADIX, alpha=alpha)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,k", [(100_003, 900), (1 << 20, 4000), ((1 << 22) + 1, 4096), ((1 << 22) + 5, 8192)])
+def test_tied_bucket(orc, dt, f32, n, k):  # noqa: F811
+    """Half of the top keys lie above one value that many neighbouring keys share: the k-th key is that value,
+    far more than 256 keys are in its bucket, and the threshold lies below it."""
+    for seed in range(3):
+        rng = np.random.default_rng(n + seed)
+        v = rng.integers(1 << 28, 1 << 30, n, dtype=np.uint32)
+        top = rng.choice(n, k // 2, replace=False)
+        v[top] = rng.integers(1 << 31, (1 << 32) - 1, top.size, dtype=np.uint32)
+        tie = int(rng.integers(0, n - k))
+        v[tie:tie + 3 * k // 4] = np.uint32((1 << 30) + 12345)
+        print(f"[case] tied bucket n={n} k={k} f32={f32} seed={seed}", flush=True)
+        check(orc, dt, as_keys(orc, v, f32), f32, k, dt.ALGO_RADIX)
