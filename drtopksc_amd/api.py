@@ -59,6 +59,12 @@ class Stats(ctypes.Structure):
         return d
 
 
+class Route(ctypes.Structure):
+    _fields_ = [("pipeline", ctypes.c_int32), ("alpha", ctypes.c_int32), ("sample_log2", ctypes.c_int32),
+                ("last_resort", ctypes.c_int32), ("delegates", ctypes.c_uint64), ("slots", ctypes.c_uint64),
+                ("kept", ctypes.c_uint64), ("reserved", ctypes.c_uint64)]
+
+
 class Row(ctypes.Structure):
     _fields_ = [("offset", ctypes.c_uint64), ("n", ctypes.c_uint64), ("k", ctypes.c_uint64),
                 ("out_offset", ctypes.c_uint64), ("dtype", ctypes.c_int32), ("reserved", ctypes.c_int32)]
@@ -114,6 +120,9 @@ def lib():
         L.drtopk_tuning_default.restype = None
         L.drtopk_workspace_check.argtypes = [vp, vp, ctypes.POINTER(ctypes.c_uint32)]
         L.drtopk_workspace_check.restype = ctypes.c_int
+        L.drtopk_select_route.argtypes = [ctypes.c_int, ctypes.c_int, u64, u64, ctypes.POINTER(Params), vp, vp,
+                                          ctypes.POINTER(Route)]
+        L.drtopk_select_route.restype = ctypes.c_int
         L.drtopk_testing_set_segment_cap.argtypes = [u64]
         L.drtopk_testing_set_segment_cap.restype = ctypes.c_int
         L.drtopk_file_count.argtypes = [ctypes.c_char_p, ctypes.POINTER(ctypes.c_uint64)]
@@ -238,6 +247,23 @@ def workspace_check(workspace, stream=None) -> int:
     ptr = workspace if isinstance(workspace, int) else workspace.data_ptr()
     _check(lib().drtopk_workspace_check(ctypes.c_void_p(ptr), _stream_ptr(stream), ctypes.byref(bits)))
     return int(bits.value)
+
+
+PIPELINES = ("general", "small", "short", "filter")  # DRTOPK_PIPELINE_*
+
+
+def select_route(n: int, k: int, algo: int = ALGO_RADIX, dtype: int = U32, p: Params | None = None, workspace=None,
+                 stream=None) -> dict:
+    """How select() serves a call without stats (drtopk_route, the pipeline by name).  With the workspace of
+    such a call: also whether it ended in the filter pipeline's last resort (synchronises the stream)."""
+    r = Route()
+    p = p or params()
+    ws = ctypes.c_void_p(workspace.data_ptr()) if workspace is not None else None
+    _check(lib().drtopk_select_route(algo, dtype, n, k, ctypes.byref(p), ws,
+                                     _stream_ptr(stream) if workspace is not None else None, ctypes.byref(r)))
+    d = {name: getattr(r, name) for name, _ in Route._fields_ if name != "reserved"}
+    d["pipeline"] = PIPELINES[r.pipeline]
+    return d
 
 
 def testing_set_segment_cap(cap: int) -> None:

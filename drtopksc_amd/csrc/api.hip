@@ -223,7 +223,7 @@ drtopk_status resolve(drtopk_algo algo, drtopk_dtype dtype, u64 n, u64 k, const 
 //    level measured, twice that when their lists do not fit LDS.  A level
 //    needs 2k ranges for the same reason as the delegates.
 bool short_plan(const Plan& pl, ShortPlan* sp) {
-    if (!pl.own_config || pl.algo == DRTOPK_ALGO_BITONIC || pl.n <= SMALL_N || pl.k > SHORT_KMAX) return false;
+    if (pl.k > SHORT_KMAX) return false;
     const u64 k = pl.k;
     int a0 = std::min(16, floor_log2(pl.n / std::max<u64>(4 * k, 4096)));
     if (cdiv(pl.n, 1ull << a0) > SMALL_N && cdiv(pl.n, 2ull << a0) >= 2 * k) ++a0;  // one level is quicker
@@ -286,9 +286,7 @@ bool short_plan(const Plan& pl, ShortPlan* sp) {
 // units that find it full (clustered keys); both have to fit the workspace.
 bool filter_plan(const Plan& pl, FilterArgs* fa, char* ws) {
     const u64 n = pl.n, k = pl.k;
-    if (!pl.own_config || pl.algo == DRTOPK_ALGO_BITONIC || n <= SMALL_N ||
-        k > n / (n < (1ull << 24) ? 8 : 4) || filter_units(n) > F_RANGES * F_RUNITS)
-        return false;
+    if (k > n / (n < (1ull << 24) ? 8 : 4) || filter_units(n) > F_RANGES * F_RUNITS) return false;
     for (int lm = n >= (1ull << 27) ? 17 : 15; lm <= 19 && (n >> lm) >= 1; lm += 2) {
         double r = (double)k * (double)(1ull << lm) / (double)n;
         if (r < 30) continue;
@@ -344,6 +342,15 @@ bool filter_plan(const Plan& pl, FilterArgs* fa, char* ws) {
         return true;
     }
     return false;
+}
+
+// The pipeline of a call without stats, and its plan; `ws` is its workspace.
+int pick_pipeline(const Plan& pl, char* ws, ShortPlan* sp, FilterArgs* fa) {
+    if (!pl.own_config || pl.algo == DRTOPK_ALGO_BITONIC || g_test_segcap.load(std::memory_order_relaxed) != 0)
+        return DRTOPK_PIPELINE_GENERAL;
+    if (pl.n <= SMALL_N) return DRTOPK_PIPELINE_SMALL;
+    if (short_plan(pl, sp)) return DRTOPK_PIPELINE_SHORT;
+    return filter_plan(pl, fa, ws) ? DRTOPK_PIPELINE_FILTER : DRTOPK_PIPELINE_GENERAL;
 }
 
 SelState make_sel(int mode, u64 m, u64 k, int nb, int B, int stop_digit, int stop_on_one, int max_passes) {
@@ -409,18 +416,26 @@ drtopk_status select_impl(const Plan& pl, const void* d_keys, void* d_workspace,
     hipStream_t st = (hipStream_t)stream;
     char* ws = (char*)d_workspace;
     Ctrl* ctrl = (Ctrl*)(ws + pl.o_ctrl);
-    if (!h_stats && pl.own_config && pl.algo != DRTOPK_ALGO_BITONIC &&
-        g_test_segcap.load(std::memory_order_relaxed) == 0) {
-        ShortArgs sa{};
-        sa.keys = (const u32*)d_keys;
-        sa.n = pl.n; sa.k = pl.k; sa.f32 = pl.f32; sa.ctrl = ctrl;
-        sa.out_keys = d_topk_keys; sa.out_idx = (i64*)d_topk_idx; sa.d_kth = d_kth;
-        if (pl.n <= SMALL_N) {
-            HIPCHK(launch_small(sa, st));
+    if (!h_stats) {
+        ShortPlan sp;
+        FilterArgs fa{};
+        const int pipeline = pick_pipeline(pl, ws, &sp, &fa);
+        if (pipeline == DRTOPK_PIPELINE_FILTER) {
+            fa.keys = (const u32*)d_keys;
+            fa.n = pl.n; fa.k = pl.k; fa.f32 = pl.f32; fa.ctrl = ctrl;
+            fa.out_keys = d_topk_keys; fa.out_idx = (i64*)d_topk_idx; fa.d_kth = d_kth;
+            HIPCHK(launch_filter(fa, st));
             return DRTOPK_OK;
         }
-        ShortPlan sp;
-        if (short_plan(pl, &sp)) {
+        if (pipeline != DRTOPK_PIPELINE_GENERAL) {
+            ShortArgs sa{};
+            sa.keys = (const u32*)d_keys;
+            sa.n = pl.n; sa.k = pl.k; sa.f32 = pl.f32; sa.ctrl = ctrl;
+            sa.out_keys = d_topk_keys; sa.out_idx = (i64*)d_topk_idx; sa.d_kth = d_kth;
+            if (pipeline == DRTOPK_PIPELINE_SMALL) {
+                HIPCHK(launch_small(sa, st));
+                return DRTOPK_OK;
+            }
             sa.alpha = sp.alpha; sa.f1 = sp.f1; sa.f2 = sp.f2;
             sa.dvals = (u32*)(ws + sp.o_dvals);
             sa.sup1 = (u32*)(ws + sp.o_sup1);
@@ -432,13 +447,6 @@ drtopk_status select_impl(const Plan& pl, const void* d_keys, void* d_workspace,
             sa.skeys = (u32*)(ws + sp.o_skeys);
             sa.sidx = (u32*)(ws + sp.o_sidx);
             HIPCHK(launch_short(sa, st));
-            return DRTOPK_OK;
-        }
-        FilterArgs fa{};
-        if (filter_plan(pl, &fa, ws)) {
-            fa.keys = sa.keys; fa.n = pl.n; fa.k = pl.k; fa.f32 = pl.f32; fa.ctrl = ctrl;
-            fa.out_keys = d_topk_keys; fa.out_idx = (i64*)d_topk_idx; fa.d_kth = d_kth;
-            HIPCHK(launch_filter(fa, st));
             return DRTOPK_OK;
         }
     }
@@ -772,6 +780,33 @@ drtopk_status drtopk_workspace_check(const void* d_workspace, void* stream, uint
         return fail(DRTOPK_ERR_INTERNAL, "device-side check failed in a call on this workspace (bits 0x%x:%s%s)",
                     bits, (bits & ERR_CONCAT_SHORT) ? " concatenation shorter than k" : "",
                     (bits & ERR_CAPACITY) ? " a buffer bound was exceeded" : "");
+    return DRTOPK_OK;
+}
+
+drtopk_status drtopk_select_route(drtopk_algo algo, drtopk_dtype dtype, uint64_t n, uint64_t k,
+                                  const drtopk_params* p, const void* d_workspace, void* stream, drtopk_route* r) {
+    clear_error();
+    if (!r) return fail(DRTOPK_ERR_INVALID_ARG, "r is NULL");
+    if (((uintptr_t)d_workspace & 255) != 0) return fail(DRTOPK_ERR_INVALID_ARG, "d_workspace must be 256-byte aligned");
+    Plan pl;
+    drtopk_status s = resolve(algo, dtype, n, k, p, &pl);
+    if (s != DRTOPK_OK) return s;
+    std::memset(r, 0, sizeof(*r));
+    ShortPlan sp;
+    FilterArgs fa{};
+    r->pipeline = pick_pipeline(pl, (char*)d_workspace, &sp, &fa);
+    if (r->pipeline == DRTOPK_PIPELINE_GENERAL) {
+        r->alpha = pl.alpha;
+        r->delegates = pl.D;
+    } else if (r->pipeline == DRTOPK_PIPELINE_SHORT) {
+        r->alpha = sp.alpha;
+        r->delegates = cdiv(n, 1ull << sp.alpha);
+        r->slots = k << sp.alpha;
+    } else if (r->pipeline == DRTOPK_PIPELINE_FILTER) {
+        r->sample_log2 = fa.lm;
+        r->kept = fa.kept;
+        if (d_workspace) HIPCHK(filter_last_resort(fa.state, (hipStream_t)stream, &r->last_resort));
+    }
     return DRTOPK_OK;
 }
 

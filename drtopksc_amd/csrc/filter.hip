@@ -1025,6 +1025,14 @@ __global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nunits
     }
 }
 
+hipError_t filter_last_resort(const void* state, hipStream_t st, int* taken) {
+    u32 kind = 0;
+    hipError_t e = hipMemcpyAsync(&kind, &((const FilterState*)state)->kind, sizeof(kind), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    *taken = kind == F_DONE;
+    return e;
+}
+
 hipError_t launch_filter(const FilterArgs& a, hipStream_t st) {
     FilterState* fs = (FilterState*)a.state;
     u32* cls = (u32*)(fs + 1);

@@ -205,7 +205,7 @@ struct FilterArgs {
     const u32* keys;   // 16-byte aligned, n >= 2^15
     u64 n, k;
     int f32;
-    int lm;            // log2 of the samples: 15, 17 or 19; n >= 2^lm
+    int lm;            // log2 of the samples: 13, 15, 17 or 19; n >= 2^lm
     u32 rp;            // sample rank bounding the k-th key from below
     u32 rlo, rhi;      // sample ranks between which the k-th key almost surely lies (rlo 0: the largest)
     u64 kept;          // keys expected above the bound
@@ -225,6 +225,8 @@ struct FilterArgs {
     void* d_kth;
 };
 hipError_t launch_filter(const FilterArgs& a, hipStream_t st);
+// Whether the last call on this state ended in the one-workgroup selection from all keys.  Synchronises.
+hipError_t filter_last_resort(const void* state, hipStream_t st, int* taken);
 
 // bitonic.hip ---------------------------------------------------------------------------
 // Bitonic family: first top-k over the delegates, whole-subrange concatenation, second

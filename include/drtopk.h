@@ -185,6 +185,28 @@ drtopk_status drtopk_sample_delegates(drtopk_dtype dtype, const void* d_keys, ui
 #define DRTOPK_DEVICE_ERR_CAPACITY     0x4u /* a buffer bound was exceeded */
 drtopk_status drtopk_workspace_check(const void* d_workspace, void* stream, uint32_t* h_error);
 
+/* How drtopk_select serves a call without stats: which pipeline, and the sizes that decide the bytes it
+ * moves.  (A call with stats always takes the general one.)  No reference counterpart. */
+#define DRTOPK_PIPELINE_GENERAL 0 /* delegates, digit / bucket passes, concatenation, second top-k */
+#define DRTOPK_PIPELINE_SMALL   1 /* the whole top-k in one workgroup */
+#define DRTOPK_PIPELINE_SHORT   2 /* delegates, one-workgroup selections */
+#define DRTOPK_PIPELINE_FILTER  3 /* sampled bound, one pass over the keys */
+typedef struct drtopk_route {
+    int32_t pipeline;      /* DRTOPK_PIPELINE_* */
+    int32_t alpha;         /* general, short: log2 of the subrange size */
+    int32_t sample_log2;   /* filter: log2 of the samples */
+    int32_t last_resort;   /* filter, with a workspace given: the last call on it found its bound or a buffer
+                            * insufficient and selected from all keys with one workgroup (exact, but slow) */
+    uint64_t delegates;    /* general, short: delegates written */
+    uint64_t slots;        /* short: most keys the selected subranges hold, k << alpha */
+    uint64_t kept;         /* filter: keys expected above the bound */
+    uint64_t reserved;
+} drtopk_route;
+/* Fills *r.  d_workspace: NULL, or the workspace of a completed or enqueued call with these arguments; the
+ * stream is then synchronised and last_resort read. */
+drtopk_status drtopk_select_route(drtopk_algo algo, drtopk_dtype dtype, uint64_t n, uint64_t k,
+                                  const drtopk_params* p, const void* d_workspace, void* stream, drtopk_route* r);
+
 /* Testing only: every later drtopk_select call in the process (any thread) lets a segment of its
  * concatenation hold at most cap entries (0 restores the full capacity).  A segment that would
  * exceed the bound raises DRTOPK_DEVICE_ERR_CAPACITY instead of being written, which exercises

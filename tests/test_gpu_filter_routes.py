@@ -1,0 +1,59 @@
+"""GPU test of the filter pipeline on calls that it is known to serve (drtopk_select_route): its edges in k and a
+defeated sample of each size.  Outputs must equal
+the oracle's and the general pipeline's bit for bit, and only a defeated sample may end in the
+one-workgroup selection from all keys."""
+import numpy as np
+import pytest
+
+from test_gpu_filter import sample_positions
+from test_gpu_short import check, dt, make  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def filtered(dt, v, f32, k):  # noqa: F811
+    """One call on the filter pipeline; whether it took the last resort."""
+    dev = torch.from_numpy(v.view(np.float32 if f32 else np.int32)).cuda()
+    ws = torch.empty(dt.workspace_size(v.size, k, dt.ALGO_RADIX, 1 if f32 else 0), dtype=torch.uint8, device="cuda")
+    dt.select(dev, k, workspace=ws)
+    r = dt.select_route(v.size, k, dtype=1 if f32 else 0, workspace=ws)
+    assert r["pipeline"] == "filter"
+    return r
+
+
+@pytest.mark.parametrize("n,k,lm", [(65_537, 8_192, 13), (73_737, 9_217, 13), (1_000_003, 125_000, 13),
+                                    (2_400_003, 8_500, 15), ((1 << 24) + 5, 1 << 22, 13), (40_000_003, 9_300, 17)])
+@pytest.mark.parametrize("dist", ["uniform", "f32"])
+def test_edges_in_k(orc, dt, dist, n, k, lm):  # noqa: F811
+    v, f32 = make(orc, dist, n, 61)
+    print(f"[case] filter edge {dist} n={n} k={k}", flush=True)
+    check(orc, dt, v, f32, k, dt.ALGO_RADIX)
+    r = filtered(dt, v, f32, k)
+    assert r["sample_log2"] == lm and r["last_resort"] == 0
+
+
+@pytest.mark.parametrize("n,k,lm", [(1_000_001, 20_000, 13), (2_400_003, 8_500, 15), (40_000_003, 9_300, 17)])
+def test_defeated_sample(orc, dt, n, k, lm):  # noqa: F811
+    """The sampled keys are the largest: the bound lets too few keys through."""
+    v, _ = make(orc, "uniform", n, 67)
+    v = (v >> np.uint32(1)) + np.uint32(1 << 30)
+    pos = sample_positions(n, lm)
+    v[pos] = np.random.default_rng(5).integers(0, 1 << 29, pos.size, dtype=np.uint32) + np.uint32((1 << 32) - (1 << 29))
+    print(f"[case] filter defeated n={n} k={k}", flush=True)
+    check(orc, dt, v, False, k, dt.ALGO_RADIX)
+    r = filtered(dt, v, False, k)
+    assert r["sample_log2"] == lm and r["last_resort"] == 1
+
+
+@pytest.mark.parametrize("dist", ["lognormal", "ascending", "descending", "f32_special", "block"])
+@pytest.mark.parametrize("n,k", [((1 << 20) + 3, 20_000), ((1 << 24) + 1, 1 << 17)])
+def test_no_last_resort(orc, dt, dist, n, k):  # noqa: F811
+    if dist == "block":
+        v, f32 = np.random.default_rng(3).integers(0, 1 << 20, n, dtype=np.uint32), False
+        v[n // 3:n // 3 + n // 16] += np.uint32(1 << 21)
+    else:
+        v, f32 = make(orc, dist, n, 71)
+    print(f"[case] filter {dist} n={n} k={k}", flush=True)
+    assert filtered(dt, v, f32, k)["last_resort"] == 0
