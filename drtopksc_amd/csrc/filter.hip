@@ -163,10 +163,6 @@ __global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample
         // few: all in descending order, two threads comparing one of them with half of the others.  At
         // 2^15 samples and 220 in the list this takes the place of two selections and a sort.
         if (t < 4 && nl + t < F_SORT) list[nl + t] = 0;
-        if (t == 0) {
-            L.misc[9] = 1;
-            L.misc[10] = 0;
-        }
         __syncthreads();
         const u32 c = (u32)t >> 1, x = c < nl ? list[c] : 0u;
         u32 rank = 0;
@@ -180,15 +176,15 @@ __global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample
         __syncthreads();
         const u32 T = nl >= rp ? srt[rp - 1] : T0, tw = nl >= rhi ? srt[rhi - 1] : T;
         const u32 up = rlo >= 1 && nl >= rlo ? srt[rlo - 1] : hi;
-        // the window's samples are consecutive: [misc 9, misc 10)
-        if ((u32)t < nl) {
-            auto in = [&](u32 y) { return y > T && y >= tw && y <= up; };
-            if (in(srt[t]) && (t == 0 || !in(srt[t - 1]))) L.misc[9] = t + 1;
-            if (in(srt[t]) && ((u32)t + 1 == nl || !in(srt[t + 1]))) L.misc[10] = t + 1;
-        }
-        __syncthreads();
-        const u32 first = L.misc[9] - 1, q = min(L.misc[10] > first ? L.misc[10] - first : 0u, F_SPLIT);
-        if (t < 256) st->split[t] = (u32)t < q ? srt[first + q - 1 - t] : 0xFFFFFFFFu;
+        // each value of the window once: samples that tie at `up` may be as many as there are in the list,
+        // and none would be left below them, where the k-th key lies
+        const u32 y = (u32)t < nl ? srt[t] : 0u;
+        const bool is = (u32)t < nl && y > T && y >= tw && y <= up && (t == 0 || srt[t - 1] != y);
+        u32 q;
+        const u32 p = wg_excl_scan<FS_NT>(is ? 1u : 0u, L.a, &q);
+        q = min(q, F_SPLIT);
+        if (is && p < q) st->split[q - 1 - p] = y;
+        if (t < 256 && (u32)t >= q) st->split[t] = 0xFFFFFFFFu;
         if (t == 0) {
             st->t = T;
             st->up = up;
@@ -205,12 +201,18 @@ __global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample
     __syncthreads();
     if (all && rlo >= 1 && nl >= rlo) up = wg_kth_between<FS_NT>(each, tw, hi, rlo, L, &gt);
     __syncthreads();
-    // splitters: the samples of the window (any 254 of them), in order
-    if (t == 0) L.misc[8] = 0;
+    // splitters: the samples of the window (any 254 of them), in order.  Of those that tie at its ends,
+    // which may be any number, one each.
+    if (t == 0) {
+        u32 c = 0;
+        if (up > T) L.cand[c++] = up;
+        if (tw > T && tw < up) L.cand[c++] = tw;
+        L.misc[8] = c;
+    }
     __syncthreads();
     for (u32 i = t; i < nl; i += FS_NT) {
         const u32 x = list[i];
-        if (x > T && x >= tw && x <= up) {
+        if (x > tw && x < up) {  // tw >= T
             const u32 p = atomicAdd(&L.misc[8], 1u);
             if (p < F_SPLIT) L.cand[p] = x;
         }

@@ -1,5 +1,5 @@
-"""GPU test of the filter pipeline on calls that it is known to serve (drtopk_select_route): its edges in k and a
-defeated sample of each size.  Outputs must equal
+"""GPU test of the filter pipeline on calls that it is known to serve (drtopk_select_route): its edges in k, a
+defeated sample of every size, and ties between the ranks that its splitters cover.  Outputs must equal
 the oracle's and the general pipeline's bit for bit, and only a defeated sample may end in the
 one-workgroup selection from all keys."""
 import numpy as np
@@ -45,6 +45,22 @@ def test_defeated_sample(orc, dt, n, k, lm):  # noqa: F811
     check(orc, dt, v, False, k, dt.ALGO_RADIX)
     r = filtered(dt, v, False, k)
     assert r["sample_log2"] == lm and r["last_resort"] == 1
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,k,tied", [(1 << 25, 1_392_508, 0.0366), (1 << 24, 696_320, 0.0366), (1 << 24, 1 << 21, 0.12),
+                                      ((1 << 24) + 3, 40_000, 0.0017), (1_000_003, 20_000, 0.017)])
+def test_ties_above_the_kth_key(orc, dt, f32, n, k, tied):  # noqa: F811
+    """Saturated keys: so many tie at the top that the tie reaches into the ranks the splitters cover, and the
+    k-th key lies below it."""
+    rng = np.random.default_rng(n)
+    v = rng.integers(0, 1 << 30, n, dtype=np.uint32) + np.uint32(1 << 31 if f32 else 0)
+    v[rng.random(n) < tied] = np.uint32((1 << 30) + (1 << 31 if f32 else 0))
+    if f32:
+        v ^= np.uint32(1 << 31)  # positive floats
+    print(f"[case] filter saturated n={n} k={k} f32={f32}", flush=True)
+    check(orc, dt, v, f32, k, dt.ALGO_RADIX)
+    assert filtered(dt, v, f32, k)["last_resort"] == 0
 
 
 @pytest.mark.parametrize("dist", ["lognormal", "ascending", "descending", "f32_special", "block"])
