@@ -274,7 +274,10 @@ bool short_plan(const Plan& pl, ShortPlan* sp) {
 // r >= 30 keeps it below the largest sample with the same certainty.  m is the smallest of 2^15, 2^17,
 // 2^19 that does; from 2^27 keys on at least 2^17, so that the k-th key's class (about n / m keys)
 // stays small; 2^13 below 2^26 keys where that holds 30, as one workgroup selects from the sample
-// (2^15: 18 us, 2^13: 12 us) and the keys kept in vain cost less.
+// (2^15: 18 us, 2^13: 12 us) and the keys kept in vain cost less.  The splitters lie between ranks
+// r -+ (6 sqrt(r) + 8), which miss the k-th key with a probability of 1e-9 at most: outside them a
+// class can outgrow its lists, and the call ends in a selection from all keys by one workgroup (1.7 s
+// at 2^30; 4 sqrt(r) + 4 missed up to 2e-5, and took the same time otherwise).
 //  Where the lines lie (general pipeline -> this one, us, uniform uint32 / normal float32):
 //  below k = n / 16384 the delegates' bound is the better one (2^30, 2^14: 748 -> about 760);
 //  2^30: k 2^16 793 -> 753 / 790 -> 759, 2^20 949 -> 788, 2^22 1020 -> 862, 2^28 5450 -> 3780;
@@ -298,7 +301,7 @@ bool filter_plan(const Plan& pl, FilterArgs* fa, char* ws) {
             lm = 15;
             r /= 4;
         }
-        const double d = 4 * std::sqrt(r) + 4;
+        const double d = 6 * std::sqrt(r) + 8;
         const u32 rp = (u32)std::ceil(r + 7 * std::sqrt(r) + 12), rhi = (u32)std::ceil(r + d);
         const u32 rlo = r > d ? (u32)(r - d) : 0u;
         const double per = (double)n / (double)(1ull << lm);  // keys per sample

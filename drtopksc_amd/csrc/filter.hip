@@ -8,7 +8,7 @@
 //  k_fsample  m pseudo-random keys, one from each of m equal strata.
 //  k_fsplit   t, the r'-th largest sample, with r' = r + 7 sqrt(r) + 12 above the expected rank
 //             r = k m / n: fewer than k keys reach t with a probability below 1e-12 (the positions
-//             do not depend on the keys).  Up to 254 samples of ranks r -+ (4 sqrt(r) + 4)
+//             do not depend on the keys).  Up to 254 samples of ranks r -+ (6 sqrt(r) + 8)
 //             become splitters.
 //  k_filter   keys > t with their indices, in index order, per unit of 2048 keys; how many
 //             equal t (counted, never stored: any number of ties at t costs nothing); and the
@@ -201,8 +201,9 @@ __global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample
     __syncthreads();
     if (all && rlo >= 1 && nl >= rlo) up = wg_kth_between<FS_NT>(each, tw, hi, rlo, L, &gt);
     __syncthreads();
-    // splitters: the samples of the window (any 254 of them), in order.  Of those that tie at its ends,
-    // which may be any number, one each.
+    // splitters: up to 254 samples of the window, in order.  Of those that tie at its ends, which may be
+    // any number, one each; of the others first one from each of 252 equal parts of the window, so that
+    // the classes come out alike, then any.
     if (t == 0) {
         u32 c = 0;
         if (up > T) L.cand[c++] = up;
@@ -210,14 +211,18 @@ __global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample
         L.misc[8] = c;
     }
     __syncthreads();
-    for (u32 i = t; i < nl; i += FS_NT) {
-        const u32 x = list[i];
-        if (x > tw && x < up) {  // tw >= T
+    const float part = (float)(F_SPLIT - 2) / (float)max(up - tw, 1u);
+    for (int pass = 0; pass < 2; ++pass) {
+        for (u32 i = t; i < nl; i += FS_NT) {
+            const u32 x = list[i];
+            if (x <= tw || x >= up) continue;  // tw >= T
+            u32* first = &L.hist[min((u32)((float)(x - tw) * part), F_SPLIT - 3)];  // 1 + the part's first sample
+            if (pass ? *first == i + 1 : atomicCAS(first, 0u, i + 1) != 0) continue;
             const u32 p = atomicAdd(&L.misc[8], 1u);
             if (p < F_SPLIT) L.cand[p] = x;
         }
+        __syncthreads();
     }
-    __syncthreads();
     const u32 q = min(L.misc[8], F_SPLIT);
     {  // the rank of each, four threads comparing it with a quarter of the others
         const u32 c = (u32)t >> 2, x = L.cand[c];

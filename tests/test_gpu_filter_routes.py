@@ -1,5 +1,6 @@
 """GPU test of the filter pipeline on calls that it is known to serve (drtopk_select_route): its edges in k, a
-defeated sample of every size, and ties between the ranks that its splitters cover.  Outputs must equal
+defeated sample of every size, ties between the ranks that its splitters cover, and a sample that places the k-th key
+five deviations too low.  Outputs must equal
 the oracle's and the general pipeline's bit for bit, and only a defeated sample may end in the
 one-workgroup selection from all keys."""
 import numpy as np
@@ -73,3 +74,24 @@ def test_no_last_resort(orc, dt, dist, n, k):  # noqa: F811
         v, f32 = make(orc, dist, n, 71)
     print(f"[case] filter {dist} n={n} k={k}", flush=True)
     assert filtered(dt, v, f32, k)["last_resort"] == 0
+
+
+@pytest.mark.parametrize("n,k", [(1 << 24, 1 << 20), (1 << 25, 1 << 22)])
+def test_unlucky_sample(orc, dt, n, k):  # noqa: F811
+    """Five standard deviations too few of the sampled keys are among the top k: the splitters still cover the
+    k-th key."""
+    lm = 13
+    assert dt.select_route(n, k)["sample_log2"] == lm
+    rng = np.random.default_rng(n)
+    pos = sample_positions(n, lm)
+    r = k * 2 ** lm / n
+    high = rng.choice(pos, int(r - 5 * r ** 0.5), replace=False)
+    rest = np.ones(n, bool)
+    rest[pos] = False
+    others = rng.choice(np.flatnonzero(rest), k - high.size, replace=False)
+    v = rng.integers(0, 1 << 31, n, dtype=np.uint32)
+    v[high] |= np.uint32(1 << 31)
+    v[others] |= np.uint32(1 << 31)
+    print(f"[case] filter unlucky n={n} k={k}", flush=True)
+    check(orc, dt, v, False, k, dt.ALGO_RADIX)
+    assert filtered(dt, v, False, k)["last_resort"] == 0
