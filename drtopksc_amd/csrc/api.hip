@@ -317,6 +317,7 @@ bool filter_plan(const Plan& pl, FilterArgs* fa, char* ws) {
         fa->state = take(filter_state_bytes());
         fa->cnt = (u32*)take(4 * units);
         fa->base = (u32*)take(4 * units);
+        fa->gq = (u32*)take(4 * units);
         fa->rg = (u32*)take(4 * F_RANGES);
         fa->rq = (u32*)take(4 * F_RANGES);
         fa->lkey = (u32*)take(4 * 64 * lcap);

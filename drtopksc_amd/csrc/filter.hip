@@ -25,6 +25,8 @@
 // Should the bound fail after all, or a buffer not hold what it was sized for, k_fkth selects from
 // the keys themselves with its one workgroup: slow, but exact.
 #include <algorithm>
+#include <cstddef>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -38,11 +40,13 @@ constexpr u32 F_ABOVE = F_CLASSES - 1;
 constexpr u32 F_SPLIT = 254;  // so that no splitter's class is 511
 constexpr int F_REPS = 4;         // replicas of the class counters
 constexpr u32 F_BATCH = WG * 8; // kept keys a workgroup takes at a time in k_fpick and k_fwrite
-// Whether a range's units go to waves that work alone instead of to the workgroup in batches: sorted or
-// clustered keys fill the units of few ranges (2^26 ascending keys, k = 2^16: k_fpick 161 -> 24 us, k_fwrite
-// 238 -> 67).  A unit with few kept keys is not worth a wave (2^28 keys, the top ones 1 in 256 of a
-// sixteenth: 380 us for the call, 219 in batches).
-__device__ __forceinline__ bool range_dense(u32 tot, u32 units) { return tot > max(2 * F_BATCH, 256 * units); }
+// Sorted or clustered keys fill the units of few ranges.  A range whose units of at least DENSE_UNIT kept keys
+// hold more than DENSE_RANGE together is listed by k_filter, and its units are shared out over the waves of
+// the whole grid: with a workgroup per range, one held all there was to do (2^30 ascending keys, k = 2^18:
+// k_fpick 154 us, k_fwrite 431; at 2^26, k = 2^16, 25 and 66).  A unit with few kept keys is not worth a wave
+// (2^28 keys, the top ones 1 in 256 of a sixteenth: 380 us for the call, 219 in batches).
+constexpr u32 DENSE_UNIT = 256, DENSE_RANGE = 2 * F_BATCH;
+constexpr u32 DENSE_ENTRY = 0x80000000u;  // a class entry of a dense range names its unit, others their range
 constexpr u32 F_SORT = 512;       // samples above the bound that are put in order at once
 constexpr u32 F_STAGE = 512;    // kept keys a wave stages in LDS
 constexpr u32 F_LISTS = 64;     // sublists of the class, so that their cursors do not serialise
@@ -55,11 +59,18 @@ struct FilterState {
     u32 fail;          // a buffer was too small
     u32 K, gt, ties;   // the k-th key, keys above it, ties taken
     u32 kind;          // F_CLASS, F_AT_T (K == t), F_DONE (outputs written by k_fkth)
-    u32 pad[7];
+    u32 ndense;        // dense ranges listed
+    u32 pad[6];
     u32 lcount[F_LISTS];
     u32 split[256];    // ascending, 0xFFFFFFFF past q
+    u32 upr;           // units per range, which k_filter seldom needs
+    u32 pad2[15];
+    // the counters behind it: classes (F_REPS replicas), kept keys of the full units per range, dense ranges
+    __host__ __device__ __forceinline__ u32* cls() const { return (u32*)(this + 1); }
+    __host__ __device__ __forceinline__ u32* dtot() const { return cls() + F_REPS * F_CLASSES; }
+    __host__ __device__ __forceinline__ u32* dlist() const { return dtot() + F_RANGES; }
 };
-size_t filter_state_bytes() { return sizeof(FilterState) + 4ull * F_REPS * F_CLASSES; }
+size_t filter_state_bytes() { return sizeof(FilterState) + 4ull * (F_REPS * F_CLASSES + 2 * F_RANGES); }
 
 // ---------------------------------------------------------------- sample
 // Sample i is a key of stratum [i n / m, (i + 1) n / m).
@@ -82,7 +93,7 @@ __device__ __forceinline__ u32 sample_stratum(u32 s, int lm) { return (s * 0x9E3
 template <class K>
 __global__ __launch_bounds__(WG) void k_fsample(const u32* __restrict__ keys, u64 n, int lm, u32* __restrict__ sample,
                                                 u32* __restrict__ sup, Ctrl* ctrl, FilterState* st,
-                                                u32* __restrict__ cls) {
+                                                u32* __restrict__ rg, u32* __restrict__ rq, u32 upr) {
     const u32 g = blockIdx.x * WG + threadIdx.x;  // 2^lm / 4 threads, at least 2048
     u32x4 v;
 #pragma unroll
@@ -95,9 +106,10 @@ __global__ __launch_bounds__(WG) void k_fsample(const u32* __restrict__ keys, u6
         const u32 m = row_max_u32(max4(v), lanes);
         if ((threadIdx.x & (lanes - 1)) == 0) sup[g / lanes] = m;
     }
-    static_assert(F_REPS * F_CLASSES <= 2048 && sizeof(FilterState) / 4 <= 2048, "one counter per thread");
-    if (g < F_REPS * F_CLASSES) cls[g] = 0;
-    if (g < sizeof(FilterState) / 4) ((u32*)st)[g] = 0;
+    static_assert(F_REPS * F_CLASSES <= 2048 && F_RANGES <= 2048 && sizeof(FilterState) / 4 <= 2048, "one counter per thread");
+    if (g < F_REPS * F_CLASSES) st->cls()[g] = 0;
+    if (g < F_RANGES) rg[g] = rq[g] = st->dtot()[g] = 0;
+    if (g < sizeof(FilterState) / 4) ((u32*)st)[g] = g == offsetof(FilterState, upr) / 4 ? upr : 0u;
     if (g == 0) ws_head_begin(&ctrl->head);
 }
 
@@ -244,13 +256,25 @@ __global__ __launch_bounds__(FS_NT) void k_fsplit(const u32* __restrict__ sample
 }
 
 // ---------------------------------------------------------------- filter
-// Class of a kept key x <= up: splitters below it, and whether it equals the next one.
-__device__ __forceinline__ u32 class_of(const u32* sp, u32 x) {
-    u32 lo = 0;
+// Classes of W kept keys x <= up at once (a search is a chain of LDS round trips): splitters below
+// each, and whether it equals the next one.
+template <int W>
+__device__ __forceinline__ void class_of(const u32* sp, const u32* x, u32 (&c)[W]) {
 #pragma unroll
-    for (u32 step = 128; step; step >>= 1)
-        if (sp[lo + step - 1] < x) lo += step;
-    return 2 * lo + (sp[lo] == x ? 1u : 0u);  // sp[255] is 0xFFFFFFFF, lo <= q
+    for (int u = 0; u < W; ++u) c[u] = 0;
+#pragma unroll
+    for (u32 step = 128; step; step >>= 1) {
+        u32 s[W];
+#pragma unroll
+        for (int u = 0; u < W; ++u) s[u] = sp[c[u] + step - 1];
+#pragma unroll
+        for (int u = 0; u < W; ++u) c[u] += s[u] < x[u] ? step : 0u;
+    }
+    u32 s[W];
+#pragma unroll
+    for (int u = 0; u < W; ++u) s[u] = sp[c[u]];  // sp[255] is 0xFFFFFFFF, c <= q
+#pragma unroll
+    for (int u = 0; u < W; ++u) c[u] = 2 * c[u] + (s[u] == x[u] ? 1u : 0u);
 }
 
 // The compare domain of a raw key: unsigned for uint32.  A float32's bits compare as a signed integer
@@ -283,16 +307,18 @@ struct FDomain<KeyF32> {
 // key and staged in the wave's LDS.  They leave, with their classes counted, when that is full:
 // on this part a load is waited for together with the stores issued before it, so a wave that
 // stored after every unit waited for a write's round trip each time (2^30 keys, 172 K kept: 694 us).
+// A wave meets consecutive units, so sorted keys leave all they keep to a few of them, and what a full unit
+// costs a wave shows in the call: it searches four classes at a time, and counts neighbours of one class
+// with one atomic (2^26 ascending keys, k = 2^16: the pass 108 -> 87 us; 50 for random keys).
 // Waves work alone, without a barrier in the loop.
 template <class K>
 __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, u32 n, u32 nunits, int rounds, u32 wcap,
                                                u32 pool_at, u32 pool_cap, FilterState* st, u32* __restrict__ skeys,
-                                               u32* __restrict__ sidx, u32* __restrict__ cnt, u32* __restrict__ base_of,
-                                               u32* __restrict__ cls) {
+                                               u32* __restrict__ sidx, u32* __restrict__ cnt, u32* __restrict__ base_of) {
     using D = FDomain<K>;
     using DT = typename D::T;
     __shared__ u32 sp[256], lh[F_CLASSES], sk[WG / WAVE][F_STAGE], si[WG / WAVE][F_STAGE];
-    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
     sp[threadIdx.x] = st->split[threadIdx.x];
     lh[threadIdx.x] = 0;
     lh[WG + threadIdx.x] = 0;
@@ -301,31 +327,63 @@ __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, 
     const bool conv = D::converts(t);  // uniform
     u32 above = 0;
     __syncthreads();
-    auto count_class = [&](u32 v) {
-        if (v > up) ++above;
-        else atomicAdd(&lh[class_of(sp, v)], 1u);
-    };
     // the wave's share of the segments, filled from its start; what its units kept and where, one unit
     // per lane until 64 of them are written
     const u32 gbase = (blockIdx.x * (WG / WAVE) + w) * wcap;
-    u32 gpos = 0, fill = 0, nrec = 0, my_unit = 0, my_cnt = 0, my_base = 0;
-    auto flush = [&]() {  // the staged keys are the last `fill` of the wave's share
+    u32 gpos = 0, nrec = 0, my_unit = 0, my_cnt = 0, my_base = 0;
+    u32 fill = 0, dst = 0, last = 0;  // staged keys, their first slot; what the last unit kept
+    bool apart = false;               // the staged keys end where others were stored past the stage
+    // classes of N keys per lane, those of `act` kept ones
+    auto count_classes = [&](auto width, const u32* v, const bool* act, bool neighbours) {
+        constexpr int N = decltype(width)::value;
+        u32 c[N];
+        class_of<N>(sp, v, c);
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const bool in = act[u] && v[u] <= up;
+            above += act[u] && v[u] > up ? 1u : 0u;
+            if (neighbours) {  // of sorted keys share a class: the first lane's is counted with one atomic
+                const u32 c0 = (u32)__builtin_amdgcn_readfirstlane((int)c[u]);
+                const u64 same = __ballot(in && c[u] == c0);
+                if (in && c[u] != c0) atomicAdd(&lh[c[u]], 1u);
+                if (same && lane == 0) atomicAdd(&lh[c0], (u32)__popcll(same));
+            } else if (in) {
+                atomicAdd(&lh[c[u]], 1u);
+            }
+        }
+    };
+    auto flush = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own LDS writes
         __builtin_amdgcn_wave_barrier();
-        for (u32 i = lane; i < fill; i += WAVE) {
-            const u32 v = sk[w][i], at = gbase + gpos - fill + i;
-            skeys[at] = v;
-            sidx[at] = si[w][i];
-            count_class(v);
+        for (u32 i0 = 0; i0 < fill; i0 += 2 * WAVE) {
+            u32 v[2];
+            bool act[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const u32 i = i0 + u * WAVE + lane;
+                act[u] = i < fill;
+                v[u] = act[u] ? sk[w][i] : 0u;
+                if (act[u]) {
+                    skeys[dst + i] = v[u];
+                    sidx[dst + i] = si[w][i];
+                }
+            }
+            count_classes(std::integral_constant<int, 2>(), v, act, false);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
         fill = 0;
+        apart = false;
     };
     auto write_units = [&]() {
         if ((u32)lane < nrec) {
             cnt[my_unit] = my_cnt;
             base_of[my_unit] = my_base;
+            const u32 c = my_cnt & 0xFFFFu;
+            if (c >= DENSE_UNIT) {
+                const u32 r = my_unit / st->upr, had = atomicAdd(&st->dtot()[r], c);
+                if (had <= DENSE_RANGE && had + c > DENSE_RANGE) st->dlist()[atomicAdd(&st->ndense, 1u)] = r;
+            }
         }
         nrec = 0;
     };
@@ -354,6 +412,8 @@ __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, 
                         for (int j = 0; j < 4; ++j) x[b][j] = e + j < n ? keys[e + j] : K::from_ord(0);  // the lowest key
                 }
             }
+            // behind the loads: what is waited for with them is the stores of the flush before
+            if (apart || fill + last > F_STAGE) flush();
             if (conv) {
 #pragma unroll
                 for (int b = 0; b < 8; ++b)
@@ -381,9 +441,9 @@ __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, 
                 eq = 0;
             }
             const bool spill = gpos + kept > wcap;  // rare: clustered keys go to the pool
-            if (fill + kept > F_STAGE || spill) flush();
-            bool staged = kept <= F_STAGE && !spill;
+            const bool staged = fill + kept <= F_STAGE && !spill;
             u32 base = gbase + gpos;
+            last = kept;
             if (spill) {
                 u32 at = 0;
                 if (lane == 0) at = atomicAdd(&st->pool, kept);
@@ -403,6 +463,8 @@ __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, 
             }
             ++nrec;
             if (kept == 0) continue;
+            if (!staged) apart = fill > 0;
+            else if (fill == 0) dst = base;
             u32 at = staged ? fill : base;
 #pragma unroll
             for (int b = 0; b < 8; ++b) {
@@ -413,20 +475,31 @@ __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, 
                     const u64 m = __ballot((DT)x[b][j] > t);
                     pos = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, pos));
                 }
+                u32 v[4];
+                bool act[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if ((DT)x[b][j] > t) {
-                        const u32 v = D::ordered(x[b][j], conv), id = k0 + 4 * (b * WAVE + lane) + j;
+                for (int j = 0; j < 4; ++j) {
+                    act[j] = (DT)x[b][j] > t;
+                    v[j] = D::ordered(x[b][j], conv);
+                    if (act[j]) {
+                        const u32 id = k0 + 4 * (b * WAVE + lane) + j;
                         if (staged) {
-                            sk[w][pos] = v;
+                            sk[w][pos] = v[j];
                             si[w][pos] = id;
                         } else {
-                            skeys[pos] = v;
+                            skeys[pos] = v[j];
                             sidx[pos] = id;
-                            count_class(v);
                         }
                         ++pos;
                     }
+                }
+                if (!staged) {
+                    bool any = false;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) any |= act[j] && v[j] <= up;
+                    if (__ballot(any)) count_classes(std::integral_constant<int, 4>(), v, act, true);
+                    else above += (u32)act[0] + (u32)act[1] + (u32)act[2] + (u32)act[3];
+                }
                 at += c[b];
             }
             if (staged) fill += kept;
@@ -436,7 +509,7 @@ __global__ __launch_bounds__(WG, 7) void k_filter(const u32* __restrict__ keys, 
     above = wave_incl_scan_u32(above);
     if (lane == WAVE - 1 && above) atomicAdd(&lh[F_ABOVE], above);
     __syncthreads();
-    u32* g = cls + (blockIdx.x % F_REPS) * F_CLASSES;
+    u32* g = st->cls() + (blockIdx.x % F_REPS) * F_CLASSES;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const u32 c = lh[j * WG + threadIdx.x];
@@ -453,8 +526,7 @@ struct FClass {
 };
 // Every thread of an NT-thread block; `lds` holds 8 words, `scratch` NT/64.  Ends with a barrier.
 template <int NT>
-__device__ __forceinline__ FClass find_class(const FilterState* st, const u32* __restrict__ cls, u32 k, u32* lds,
-                                             u32* scratch) {
+__device__ __forceinline__ FClass find_class(const FilterState* st, u32 k, u32* lds, u32* scratch) {
     constexpr int PER = NT >= 512 ? 1 : (int)F_CLASSES / NT;
     u32 c[PER], s = 0, tot;
 #pragma unroll
@@ -464,7 +536,7 @@ __device__ __forceinline__ FClass find_class(const FilterState* st, const u32* _
         if (b >= 0) {
             u32 r[F_REPS];
 #pragma unroll
-            for (int i = 0; i < F_REPS; ++i) r[i] = cls[i * F_CLASSES + b];
+            for (int i = 0; i < F_REPS; ++i) r[i] = st->cls()[i * F_CLASSES + b];
 #pragma unroll
             for (int i = 0; i < F_REPS; ++i) c[j] += r[i];
         }
@@ -545,13 +617,30 @@ __device__ __forceinline__ void range_slots(const RangeLds& R, u32 e, u32 tot, u
     }
 }
 
-__global__ __launch_bounds__(WG) void k_fpick(FilterState* st, const u32* __restrict__ cls, u32 k, u32 nunits, u32 upr,
+// The units of the dense ranges, over the waves of the grid: f(range, unit, kept keys, first slot), every lane
+// of the wave at once.
+template <class F>
+__device__ __forceinline__ void dense_units(const FilterState* st, u32 ndense, u32 nranges, u32 nunits, u32 upr,
+                                            const u32* __restrict__ cnt, const u32* __restrict__ base_of, F&& f) {
+    for (u32 j = blockIdx.x * (WG / WAVE) + threadIdx.x / WAVE; j < ndense * upr; j += nranges * (WG / WAVE)) {
+        const u32 r = st->dlist()[j / upr], u = r * upr + j % upr;
+        if (u < nunits) f(r, u, cnt[u] & 0xFFFFu, base_of[u]);
+    }
+}
+
+// Writes, per range, the kept keys above the class (and those equal to it where it is one value); for the units
+// of dense ranges the same in gq, above << 16 | equal.  2048 workgroups are one round of the chip at eight waves
+// per SIMD, which more than 80 scalar registers do not allow (2^28 keys, k = 2^24: 49 us with 86, 40 with 80).
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_num_sgpr(80))) void k_fpick(FilterState* st, u32 k, u32 nranges, u32 nunits, u32 upr,
                                               const u32* __restrict__ cnt, const u32* __restrict__ base_of,
-                                              const u32* __restrict__ skeys, u32* __restrict__ rg, u32* __restrict__ rq,
-                                              u32 lcap, u32* __restrict__ lkey, u32* __restrict__ lrange) {
+                                              const u32* __restrict__ skeys, u32* __restrict__ gq, u32* __restrict__ rg,
+                                              u32* __restrict__ rq, u32 lcap, u32* __restrict__ lkey,
+                                              u32* __restrict__ lrange) {
     __shared__ RangeLds R;
-    const FClass f = find_class<WG>(st, cls, k, R.lds, R.scratch);
     const u32 r = blockIdx.x, u0 = r * upr, u1 = min(u0 + upr, nunits);
+    const u32 ndense = st->ndense;
+    const bool dense = ndense && st->dtot()[r] > DENSE_RANGE;  // uniform
+    const FClass f = find_class<WG>(st, k, R.lds, R.scratch);
     u32 eq;
     const u32 tot = range_open(R, cnt, base_of, u0, u1, &eq);
     if (f.kept < k) {  // K == t, or the bound failed
@@ -563,41 +652,6 @@ __global__ __launch_bounds__(WG) void k_fpick(FilterState* st, const u32* __rest
     }
     const bool known = f.hi - f.lo == 1;  // one value: counted, not listed
     u32 g = 0, q = 0;
-    const bool dense = range_dense(tot, u1 - u0);
-    if (dense) {  // uniform; each unit by a wave alone
-        const u32 lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-        for (u32 i = w; i < u1 - u0; i += WG / WAVE) {
-            const u32 c = R.pref[i + 1] - R.pref[i], from = R.base[i];
-            for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
-                u32 x[8], in = 0;
-#pragma unroll
-                for (u32 u = 0; u < 8; ++u) x[u] = skeys[from + min(j0 + u * WAVE + lane, c - 1)];
-#pragma unroll
-                for (u32 u = 0; u < 8; ++u) {
-                    if (j0 + u * WAVE + lane >= c) x[u] = 0;  // neither above nor in the class
-                    g += x[u] > f.hi ? 1u : 0u;
-                    in += x[u] > f.lo && x[u] <= f.hi ? 1u : 0u;
-                }
-                q += in;
-                if (known) continue;
-                const u32 inc = wave_incl_scan_u32(in), n = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
-                if (n == 0) continue;  // uniform over the wave
-                const u32 list = (r + 4 * i + j0 / (8 * WAVE)) % F_LISTS;
-                u32 b = 0;
-                if (lane == 0) b = atomicAdd(&st->lcount[list], n);
-                u32 to = (u32)__builtin_amdgcn_readfirstlane((int)b) + inc - in;
-#pragma unroll
-                for (u32 u = 0; u < 8; ++u)
-                    if (x[u] > f.lo && x[u] <= f.hi) {
-                        if (to < lcap) {
-                            lkey[list * lcap + to] = x[u];
-                            lrange[list * lcap + to] = r;
-                        }
-                        ++to;
-                    }
-            }
-        }
-    }
     for (u32 e0 = dense ? tot : 0; e0 < tot; e0 += F_BATCH) {
         u32 at[8], x[8], in = 0;
         range_slots(R, e0 + 8 * threadIdx.x, tot, at);
@@ -629,22 +683,63 @@ __global__ __launch_bounds__(WG) void k_fpick(FilterState* st, const u32* __rest
             }
         __syncthreads();
     }
-    u32 gs, qs;
-    wg_excl_scan<WG>(g, R.scratch, &gs);
-    wg_excl_scan<WG>(q, R.scratch, &qs);
-    if (threadIdx.x == 0) {
-        rg[r] = gs;
-        rq[r] = known ? qs : 0u;
+    if (!dense) {
+        u32 gs, qs;
+        wg_excl_scan<WG>(g, R.scratch, &gs);
+        wg_excl_scan<WG>(q, R.scratch, &qs);
+        if (threadIdx.x == 0) {
+            rg[r] = gs;
+            rq[r] = known ? qs : 0u;
+        }
     }
+    const u32 lane = threadIdx.x & (WAVE - 1);
+    dense_units(st, ndense, nranges, nunits, upr, cnt, base_of, [&](u32 rr, u32 unit, u32 c, u32 from) {
+        u32 m = 0;  // above << 16 | in the class
+        for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
+            u32 x[8], in = 0;
+#pragma unroll
+            for (u32 u = 0; u < 8; ++u) x[u] = skeys[from + min(j0 + u * WAVE + lane, c - 1)];
+#pragma unroll
+            for (u32 u = 0; u < 8; ++u) {
+                if (j0 + u * WAVE + lane >= c) x[u] = 0;  // neither above nor in the class
+                m += x[u] > f.hi ? 0x10000u : 0u;
+                in += x[u] > f.lo && x[u] <= f.hi ? 1u : 0u;
+            }
+            m += in;
+            if (known) continue;
+            const u32 inc = wave_incl_scan_u32(in), n = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+            if (n == 0) continue;  // uniform over the wave
+            const u32 list = (unit + j0 / (8 * WAVE)) % F_LISTS;
+            u32 b = 0;
+            if (lane == 0) b = atomicAdd(&st->lcount[list], n);
+            u32 to = (u32)__builtin_amdgcn_readfirstlane((int)b) + inc - in;
+#pragma unroll
+            for (u32 u = 0; u < 8; ++u)
+                if (x[u] > f.lo && x[u] <= f.hi) {
+                    if (to < lcap) {
+                        lkey[list * lcap + to] = x[u];
+                        lrange[list * lcap + to] = DENSE_ENTRY | unit;
+                    }
+                    ++to;
+                }
+        }
+        m = wave_incl_scan_u32(m);
+        if (lane == WAVE - 1) {
+            gq[unit] = known ? m : m & 0xFFFF0000u;
+            if (m >> 16) atomicAdd(&rg[rr], m >> 16);
+            if (known && (m & 0xFFFFu)) atomicAdd(&rq[rr], m & 0xFFFFu);
+        }
+    });
 }
 
 // ---------------------------------------------------------------- k-th key and range offsets
 template <class K>
-__global__ __launch_bounds__(FS_NT) void k_fkth(FilterState* st, const u32* __restrict__ cls, u32 k, u32 nranges,
+__global__ __launch_bounds__(FS_NT) void k_fkth(FilterState* st, u32 k, u32 nranges,
                                                 u32* __restrict__ rg, u32* __restrict__ rq, u32 lcap,
-                                                const u32* __restrict__ lkey, const u32* __restrict__ lrange,
-                                                const u32* __restrict__ keys, u32 n, u32* __restrict__ out_keys,
-                                                i64* __restrict__ out_idx, u32* __restrict__ d_kth) {
+                                                const u32* __restrict__ lkey, const u32* __restrict__ lrange, u32 upr,
+                                                u32* __restrict__ gq, const u32* __restrict__ keys, u32 n,
+                                                u32* __restrict__ out_keys, i64* __restrict__ out_idx,
+                                                u32* __restrict__ d_kth) {
     __shared__ WgSel<FS_NT> L;
     __shared__ __align__(16) u32 el[wg_words<FS_NT>(32768)];
     __shared__ u32 lpref[F_LISTS + 1], lds[8];
@@ -660,7 +755,7 @@ __global__ __launch_bounds__(FS_NT) void k_fkth(FilterState* st, const u32* __re
         q[j] = r < nranges ? rq[r] : 0u;
     }
     const u32 in_list = t < (int)F_LISTS ? st->lcount[t] : 0u;
-    const FClass f = find_class<FS_NT>(st, cls, k, lds, L.a);
+    const FClass f = find_class<FS_NT>(st, k, lds, L.a);
     u32 qs = 0, eqs;
 #pragma unroll
     for (int j = 0; j < RPT; ++j) qs += q[j];
@@ -715,12 +810,27 @@ __global__ __launch_bounds__(FS_NT) void k_fkth(FilterState* st, const u32* __re
                 },
                 f.lo + 1, f.hi, f.kk, L, &gt);
             gt += f.above;
-            // the class's keys above K and equal to it, back to their ranges
+            // the class's keys above K and equal to it, back to their ranges (and units of dense ones)
             u32* add = el + 32768;
             for (u32 i = t; i < 2 * F_RANGES; i += FS_NT) add[i] = 0;
             __syncthreads();
             each_entry([&](u32, u32 s, u32 x) {
-                if (x >= Kk) atomicAdd(&add[(x > Kk ? 0u : F_RANGES) + lrange[s]], 1u);
+                if (x < Kk) return;
+                const bool gr = x > Kk;
+                const u32 r = lrange[s];
+                if (!(r & DENSE_ENTRY)) {
+                    atomicAdd(&add[(gr ? 0u : F_RANGES) + r], 1u);
+                    return;
+                }
+                // entries of a dense unit lie side by side: those of the first lane's together
+                const u32 unit = r & ~DENSE_ENTRY, unit0 = (u32)__builtin_amdgcn_readfirstlane((int)unit), to = unit / upr;
+                const u32 ng = (u32)__popcll(__ballot(unit == unit0 && gr)), nq = (u32)__popcll(__ballot(unit == unit0 && !gr));
+                const bool lead = lane == __ffsll((unsigned long long)__ballot(true)) - 1;
+                if (unit == unit0 && !lead) return;
+                const u32 a = lead ? ng : (gr ? 1u : 0u), b = lead ? nq : (gr ? 0u : 1u);
+                atomicAdd(&gq[unit], a << 16 | b);
+                if (a) atomicAdd(&add[to], a);
+                if (b) atomicAdd(&add[F_RANGES + to], b);
             });
             __syncthreads();
 #pragma unroll
@@ -839,14 +949,15 @@ __global__ __launch_bounds__(FS_NT) void k_fkth(FilterState* st, const u32* __re
 
 // ---------------------------------------------------------------- outputs
 template <class K>
-__global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nunits, u32 upr, const u32* __restrict__ cnt,
-                                               const u32* __restrict__ base_of, const u32* __restrict__ skeys,
-                                               const u32* __restrict__ sidx, const u32* __restrict__ rg,
+__global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nranges, u32 nunits, u32 upr,
+                                               const u32* __restrict__ cnt, const u32* __restrict__ base_of,
+                                               const u32* __restrict__ skeys, const u32* __restrict__ sidx,
+                                               const u32* __restrict__ gq, const u32* __restrict__ rg,
                                                const u32* __restrict__ rq, const u32* __restrict__ keys, u32 n, u32 k,
                                                u32* __restrict__ out_keys, i64* __restrict__ out_idx) {
     __shared__ RangeLds R;
     __shared__ u32 sk[F_BATCH], si[F_BATCH];
-    const u32 kind = st->kind, K0 = st->K, ties = st->ties;
+    const u32 kind = st->kind, K0 = st->K, ties = st->ties, ndense = st->ndense;
     if (kind == F_DONE) return;
     u32 r = blockIdx.x, sub = 0, subs = 1;
     if (kind == F_AT_T) {
@@ -854,7 +965,7 @@ __global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nunits
         // bound may all be taken from the first of the ranges.
         __shared__ u16 act[F_RANGES];
         constexpr u32 RPT = F_RANGES / WG;
-        const u32 nr = gridDim.x, r0 = threadIdx.x * RPT;
+        const u32 nr = nranges, r0 = threadIdx.x * RPT;
         u32 on = 0, na;
 #pragma unroll
         for (u32 j = 0; j < RPT; ++j)
@@ -932,62 +1043,46 @@ __global__ __launch_bounds__(WG) void k_fwrite(const FilterState* st, u32 nunits
         }
         return;
     }
-    if (range_dense(tot, u1 - u0)) {  // each unit by a wave alone: counted, then written
-        const u32 lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-        for (u32 i = w; i < u1 - u0; i += WG / WAVE) {
-            const u32 c = R.pref[i + 1] - R.pref[i], from = R.base[i];
-            u32 m = 0;  // above << 16 | ties
-            for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
-                u32 x[8];
+    const bool dense = ndense && st->dtot()[r] > DENSE_RANGE;  // uniform
+    dense_units(st, ndense, nranges, nunits, upr, cnt, base_of, [&](u32 rr, u32 unit, u32 c, u32 from) {
+        const u32 lane = threadIdx.x & (WAVE - 1), first = rr * upr, mine = gq[unit];
+        if (mine == 0) return;
+        u32 gs = 0, qs = 0;  // in the range's units before this one
+        for (u32 i = lane; i < unit - first; i += WAVE) {
+            const u32 m = gq[first + i];
+            gs += m >> 16;
+            qs += m & 0xFFFFu;
+        }
+        u32 gu = rg[rr] + (u32)__builtin_amdgcn_readlane((int)wave_incl_scan_u32(gs), WAVE - 1);
+        u32 qu = rq[rr] + (u32)__builtin_amdgcn_readlane((int)wave_incl_scan_u32(qs), WAVE - 1);
+        if (mine >> 16 == 0 && qu >= ties) return;
+        for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
+            u32 x[8], id[8];
 #pragma unroll
-                for (u32 u = 0; u < 8; ++u) x[u] = skeys[from + min(j0 + u * WAVE + lane, c - 1)];
-#pragma unroll
-                for (u32 u = 0; u < 8; ++u)
-                    m += j0 + u * WAVE + lane < c ? (x[u] > K0 ? 0x10000u : (x[u] == K0 ? 1u : 0u)) : 0u;
+            for (u32 u = 0; u < 8; ++u) {
+                const u32 at = from + min(j0 + u * WAVE + lane, c - 1);
+                x[u] = skeys[at];
+                id[u] = sidx[at];
             }
-            m = wave_incl_scan_u32(m);
-            if (lane == WAVE - 1) sk[i] = m;
-        }
-        __syncthreads();
-        const u32 m = threadIdx.x < u1 - u0 ? sk[threadIdx.x] : 0u;
-        u32 all;
-        const u32 gx = wg_excl_scan<WG>(m >> 16, R.scratch, &all), qx = wg_excl_scan<WG>(m & 0xFFFFu, R.scratch, &all);
-        if (threadIdx.x < F_RUNITS) {
-            sk[threadIdx.x] = g + gx;
-            si[threadIdx.x] = q + qx;
-        }
-        __syncthreads();
-        for (u32 i = w; i < u1 - u0; i += WG / WAVE) {
-            const u32 c = R.pref[i + 1] - R.pref[i], from = R.base[i];
-            u32 gu = sk[i], qu = si[i];
-            for (u32 j0 = 0; j0 < c; j0 += 8 * WAVE) {
-                u32 x[8], id[8];
 #pragma unroll
-                for (u32 u = 0; u < 8; ++u) {
-                    const u32 at = from + min(j0 + u * WAVE + lane, c - 1);
-                    x[u] = skeys[at];
-                    id[u] = sidx[at];
-                }
-#pragma unroll
-                for (u32 u = 0; u < 8; ++u) {
-                    const bool ok = j0 + u * WAVE + lane < c, isg = ok && x[u] > K0, isq = ok && x[u] == K0;
-                    const unsigned long long mg = __ballot(isg), mq = __ballot(isq);
-                    const u32 gb = gu + __builtin_amdgcn_mbcnt_hi((u32)(mg >> 32), __builtin_amdgcn_mbcnt_lo((u32)mg, 0));
-                    const u32 qb = qu + __builtin_amdgcn_mbcnt_hi((u32)(mq >> 32), __builtin_amdgcn_mbcnt_lo((u32)mq, 0));
-                    if (isg || (isq && qb < ties)) {
-                        const u32 p = gb + min(qb, ties);
-                        if (p < k) {
-                            if (out_keys) out_keys[p] = K::from_ord(x[u]);
-                            if (out_idx) out_idx[p] = (i64)id[u];
-                        }
+            for (u32 u = 0; u < 8; ++u) {
+                const bool ok = j0 + u * WAVE + lane < c, isg = ok && x[u] > K0, isq = ok && x[u] == K0;
+                const unsigned long long mg = __ballot(isg), mq = __ballot(isq);
+                const u32 gb = gu + __builtin_amdgcn_mbcnt_hi((u32)(mg >> 32), __builtin_amdgcn_mbcnt_lo((u32)mg, 0));
+                const u32 qb = qu + __builtin_amdgcn_mbcnt_hi((u32)(mq >> 32), __builtin_amdgcn_mbcnt_lo((u32)mq, 0));
+                if (isg || (isq && qb < ties)) {
+                    const u32 p = gb + min(qb, ties);
+                    if (p < k) {
+                        if (out_keys) out_keys[p] = K::from_ord(x[u]);
+                        if (out_idx) out_idx[p] = (i64)id[u];
                     }
-                    gu += (u32)__popcll(mg);
-                    qu += (u32)__popcll(mq);
                 }
+                gu += (u32)__popcll(mg);
+                qu += (u32)__popcll(mq);
             }
         }
-        return;
-    }
+    });
+    if (dense) return;
     q = min(q, ties);
     // a batch of 8 keys per thread in index order: those above K0 and the ties still to take
     auto emit = [&](const u32 (&x)[8], const u32 (&id)[8], u32 nv) {
@@ -1042,7 +1137,6 @@ hipError_t filter_last_resort(const void* state, hipStream_t st, int* taken) {
 
 hipError_t launch_filter(const FilterArgs& a, hipStream_t st) {
     FilterState* fs = (FilterState*)a.state;
-    u32* cls = (u32*)(fs + 1);
     const u32 n = (u32)a.n, k = (u32)a.k;
     const u32 nunits = filter_units(a.n);
     // Units per range: about half a batch of kept keys, in 512 .. F_RANGES ranges (2^24 random keys, k = 2^16:
@@ -1061,20 +1155,20 @@ hipError_t launch_filter(const FilterArgs& a, hipStream_t st) {
 #define F_LAUNCH(K)                                                                                                     \
     do {                                                                                                                \
         hipLaunchKernelGGL((k_fsample<K>), dim3((1u << a.lm) / 4 / WG), dim3(WG), 0, st, a.keys, a.n, a.lm, a.sample,  \
-                           a.sample + (1u << a.lm), a.ctrl, fs, cls);                                                   \
+                           a.sample + (1u << a.lm), a.ctrl, fs, a.rg, a.rq, upr);                                      \
         if (a.lm == 13) F_SPLIT_LAUNCH(13);                                                                            \
         else if (a.lm == 15) F_SPLIT_LAUNCH(15);                                                                       \
         else if (a.lm == 17) F_SPLIT_LAUNCH(17);                                                                       \
         else F_SPLIT_LAUNCH(19);                                                                                       \
         hipLaunchKernelGGL((k_filter<K>), dim3(fg.grid), dim3(WG), 0, st, a.keys, n, nunits, fg.rounds, a.wcap,        \
-                           fg.grid * 4 * a.wcap, a.pool_cap, fs, a.skeys, a.sidx, a.cnt, a.base, cls);                        \
-        hipLaunchKernelGGL(k_fpick, dim3(nranges), dim3(WG), 0, st, fs, cls, k, nunits, upr, a.cnt, a.base, a.skeys,   \
-                           a.rg, a.rq, a.lcap, a.lkey, a.lrange);                                                      \
-        hipLaunchKernelGGL((k_fkth<K>), dim3(1), dim3(FS_NT), 0, st, fs, cls, k, nranges, a.rg, a.rq, a.lcap, a.lkey,  \
-                           a.lrange, a.keys, n, (u32*)a.out_keys, a.out_idx, (u32*)a.d_kth);                           \
+                           fg.grid * 4 * a.wcap, a.pool_cap, fs, a.skeys, a.sidx, a.cnt, a.base);                      \
+        hipLaunchKernelGGL(k_fpick, dim3(nranges), dim3(WG), 0, st, fs, k, nranges, nunits, upr, a.cnt, a.base,        \
+                           a.skeys, a.gq, a.rg, a.rq, a.lcap, a.lkey, a.lrange);                                       \
+        hipLaunchKernelGGL((k_fkth<K>), dim3(1), dim3(FS_NT), 0, st, fs, k, nranges, a.rg, a.rq, a.lcap, a.lkey,       \
+                           a.lrange, upr, a.gq, a.keys, n, (u32*)a.out_keys, a.out_idx, (u32*)a.d_kth);                \
         if (a.out_keys || a.out_idx)                                                                                   \
-            hipLaunchKernelGGL((k_fwrite<K>), dim3(nranges), dim3(WG), 0, st, fs, nunits, upr, a.cnt, a.base, a.skeys, \
-                               a.sidx, a.rg, a.rq, a.keys, n, k, (u32*)a.out_keys, a.out_idx);                         \
+            hipLaunchKernelGGL((k_fwrite<K>), dim3(nranges), dim3(WG), 0, st, fs, nranges, nunits, upr, a.cnt, a.base, \
+                               a.skeys, a.sidx, a.gq, a.rg, a.rq, a.keys, n, k, (u32*)a.out_keys, a.out_idx);          \
     } while (0)
     if (a.f32) F_LAUNCH(KeyF32);
     else F_LAUNCH(KeyU32);

@@ -217,8 +217,9 @@ struct FilterArgs {
     u32* sample;       // [2^lm + 2^14]
     u32* cnt;          // [units] kept | equal to the bound << 16
     u32* base;         // [units] first slot of the unit's kept keys
+    u32* gq;           // [units] of dense ranges: keys above the k-th | equal to it, low half
     u32 *rg, *rq;      // [F_RANGES]
-    u32 *lkey, *lrange;  // [64 * lcap]
+    u32 *lkey, *lrange;  // [64 * lcap]: the class's keys, and the range (or unit) of each
     u32 *skeys, *sidx;   // [4 * workgroups * wcap + pool_cap]
     void* out_keys;
     i64* out_idx;

@@ -1,8 +1,8 @@
 """GPU test of the filter pipeline on calls that it is known to serve (drtopk_select_route): its edges in k, a
-defeated sample of every size, ties between the ranks that its splitters cover, and a sample that places the k-th key
-five deviations too low.  Outputs must equal
-the oracle's and the general pipeline's bit for bit, and only a defeated sample may end in the
-one-workgroup selection from all keys."""
+defeated sample of every size, ties between the ranks that its splitters cover, a sample that places the k-th
+key five deviations too low, and units and ranges at the edges of being full.  Outputs must equal the oracle's
+and the general pipeline's bit for bit, and only a defeated sample may end in the one-workgroup selection from
+all keys."""
 import numpy as np
 import pytest
 
@@ -95,3 +95,31 @@ def test_unlucky_sample(orc, dt, n, k):  # noqa: F811
     print(f"[case] filter unlucky n={n} k={k}", flush=True)
     check(orc, dt, v, False, k, dt.ALGO_RADIX)
     assert filtered(dt, v, False, k)["last_resort"] == 0
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("counts", [(255, 256, 257), (2048,), (2047, 1, 0, 2048), (4, 256, 0, 512, 513, 1500)])
+@pytest.mark.parametrize("values", ["distinct", "tied", "ascending"])
+@pytest.mark.parametrize("n,k", [((1 << 22) + 5, 20_000), ((1 << 25) + 3, 40_001)])
+def test_full_units(orc, dt, values, counts, f32, n, k):  # noqa: F811
+    """1.5 k large keys, so many of them in every unit of 2048 as `counts` says in turn: units and ranges at and
+    beside the counts from which they are shared out over the grid."""
+    rng = np.random.default_rng(n + len(counts))
+    v = rng.integers(0, 1 << 30, n, dtype=np.uint32)
+    unit, left, at = n // 4096, 3 * k // 2, []
+    while left > 0:
+        c = min(counts[(unit - n // 4096) % len(counts)], left)
+        at.append(2048 * unit + np.sort(rng.choice(2048, c, replace=False)))
+        unit, left = unit + 1, left - c
+    at = np.concatenate(at)
+    if values == "distinct":
+        v[at] = rng.integers(1 << 31, 1 << 32, at.size, dtype=np.uint32)
+    elif values == "tied":
+        v[at] = rng.integers(0, 7, at.size, dtype=np.uint32) * np.uint32(1000) + np.uint32(1 << 31)
+    else:
+        v[at] = np.arange(at.size, dtype=np.uint32) + np.uint32(1 << 31)
+    if f32:
+        v = np.where(v >> 31 != 0, v ^ np.uint32(1 << 31), ~v).astype(np.uint32)
+    print(f"[case] filter units {values} {counts} n={n} k={k} f32={f32}", flush=True)
+    check(orc, dt, v, f32, k, dt.ALGO_RADIX)
+    assert filtered(dt, v, f32, k)["last_resort"] == 0
