@@ -187,13 +187,39 @@ __device__ __forceinline__ u32 wg_kth_between(It&& it, u32 lo, u32 hi, u32 k, Wg
         u32* M = L.misc + 4 * (pass & 1);
         const int bits = 32 - __clz((int)span);
         const int sh = bits > 11 ? bits - 11 : 0;
+        // Ties, or keys that an outlier leaves in one bin, would queue on one LDS word, 128 cycles a wave
+        // instruction: where a quarter of a wave's first keys share a bin, it counts that one in a register.
+        const u32 bins = span >> sh;
+        u32 heavy = 0, z = 0;
+        int mode = -1;
         it([&](const u32x4& x) {
+            if (mode < 0) {
+                const u32 b = (x[0] - base) >> sh;
+                heavy = (u32)__builtin_amdgcn_readfirstlane((int)b);
+                mode = heavy <= bins && __popcll(__ballot(b == heavy)) >= WAVE / 4 ? 1 : 0;
+            }
+            if (mode) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u32 d = x[j] - base;
-                if (d <= span) atomicAdd(&L.hist[d >> sh], 1u);
+                for (int j = 0; j < 4; ++j) {
+                    const u32 d = x[j] - base, b = d >> sh;
+                    const bool in = d <= span;
+                    z += in && b == heavy ? 1u : 0u;
+                    if (in && b != heavy) atomicAdd(&L.hist[b], 1u);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const u32 d = x[j] - base;
+                    if (d <= span) atomicAdd(&L.hist[d >> sh], 1u);
+                }
             }
         });
+        if (__ballot(mode > 0)) {
+            const u32 h0 = (u32)__builtin_amdgcn_readfirstlane((int)heavy);
+            const u32 all = wave_incl_scan_u32(heavy == h0 ? z : 0u);
+            if ((t & (WAVE - 1)) == WAVE - 1 && all) atomicAdd(&L.hist[h0], all);
+            if (heavy != h0 && z) atomicAdd(&L.hist[heavy], z);  // lanes that `it` visits apart
+        }
         if (t == 0) {
             M[0] = 0;
             L.misc[8] = 0;  // candidates collected

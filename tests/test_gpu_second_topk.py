@@ -1,6 +1,6 @@
 """GPU test of the short pipeline's second top-k on inputs that single out one branch of it each: sparse
-keys, whose k-th key lies in the bucket that starts at the lowest key of all, and ties that fill the k-th
-key's bucket of a concatenation held in LDS.  Outputs must equal the
+keys, whose k-th key lies in the bucket that starts at the lowest key of all, ties that fill the k-th key's
+bucket of a concatenation held in LDS, and one value that most keys share.  Outputs must equal the
 oracle's and the general pipeline's (the same call with stats) bit for bit."""
 import numpy as np
 import pytest
@@ -49,3 +49,17 @@ def test_tied_bucket(orc, dt, f32, n, k):  # noqa: F811
         v[tie:tie + 3 * k // 4] = np.uint32((1 << 30) + 12345)
         print(f"[case] tied bucket n={n} k={k} f32={f32} seed={seed}", flush=True)
         check(orc, dt, as_keys(orc, v, f32), f32, k, dt.ALGO_RADIX)
+
+
+@pytest.mark.parametrize("n,k", [(257, 100), (4096, 1000), (36_864, 30_000), (300_001, 2_000)])
+@pytest.mark.parametrize("share", [1.0, 0.9, 0.3])
+def test_heavy_value(orc, dt, share, n, k):  # noqa: F811
+    """One value that most keys share, an outlier above and a few keys below: every pass of a selection meets
+    waves full of one bucket."""
+    rng = np.random.default_rng(n)
+    v = rng.integers(0, 1 << 31, n, dtype=np.uint32)
+    v[rng.random(n) < share] = 1000
+    v[n // 3] = np.uint32(2 ** 32 - 1)
+    v[n // 2:n // 2 + 16] = 5
+    print(f"[case] heavy value n={n} k={k} share={share}", flush=True)
+    check(orc, dt, v, False, k, dt.ALGO_RADIX)
