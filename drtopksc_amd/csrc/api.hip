@@ -252,7 +252,7 @@ bool short_plan(const Plan& pl, ShortPlan* sp) {
         sp->f1 = f1;
         sp->f2 = f2;
         u64 o = align_up(sizeof(Ctrl), 256);
-        sp->o_dvals = o; o = align_up(o + 4 * S, 256);
+        sp->o_dvals = o; o = align_up(o + 4 * std::max(S, ns), 256);
         sp->o_sel = o; o = align_up(o + 4 * k, 256);
         sp->o_hist = o; o = align_up(o + 4 * 2048, 256);
         sp->o_cnt = o; o = align_up(o + 4 * ns, 256);
@@ -448,6 +448,7 @@ drtopk_status select_impl(const Plan& pl, const void* d_keys, void* d_workspace,
             sa.ghist = (u32*)(ws + sp.o_hist);
             sa.cnt = (u32*)(ws + sp.o_cnt);
             sa.segmax = (u32*)(ws + sp.o_max);
+            sa.rcnt = sa.dvals;
             sa.skeys = (u32*)(ws + sp.o_skeys);
             sa.sidx = (u32*)(ws + sp.o_sidx);
             HIPCHK(launch_short(sa, st));

@@ -108,7 +108,10 @@ struct Ctrl {
     u64 count_gt;         // keys > k-th largest
     u64 ties;             // keys == k-th largest in the top-k set
     u32 kth;              // ordered bits of the k-th largest
-    u32 pad[15];
+    u32 arrived;          // short pipeline: workgroups of the last kernel that have reduced their segments
+    u32 bin_lo, bin_hi;   // and the least and largest key they found in the k-th key's bucket
+    u32 bucket_sh;        // and how its buckets lie
+    u32 pad[11];
 };
 
 enum : u32 {

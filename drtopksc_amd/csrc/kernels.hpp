@@ -171,6 +171,7 @@ struct ShortArgs {
     u32* sidx;         // and indices
     u32* cnt;          // [short_segments]
     u32* segmax;       // [short_segments]
+    u32* rcnt;         // [short_segments] counts of the reduced segments: the delegates' area, dead by then
     void* out_keys;
     i64* out_idx;
     void* d_kth;

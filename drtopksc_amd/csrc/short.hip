@@ -13,11 +13,14 @@
 //            ranges hold the k largest delegates for the same reason that the k largest
 //            subranges hold the k largest keys.
 //  k_collect keys >= T of those subranges with their indices, a segment per workgroup
-//            (CreateConcatenateRange_optimized, radixselect.cuh:1575-1607), counted into 2048
-//            buckets of [T, largest key] on the way.
+//            (CreateConcatenateRange_optimized, radixselect.cuh:1575-1607), counted into
+//            buckets of their distance from T on the way.
 //  k_final   second top-k over the concatenation and the index-ordered outputs
-//            (radixselect.cuh:1411-1470, MultiGPU/radixselect.cuh:1355-1383).
+//            (radixselect.cuh:1411-1470, MultiGPU/radixselect.cuh:1355-1383), by one workgroup where
+//            the concatenation fits its LDS; clustered and tied keys leave up to 2^24 of them, which
+//            several workgroups first reduce to those that can be in the top k.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -118,12 +121,31 @@ __global__ __launch_bounds__(WG) void k_super(const u32* __restrict__ dvals, u32
 }
 
 // ---------------------------------------------------------------- first top-k and range selection
-// Buckets of [T, hi] that k_collect counts into.
-__device__ __forceinline__ int collect_shift(u32 T, u32 hi) {
-    const u32 span = hi - T;
-    const int bits = span ? 32 - __clz((int)span) : 0;
-    return bits > 11 ? bits - 11 : 0;
-}
+// Buckets that k_collect counts into, by the distance of a key from T; bucket 0 is T alone.  Equal ones of
+// 2^sh values up to the largest delegate, which keep sorted keys apart; or, where few of the selected
+// delegates lie in the upper 31/32 of that range (an outlier, a heavy tail: all other keys would share a
+// bucket), 64 to each power of two (LOG_BUCKETS).
+constexpr int DB_BITS = 6;
+constexpr u32 LOG_BUCKETS = 64;
+struct Buckets {
+    int lo, hi;  // least and largest bits dropped from a distance
+    __device__ __forceinline__ explicit Buckets(u32 sh)
+        : lo(sh == LOG_BUCKETS ? 0 : (int)sh), hi(sh == LOG_BUCKETS ? 31 - DB_BITS : (int)sh) {}
+    __device__ __forceinline__ u32 of(u32 d) const {  // d >= 1
+        d -= 1;
+        const int e = min(max(31 - DB_BITS - __clz((int)(d | 1u)), lo), hi);
+        return min(1 + ((u32)(e - lo) << DB_BITS) + (d >> e), (u32)WS_BINS - 1);
+    }
+    // The least distance in bucket b, and the bucket's width less 1.
+    __device__ __forceinline__ u32 from(u32 b, u32* span) const {
+        *span = 0;
+        if (b == 0) return 0;
+        const u32 c = b - 1, e = lo == hi ? (u32)lo : (c >> (DB_BITS + 1) ? (c >> DB_BITS) - 1 : 0u);
+        *span = ((b == WS_BINS - 1 ? 2u : 1u) << e) - 1;  // the last one takes what the range leaves over
+        return 1 + ((c - ((e - (u32)lo) << DB_BITS)) << e);
+    }
+};
+static_assert(((32 - DB_BITS + 1) << DB_BITS) + 1 < WS_BINS, "buckets of every distance");
 
 // The k largest delegates, lowest ids first among equals.  With f1 == 0 from the S delegates at once;
 // otherwise from the topmost maxima down (sup2 when f2 > 0, sup1, the delegates), each level
@@ -139,7 +161,13 @@ __global__ __launch_bounds__(SH_NT) void k_first(const u32* __restrict__ dvals, 
     __shared__ __align__(16) u32 el[wg_words<SH_NT>(CAP)];
     __shared__ u32 lists[LISTK ? 3 * LISTK : 1];
     const int t = threadIdx.x;
-    if (t == 0) ws_head_begin(&ctrl->head);
+    if (t == 0) {
+        ws_head_begin(&ctrl->head);
+        ctrl->arrived = 0;
+        ctrl->bin_lo = 0xFFFFFFFFu;
+        ctrl->bin_hi = 0;
+        L.misc[11] = 0;
+    }
     wg_init<SH_NT>(L);
 #pragma unroll
     for (int j = 0; j < WS_BINS / SH_NT; ++j) ghist[j * SH_NT + t] = 0;
@@ -161,18 +189,27 @@ __global__ __launch_bounds__(SH_NT) void k_first(const u32* __restrict__ dvals, 
         auto each = [&](auto&& f) { wg_each(el, ni, f); };
         if (level == top) T = wg_kth<SH_NT>(each, k, L, &gt);
         else T = wg_kth_between<SH_NT>(each, T, L.hi, k, L, &gt);  // the level above bounds this one's
-        if (level == 0 && t == 0) {
-            ctrl->first.result = T;
-            ctrl->first.hi = L.hi;
-        }
-        if (top == 0) {
-            wg_emit<SH_NT>(el, ni, T, gt, k - gt, L, [&](u32 p, u32 e, u32) { sel_ids[p] = e; });
-            return;
-        }
+        // the selected delegates in the upper 31/32 of their range
+        const u32 range = L.hi - T;
+        u32 far = 0;
         // the values' numbers first, then their ids all at once: reading the list where a value is
         // emitted would wait for it there
-        wg_emit<SH_NT>(el, ni, T, gt, k - gt, L, [&](u32 p, u32 e, u32) { picked[p] = e; });
+        u32* const to = top == 0 ? sel_ids : picked;
+        wg_emit<SH_NT>(el, ni, T, gt, k - gt, L, [&](u32 p, u32 e, u32 x) {
+            to[p] = e;
+            far += x - T > range >> 5 ? 1u : 0u;
+        });
+        if (level == 0) {
+            far = wave_incl_scan_u32(far);
+            if ((t & (WAVE - 1)) == WAVE - 1 && far) atomicAdd(&L.misc[11], far);
+        }
         __syncthreads();
+        if (level == 0 && t == 0) {
+            const u32 bits = range ? 32 - __clz((int)range) : 0;
+            ctrl->first.result = T;
+            ctrl->bucket_sh = L.misc[11] < k / 32 ? LOG_BUCKETS : (bits > 11 ? bits - 11 : 0);
+        }
+        if (top == 0) return;
         u32* next = picked + (level == 1 ? k : 2 * k);
         for (u32 p = t; p < k; p += SH_NT) (level == 0 ? sel_ids : next)[p] = id(picked[p]);
         list = next;
@@ -183,7 +220,8 @@ __global__ __launch_bounds__(SH_NT) void k_first(const u32* __restrict__ dvals, 
 // ---------------------------------------------------------------- concatenation
 // Workgroup s takes slots [s*4096, (s+1)*4096) of the selected subranges laid back to back (alpha >=
 // 2), 16 consecutive slots per thread, and leaves the keys >= T in index order at [s*4096, ...), their
-// count and how many equal T, and the largest of them.
+// count and how many equal T, and the largest of them.  The buckets leave out the keys equal to T, which
+// would all go to one word (2^26 keys, one value and an outlier, k = 8192: 345 us for the call).
 constexpr u32 COLLECT_TILE = 4096;
 
 template <class K, bool IDX>
@@ -206,7 +244,7 @@ __global__ __launch_bounds__(WG) void k_collect(const u32* __restrict__ keys, u3
 #pragma unroll
     for (int q = 0; q < 4; ++q) r[q] = *(const u32x4*)(keys + (g[q] + 4 <= n ? g[q] : 0u));
     const u32 T = ctrl->first.result;
-    const int sh = collect_shift(T, ctrl->first.hi);
+    const Buckets bk(ctrl->bucket_sh);
 #pragma unroll
     for (int j = 0; j < WS_BINS / WG; ++j) lh[j * WG + threadIdx.x] = 0;
     u32 take = 0, eq = 0, mx = 0;  // take: bit per slot
@@ -230,16 +268,25 @@ __global__ __launch_bounds__(WG) void k_collect(const u32* __restrict__ keys, u3
     u32 tot;  // survivors | keys equal to T << 16, at most 4096 each
     u32 slot = block_excl_scan_u32<WG>((u32)__popc(take) | (eq << 16), scratch, &tot) & 0xFFFFu;
     const u32 base = blockIdx.x * COLLECT_TILE;
+    u32 cur = 0, run = 0;  // sorted keys: a thread's run in one bucket with one atomic
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         if (take & (1u << j)) {
             const u32 o = r[j >> 2][j & 3];
             skeys[base + slot] = o;
             if (IDX) sidx[base + slot] = g[j >> 2] + (u32)(j & 3);
-            atomicAdd(&lh[(o - T) >> sh], 1u);
             ++slot;
+            if (o == T) continue;
+            const u32 b = bk.of(o - T);
+            if (b != cur) {
+                if (cur) atomicAdd(&lh[cur], run);
+                cur = b;
+                run = 0;
+            }
+            ++run;
         }
     }
+    if (cur) atomicAdd(&lh[cur], run);
     mx = wave_max_last(mx);
     if ((threadIdx.x & (WAVE - 1)) == WAVE - 1) wmax[threadIdx.x / WAVE] = mx;
     __syncthreads();
@@ -256,20 +303,27 @@ __global__ __launch_bounds__(WG) void k_collect(const u32* __restrict__ keys, u3
 
 // ---------------------------------------------------------------- second top-k and extraction
 constexpr u32 FIN_CAP = 12288;  // concatenation held in LDS (k <= 8192 random keys leave 11.4 K)
+constexpr u32 FIN_WGS = 128;    // most workgroups of k_final
+constexpr u32 FIN_ALONE = 32;   // segments from which one workgroup takes the keys it needs without the others
 
+// One workgroup holds a concatenation of up to FIN_CAP keys in LDS, or, of a longer one, those from the k-th
+// key's bucket up where they lie in few segments (sorted keys); the others then have nothing to do.  Else
+// (up to 2^24 keys) all of them first reduce it: to the keys from the k-th key's bucket
+// up, or, where fewer than k keys lie above T, to the outputs themselves, whose places the counts of the
+// segments tell.  One workgroup alone read 2^19 .. 2^20 keys in 100 us and more (2^24 keys, a sixteenth of
+// them large in one block, k = 8192: 203 us for the call).  The workgroup that arrives last goes on with
+// what the others left; none waits.
 template <class K>
-__global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, const u32* __restrict__ sidx,
-                                                 const u32* __restrict__ cnt, const u32* __restrict__ segmax,
-                                                 const u32* __restrict__ ghist, u32 nseg, u32 k, Ctrl* ctrl,
-                                                 u32* __restrict__ out_keys, i64* __restrict__ out_idx,
-                                                 u32* __restrict__ d_kth) {
+__global__ __launch_bounds__(SH_NT) void k_final(u32* skeys, u32* sidx, const u32* __restrict__ cnt,
+                                                 const u32* __restrict__ segmax, const u32* __restrict__ ghist, u32 nseg,
+                                                 u32 k, Ctrl* ctrl, u32* rcnt, u32* __restrict__ out_keys,
+                                                 i64* __restrict__ out_idx, u32* __restrict__ d_kth) {
     __shared__ WgSel<SH_NT> L;
     __shared__ u32 pref[SHORT_SEGS + 1];  // keys before each segment
     __shared__ __align__(16) u32 el[wg_words<SH_NT>(FIN_CAP)], ix[wg_words<SH_NT>(FIN_CAP)];
     const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE;
     constexpr int SPT = SHORT_SEGS / SH_NT, PER = WS_BINS / SH_NT;
-    const u32 T = ctrl->first.result, hi = ctrl->first.hi;
-    const int sh = collect_shift(T, hi);
+    const u32 T = ctrl->first.result;
     u32 hc[PER], pc[SPT];  // this thread's buckets and segments
 #pragma unroll
     for (int j = 0; j < PER; ++j) hc[j] = ghist[WS_BINS - 1 - (t * PER + j)];
@@ -280,31 +334,235 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
         L.misc[8] = 0;
     }
     wg_init<SH_NT>(L);
-    u32 C, Q = 0;  // entries, and those equal to T
-    {
-        u32 s = 0, q = 0;
+    // keys before each segment, from the low halves of pc; returns their number
+    auto set_pref = [&]() {
+        u32 s = 0, tot;
 #pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            s += pc[j] & 0xFFFFu;
-            q += pc[j] >> 16;
-        }
-        wg_excl_scan<SH_NT>(q, L.b, &Q);
-        u32 run = wg_excl_scan<SH_NT>(s, L.a, &C);
+        for (int j = 0; j < SPT; ++j) s += pc[j] & 0xFFFFu;
+        u32 run = wg_excl_scan<SH_NT>(s, L.a, &tot);
 #pragma unroll
         for (int j = 0; j < SPT; ++j) {
             pref[t * SPT + j] = run;
             run += pc[j] & 0xFFFFu;
         }
-        if (t == SH_NT - 1) pref[SHORT_SEGS] = C;
-    }
+        if (t == SH_NT - 1) pref[SHORT_SEGS] = tot;
+        return tot;
+    };
+    u32 C = set_pref(), Q, q = 0;  // entries, and those equal to T, which the buckets leave out
+#pragma unroll
+    for (int j = 0; j < SPT; ++j) q += pc[j] >> 16;
+    wg_excl_scan<SH_NT>(q, L.b, &Q);
+    if (t == SH_NT - 1) hc[PER - 1] += Q;
     wg_find_bin<SH_NT>(hc, k, L, L.misc);
     __syncthreads();
     if (C < k || L.misc[0] == 0xFFFFFFFFu) {  // not for valid input: every key of the top-k set is here
-        if (t == 0) ctrl_fail(ctrl, ERR_CONCAT_SHORT);
+        if (t == 0 && blockIdx.x == 0) ctrl_fail(ctrl, ERR_CONCAT_SHORT);
         return;
     }
     const u32 kth_bin = L.misc[0], above = L.misc[1], in_bin = L.misc[2];
     __syncthreads();  // the selection below reuses misc, and no barrier need come before it
+    const bool at_t = C - Q < k;  // fewer than k keys above T: ties at T fill the rest
+    const u32 kk = k - above;
+    u32 span;
+    const u32 base = T + Buckets(ctrl->bucket_sh).from(kth_bin, &span);
+    span = min(span, 0xFFFFFFFFu - base);
+    // f(keys, indices, m, i) for every lane of each 256-slot step of segment s by one wave, `U` 16-byte
+    // loads of each in flight; m the lane's valid keys from slot i on
+    auto each_of = [&](u32 s, auto U, auto&& f) {
+        constexpr u32 N = decltype(U)::value;
+        const u32 c = pref[s + 1] - pref[s];
+        const u32 *p = skeys + (u64)s * COLLECT_TILE, *pi = sidx + (u64)s * COLLECT_TILE;
+        for (u32 i0 = 0; i0 < c; i0 += N * 4 * WAVE) {
+            u32x4 x[N], y[N];
+#pragma unroll
+            for (u32 u = 0; u < N; ++u) {
+                const u32 at = min(i0 + 4 * (u * WAVE + lane), COLLECT_TILE - 4);
+                x[u] = *(const u32x4*)(p + at);
+                y[u] = out_idx ? *(const u32x4*)(pi + at) : u32x4{0, 0, 0, 0};
+            }
+#pragma unroll
+            for (u32 u = 0; u < N; ++u) {
+                const u32 i = i0 + 4 * (u * WAVE + lane);
+                if (i0 + 4 * u * WAVE < c) f(x[u], y[u], i < c ? min(c - i, 4u) : 0u, i);
+            }
+        }
+    };
+    constexpr std::integral_constant<u32, 4> U4{};
+    // the outputs of the segments first, first + step, .. for this wave: keys > K0, `gt` of them in all, and
+    // the first ties; sg and sq hold the counts of each segment's keys above and equal to K0
+    u32* sg = el;
+    u32* sq = ix;
+    auto write_segments = [&](u32 K0, u32 ties, u32 first, u32 step) {
+        __syncthreads();
+        {
+            u32 g[SPT], q[SPT], gs = 0, qs = 0, tot;
+#pragma unroll
+            for (int j = 0; j < SPT; ++j) {
+                g[j] = sg[t * SPT + j];
+                q[j] = sq[t * SPT + j];
+                gs += g[j];
+                qs += q[j];
+            }
+            u32 gr = wg_excl_scan<SH_NT>(gs, L.a, &tot);
+            u32 qr = wg_excl_scan<SH_NT>(qs, L.b, &tot);
+#pragma unroll
+            for (int j = 0; j < SPT; ++j) {
+                // a segment with nothing to write is marked by an impossible first output
+                const bool none = g[j] == 0 && (q[j] == 0 || qr >= ties);
+                sg[t * SPT + j] = none ? 0xFFFFFFFFu : gr;
+                sq[t * SPT + j] = qr;
+                gr += g[j];
+                qr += q[j];
+            }
+        }
+        __syncthreads();
+        for (u32 s = first; s < nseg; s += step) {
+            u32 gr = sg[s], qr = sq[s];
+            if (gr == 0xFFFFFFFFu) continue;
+            each_of(s, U4, [&](const u32x4& x, const u32x4& y, u32 m, u32) {
+                u32 mine = 0;  // above << 16 | ties
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j) mine += j < m ? (x[j] > K0 ? 0x10000u : (x[j] == K0 ? 1u : 0u)) : 0u;
+                if (__ballot(mine != 0) == 0) return;
+                const u32 inc = wave_incl_scan_u32(mine);
+                u32 gb = gr + ((inc - mine) >> 16), qb = qr + ((inc - mine) & 0xFFFFu);
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j) {
+                    if (j >= m || x[j] < K0) continue;
+                    if (x[j] > K0 || qb < ties) {
+                        const u32 p = gb + min(qb, ties);
+                        if (out_keys && p < k) out_keys[p] = K::from_ord(x[j]);
+                        if (out_idx && p < k) out_idx[p] = (i64)y[j];
+                    }
+                    gb += x[j] > K0 ? 1u : 0u;
+                    qb += x[j] == K0 ? 1u : 0u;
+                }
+                const u32 all = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+                gr += all >> 16;
+                qr += all & 0xFFFFu;
+            });
+        }
+    };
+    bool held = C <= FIN_CAP, placed = false, tied = false;
+    u32 f = 0, nv = 0;  // this thread's segments with a key >= base, and how many there are
+    if (!held && !at_t) {
+#pragma unroll
+        for (int j = 0; j < SPT; ++j) f |= (u32)(t * SPT + j) < nseg && segmax[t * SPT + j] >= base ? 1u << j : 0u;
+        f |= wg_excl_scan<SH_NT>((u32)__popc(f), L.a, &nv) << SPT;
+        placed = above + in_bin <= FIN_CAP && nv <= FIN_ALONE;
+    }
+    if (held || placed) {
+        if (blockIdx.x) return;
+    }
+    if (held) {
+    } else if (placed) {
+        // the keys from the bucket up fit and lie in few segments: counted per segment, then placed in order
+        // as if they were the whole concatenation
+        u32 at = f >> SPT;
+#pragma unroll
+        for (int j = 0; j < SPT; ++j)
+            if (f >> j & 1) L.cand[at++] = (u32)(t * SPT + j);
+        C = above + in_bin;
+        const u32 ni = (u32)wg_granules<SH_NT>(C);
+        for (u32 i = 0; i < ni; ++i) *(u32x4*)(el + 4 * (t * (ni | 1) + i)) = u32x4{0, 0, 0, 0};
+        __syncthreads();
+        for (u32 v = w; v < nv; v += SH_NT / WAVE) {
+            u32 c = 0;
+            each_of(L.cand[v], U4, [&](const u32x4& x, const u32x4&, u32 m, u32) {
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j) c += j < m && x[j] >= base ? 1u : 0u;
+            });
+            c = wave_incl_scan_u32(c);
+            if (lane == WAVE - 1) L.hist[v] = c;
+        }
+        __syncthreads();
+        for (u32 v = w; v < nv; v += SH_NT / WAVE) {
+            const u32 inc = wave_incl_scan_u32((u32)lane < v ? L.hist[lane & (FIN_ALONE - 1)] : 0u);
+            u32 to = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+            each_of(L.cand[v], U4, [&](const u32x4& x, const u32x4& y, u32 m, u32) {
+                u32 c = 0;
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j) c += j < m && x[j] >= base ? 1u : 0u;
+                const u32 inc = wave_incl_scan_u32(c);
+                u32 e = to + inc - c;
+#pragma unroll
+                for (u32 j = 0; j < 4; ++j)
+                    if (j < m && x[j] >= base) {
+                        const u32 o = e / (4 * ni), q = 4 * o * (ni | 1) + (e - 4 * ni * o);
+                        el[q] = x[j];
+                        ix[q] = y[j];
+                        ++e;
+                    }
+                to += (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+            });
+        }
+        __syncthreads();
+        wg_init<SH_NT>(L);
+        __syncthreads();
+        held = true;
+    } else if (at_t) {
+        if (t == 0 && blockIdx.x == 0 && d_kth) *d_kth = K::from_ord(T);
+        if (!out_keys && !out_idx) return;
+#pragma unroll
+        for (int j = 0; j < SPT; ++j) {
+            sg[t * SPT + j] = (pc[j] & 0xFFFFu) - (pc[j] >> 16);
+            sq[t * SPT + j] = pc[j] >> 16;
+        }
+        write_segments(T, k - (C - Q), blockIdx.x * (SH_NT / WAVE) + w, gridDim.x * (SH_NT / WAVE));
+        return;
+    } else {
+        // this workgroup's segments to their keys >= base, in place: a wave has read what it overwrites.  Counts
+        // of keys | keys of the bucket << 16; its least and largest key tell whether it is one value.
+        u32 blo = 0xFFFFFFFFu, bhi = 0;
+        for (u32 s = blockIdx.x * (SH_NT / WAVE) + w; s < nseg; s += gridDim.x * (SH_NT / WAVE)) {
+            u32 to = 0, b = 0;
+            if (segmax[s] >= base) {
+                u32 *p = skeys + (u64)s * COLLECT_TILE, *pi = sidx + (u64)s * COLLECT_TILE;
+                each_of(s, U4, [&](const u32x4& x, const u32x4& y, u32 m, u32) {
+                    u32 c = 0;
+#pragma unroll
+                    for (u32 j = 0; j < 4; ++j) c += j < m && x[j] >= base ? 1u : 0u;
+                    const u32 inc = wave_incl_scan_u32(c);
+                    u32 e = to + inc - c;
+#pragma unroll
+                    for (u32 j = 0; j < 4; ++j)
+                        if (j < m && x[j] >= base) {
+                            p[e] = x[j];
+                            if (out_idx) pi[e] = y[j];
+                            ++e;
+                            if (x[j] - base <= span) {
+                                ++b;
+                                blo = min(blo, x[j]);
+                                bhi = max(bhi, x[j]);
+                            }
+                        }
+                    to += (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
+                });
+            }
+            b = wave_incl_scan_u32(b);
+            if (lane == WAVE - 1) rcnt[s] = to | b << 16;
+        }
+        bhi = wave_max_last(bhi);
+        blo = ~wave_max_last(~blo);
+        if (lane == WAVE - 1 && bhi >= base) {
+            atomicMin(&ctrl->bin_lo, blo);
+            atomicMax(&ctrl->bin_hi, bhi);
+        }
+        __threadfence();  // the keys and counts before the arrival
+        __syncthreads();
+        if (t == 0) L.misc[11] = atomicAdd(&ctrl->arrived, 1u);
+        __syncthreads();
+        if (L.misc[11] != gridDim.x - 1) return;
+        __threadfence();
+#pragma unroll
+        for (int j = 0; j < SPT; ++j) pc[j] = (u32)(t * SPT + j) < nseg ? rcnt[t * SPT + j] : 0u;
+        tied = __hip_atomic_load(&ctrl->bin_lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               __hip_atomic_load(&ctrl->bin_hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        C = set_pref();
+        held = C <= FIN_CAP;
+        __syncthreads();
+    }
     // concatenation element e: its segment is the last one starting at or before e (an empty
     // segment shares its start with the next one, which is the one found)
     auto seg_of = [&](u32 e) {
@@ -314,10 +572,9 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
             if (pref[lo + step] <= e) lo += step;
         return lo;
     };
-    bool held = C <= FIN_CAP;
-    int ni = wg_granules<SH_NT>(C);
-    u32 own = 4 * (u32)t * ((u32)ni | 1);  // this thread's elements in el and ix
-    if (held) {  // every thread fetches its own consecutive elements
+    const int ni = wg_granules<SH_NT>(C);
+    const u32 own = 4 * (u32)t * ((u32)ni | 1);  // this thread's elements in el and ix
+    if (held && !placed) {  // every thread fetches its own consecutive elements
         const u32 e0 = 4 * (u32)(t * ni);
         u32 s = e0 < C ? seg_of(e0) : 0u;
 #pragma unroll 2
@@ -338,138 +595,40 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
             *(u32x4*)(ix + own + 4 * i) = y;
         }
     }
-    // one wave over slots [i0, i1) of segment s (i0 a multiple of 4), eight 16-byte loads in flight:
-    // f(keys, m, i) for every lane of each 256-slot step, m the lane's valid keys from slot i on
-    auto each_in = [&](u32 s, u32 i0, u32 i1, auto&& f) {
-        const u32 c = min(pref[s + 1] - pref[s], i1);
-        const u32* p = skeys + (u64)s * COLLECT_TILE;
-        for (; i0 < c; i0 += 32 * WAVE) {
-            u32x4 x[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) x[u] = *(const u32x4*)(p + min(i0 + 4 * (u * WAVE + lane), COLLECT_TILE - 4));
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const u32 i = i0 + 4 * (u * WAVE + lane);
-                if (i0 + 4 * u * WAVE < c) f(x[u], i < c ? min(c - i, 4u) : 0u, i);
-            }
-        }
-    };
-    auto each_of = [&](u32 s, auto&& f) { each_in(s, 0, COLLECT_TILE, f); };
     u32 K0, gt;
-    if (C - Q < k) {  // fewer than k keys above T: ties at T fill the rest
+    if (at_t) {
         K0 = T;
         gt = C - Q;
-    } else {
-        // the k-th key's bucket, then its rank among the bucket's keys
-        const u32 base = T + (kth_bin << sh), kk = k - above;
-        const u32 span = min((1u << sh) - 1u, hi - base);
-        if (!held && above + in_bin <= FIN_CAP) {
-            // clustered keys: the concatenation exceeds LDS, but the keys from the bucket up fit.  The
-            // segments that reach it, in units of 2048 slots over the waves: counted, then placed in
-            // order as if they were the whole concatenation
-            u32 f = 0, nv;
-#pragma unroll
-            for (int j = 0; j < SPT; ++j) f |= (u32)(t * SPT + j) < nseg && segmax[t * SPT + j] >= base ? 1u << j : 0u;
-            u32 at = wg_excl_scan<SH_NT>((u32)__popc(f), L.a, &nv);
-            constexpr u32 UNIT = 32 * WAVE, UPS = COLLECT_TILE / UNIT;  // units per segment
-            if (nv * UPS <= (u32)WS_BINS && nv <= WgSel<SH_NT>::CAND) {
-#pragma unroll
-                for (int j = 0; j < SPT; ++j)
-                    if (f & (1u << j)) L.cand[at++] = (u32)(t * SPT + j);
-                __syncthreads();
-                for (u32 u = w; u < nv * UPS; u += SH_NT / WAVE) {
-                    u32 c = 0;
-                    each_in(L.cand[u / UPS], u % UPS * UNIT, u % UPS * UNIT + UNIT,
-                            [&](const u32x4& x, u32 m, u32) {
-#pragma unroll
-                                for (u32 j = 0; j < 4; ++j) c += j < m && x[j] >= base ? 1u : 0u;
-                            });
-                    c = wave_incl_scan_u32(c);
-                    if (lane == WAVE - 1) L.hist[u] = c;
-                }
-                C = above + in_bin;
-                ni = wg_granules<SH_NT>(C);
-                own = 4 * (u32)t * ((u32)ni | 1);
-                for (int i = 0; i < ni; ++i) *(u32x4*)(el + own + 4 * i) = u32x4{0, 0, 0, 0};
-                __syncthreads();
-                u32 c[PER], n = 0, tot;
-#pragma unroll
-                for (int j = 0; j < PER; ++j) n += c[j] = L.hist[t * PER + j];
-                n = wg_excl_scan<SH_NT>(n, L.a, &tot);
-#pragma unroll
-                for (int j = 0; j < PER; ++j) {
-                    L.hist[t * PER + j] = n;
-                    n += c[j];
-                }
-                __syncthreads();
-                for (u32 u = w; u < nv * UPS; u += SH_NT / WAVE) {
-                    const u32 s = L.cand[u / UPS];
-                    u32 to = L.hist[u];
-                    each_in(s, u % UPS * UNIT, u % UPS * UNIT + UNIT, [&](const u32x4& x, u32 m, u32 i) {
-                        u32 c = 0;
-#pragma unroll
-                        for (u32 j = 0; j < 4; ++j) c += j < m && x[j] >= base ? 1u : 0u;
-                        const u32 inc = wave_incl_scan_u32(c);
-                        u32 e = to + inc - c;
-#pragma unroll
-                        for (u32 j = 0; j < 4; ++j)
-                            if (j < m && x[j] >= base) {
-                                const u32 o = e / (4 * (u32)ni), q = 4 * o * ((u32)ni | 1) + (e - 4 * (u32)ni * o);
-                                el[q] = x[j];
-                                if (out_idx) ix[q] = sidx[(u64)s * COLLECT_TILE + i + j];
-                                ++e;
-                            }
-                        to += (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
-                    });
-                }
-                __syncthreads();
-                wg_init<SH_NT>(L);
-                __syncthreads();
-                held = true;
-            }
-        }
-        if (span == 0) {
-            K0 = base;
-            gt = above;
-        } else if (held && in_bin <= WgSel<SH_NT>::CAND && base) {
-            // (a bucket that starts at 0 would take in the zeros past the concatenation, which its count
-            // doesn't cover: below, they count as keys of their own)
+    } else if (span == 0 || tied) {
+        K0 = tied ? __hip_atomic_load(&ctrl->bin_lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : base;
+        gt = above;
+    } else if (held && in_bin <= WgSel<SH_NT>::CAND) {
+        // (base > T, so the zeros past the concatenation, which the bucket's count does not cover, are not in it)
 #pragma unroll 1
-            for (int i = 0; i < ni; ++i) wg_collect<SH_NT>(*(const u32x4*)(el + own + 4 * i), base, span, L);
-            __syncthreads();
-            u32 g;
-            K0 = wg_rank<SH_NT>(in_bin, kk, L, &g);
-            gt = above + g;
-        } else {
-            // more keys than can be ranked directly (ties), or a concatenation larger than LDS (clustered
-            // keys): its segments that reach the bucket are streamed once for the bucket's keys, or in
-            // every pass when they do not fit either
-            const bool fits = !held && in_bin <= FIN_CAP;
-            auto keys_of_bin = [&](auto&& f) {
-                for (u32 s = w; s < nseg; s += SH_NT / WAVE)
-                    if (segmax[s] >= base)
-                        each_of(s, [&](const u32x4& x, u32 m, u32) {
+        for (int i = 0; i < ni; ++i) wg_collect<SH_NT>(*(const u32x4*)(el + own + 4 * i), base, span, L);
+        __syncthreads();
+        u32 g;
+        K0 = wg_rank<SH_NT>(in_bin, kk, L, &g);
+        gt = above + g;
+    } else {
+        // more keys than can be ranked directly: from LDS, or read from memory on every pass
+        K0 = wg_kth_between<SH_NT>(
+            [&](auto&& f) {
+                if (held) {
+                    wg_each(el, ni, f);
+                } else {
+                    for (u32 s = w; s < nseg; s += SH_NT / WAVE)
+                        each_of(s, U4, [&](const u32x4& x, const u32x4&, u32 m, u32) {
+                            // (a key below the bucket, of which there are none left, for the slots past the end)
+                            u32x4 v;
 #pragma unroll
-                            for (u32 j = 0; j < 4; ++j)
-                                if (j < m && x[j] - base <= span) f(x[j]);
+                            for (u32 j = 0; j < 4; ++j) v[j] = j < m ? x[j] : base - 1;
+                            f(v);
                         });
-            };
-            if (fits) {
-                keys_of_bin([&](u32 x) { el[atomicAdd(&L.misc[8], 1u)] = x; });
-                __syncthreads();
-            }
-            K0 = wg_kth_between<SH_NT>(
-                [&](auto&& f) {
-                    if (held)
-                        wg_each(el, ni, f);
-                    else if (fits)
-                        for (u32 i = t; i < in_bin; i += SH_NT) f(u32x4{el[i], 0, 0, 0});
-                    else
-                        keys_of_bin([&](u32 x) { f(u32x4{x, 0, 0, 0}); });
-                },
-                base, base + span, kk, L, &gt);
-            gt += above;
-        }
+                }
+            },
+            base, base + span, kk, L, &gt);
+        gt += above;
     }
     if (t == 0 && d_kth) *d_kth = K::from_ord(K0);
     if (!out_keys && !out_idx) return;
@@ -483,22 +642,17 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
         });
         return;
     }
-    // keys > K0 and == K0 of every segment (a segment whose largest key is below K0 has none; at
-    // K0 == T k_collect counted them), then their exclusive prefixes, in the LDS of el and ix
-    u32* sg = el;
-    u32* sq = ix;
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < SPT; ++j) {
-        sg[t * SPT + j] = K0 == T ? (pc[j] & 0xFFFFu) - (pc[j] >> 16) : 0u;
-        sq[t * SPT + j] = K0 == T ? pc[j] >> 16 : 0u;
+        sg[t * SPT + j] = (pc[j] & 0xFFFFu) - (pc[j] >> 16);
+        sq[t * SPT + j] = pc[j] >> 16;
     }
-    if (K0 != T) {
+    if (span && !tied) {  // the bucket holds more than one value
         __syncthreads();
         for (u32 s = w; s < nseg; s += SH_NT / WAVE) {
-            if (segmax[s] < K0) continue;
             u32 g = 0, q = 0;
-            each_of(s, [&](const u32x4& x, u32 m, u32) {
+            each_of(s, U4, [&](const u32x4& x, const u32x4&, u32 m, u32) {
 #pragma unroll
                 for (u32 j = 0; j < 4; ++j) {
                     g += j < m && x[j] > K0 ? 1u : 0u;
@@ -513,58 +667,7 @@ __global__ __launch_bounds__(SH_NT) void k_final(const u32* __restrict__ skeys, 
             }
         }
     }
-    __syncthreads();
-    {
-        u32 g[SPT], q[SPT], gs = 0, qs = 0, tot;
-#pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            g[j] = sg[t * SPT + j];
-            q[j] = sq[t * SPT + j];
-            gs += g[j];
-            qs += q[j];
-        }
-        u32 gr = wg_excl_scan<SH_NT>(gs, L.a, &tot);
-        u32 qr = wg_excl_scan<SH_NT>(qs, L.b, &tot);
-#pragma unroll
-        for (int j = 0; j < SPT; ++j) {
-            // a segment with nothing to write is marked by an impossible first output
-            const bool none = g[j] == 0 && (q[j] == 0 || qr >= ties);
-            sg[t * SPT + j] = none ? 0xFFFFFFFFu : gr;
-            sq[t * SPT + j] = qr;
-            gr += g[j];
-            qr += q[j];
-        }
-    }
-    __syncthreads();
-    for (u32 s = w; s < nseg; s += SH_NT / WAVE) {
-        u32 gr = sg[s], qr = sq[s];
-        if (gr == 0xFFFFFFFFu) continue;
-        const u32* si = sidx + (u64)s * COLLECT_TILE;
-        each_of(s, [&](const u32x4& x, u32 m, u32 i) {
-            u32 g = 0, q = 0;
-#pragma unroll
-            for (u32 j = 0; j < 4; ++j) {
-                g += j < m && x[j] > K0 ? 1u : 0u;
-                q += j < m && x[j] == K0 ? 1u : 0u;
-            }
-            const u32 mine = (g << 16) | q, inc = wave_incl_scan_u32(mine);
-            u32 gb = gr + ((inc - mine) >> 16), qb = qr + ((inc - mine) & 0xFFFFu);
-#pragma unroll
-            for (u32 j = 0; j < 4; ++j) {
-                if (j >= m || x[j] < K0) continue;
-                if (x[j] > K0 || qb < ties) {
-                    const u32 p = gb + min(qb, ties);
-                    if (out_keys && p < k) out_keys[p] = K::from_ord(x[j]);
-                    if (out_idx && p < k) out_idx[p] = (i64)si[i + j];
-                }
-                gb += x[j] > K0 ? 1u : 0u;
-                qb += x[j] == K0 ? 1u : 0u;
-            }
-            const u32 all = (u32)__builtin_amdgcn_readlane((int)inc, WAVE - 1);
-            gr += all >> 16;
-            qr += all & 0xFFFFu;
-        });
-    }
+    write_segments(K0, ties, w, SH_NT / WAVE);
 }
 
 u32 short_segments(u64 V) { return (u32)((V + COLLECT_TILE - 1) / COLLECT_TILE); }
@@ -595,12 +698,14 @@ hipError_t launch_short(const ShortArgs& a, hipStream_t st) {
     else FI_LAUNCH(SMALL_N, 0);
 #undef FI_LAUNCH
     const bool out = a.out_keys || a.out_idx;
+    // a wave per segment, where there can be more keys than one workgroup holds
+    const u32 fin = V <= FIN_CAP ? 1 : std::min(FIN_WGS, (nseg + SH_NT / WAVE - 1) / (SH_NT / WAVE));
 #define CO_LAUNCH(K, I)                                                                                               \
     hipLaunchKernelGGL((k_collect<K, I>), dim3(nseg), dim3(WG), 0, st, a.keys, (u32)a.n, a.alpha, a.sel_ids, (u32)a.k, \
                        a.ctrl, a.skeys, a.sidx, a.cnt, a.segmax, a.ghist)
 #define FN_LAUNCH(K)                                                                                                  \
-    hipLaunchKernelGGL((k_final<K>), dim3(1), dim3(SH_NT), 0, st, a.skeys, a.sidx, a.cnt, a.segmax, a.ghist, nseg, \
-                       (u32)a.k, a.ctrl, (u32*)a.out_keys, a.out_idx, (u32*)a.d_kth)
+    hipLaunchKernelGGL((k_final<K>), dim3(fin), dim3(SH_NT), 0, st, a.skeys, a.sidx, a.cnt, a.segmax, a.ghist, nseg, \
+                       (u32)a.k, a.ctrl, a.rcnt, (u32*)a.out_keys, a.out_idx, (u32*)a.d_kth)
     if (a.f32) {
         if (out) CO_LAUNCH(KeyF32, true); else CO_LAUNCH(KeyF32, false);
         FN_LAUNCH(KeyF32);

@@ -1,6 +1,7 @@
 """GPU test of the short pipeline's second top-k on inputs that single out one branch of it each: sparse
 keys, whose k-th key lies in the bucket that starts at the lowest key of all, ties that fill the k-th key's
-bucket of a concatenation held in LDS, and one value that most keys share.  Outputs must equal the
+bucket of a concatenation held in LDS, concatenations that LDS does not hold, reduced by one workgroup or
+several, with every way to go on from there, and one value that most keys share.  Outputs must equal the
 oracle's and the general pipeline's (the same call with stats) bit for bit."""
 import numpy as np
 import pytest
@@ -49,6 +50,46 @@ def test_tied_bucket(orc, dt, f32, n, k):  # noqa: F811
         v[tie:tie + 3 * k // 4] = np.uint32((1 << 30) + 12345)
         print(f"[case] tied bucket n={n} k={k} f32={f32} seed={seed}", flush=True)
         check(orc, dt, as_keys(orc, v, f32), f32, k, dt.ALGO_RADIX)
+
+
+def clustered(kind, n, k, seed):
+    """Ordered keys whose k selected subranges hold far more keys >= the threshold than k."""
+    rng = np.random.default_rng(seed)
+    v = rng.integers(0, 1 << 20, n, dtype=np.uint32)
+    lo, hi = n // 3, n // 3 + n // 16
+    if kind == "scatter":  # fewer than k keys above the threshold, in as many segments
+        v[:] = 0
+        v[rng.integers(0, n, k // 2)] = rng.integers(1, 1 << 31, k // 2, dtype=np.uint32)
+    elif kind == "ascending":
+        v = np.arange(n, dtype=np.uint32) * np.uint32(5)
+    elif kind == "saw":
+        v = np.arange(n, dtype=np.uint32) % np.uint32(100_003)
+    elif kind == "block":
+        v[lo:hi] += np.uint32(1 << 21)
+    elif kind == "block+outlier":  # logarithmic buckets
+        v[lo:hi] += np.uint32(1 << 21)
+        v[5] = np.uint32(2 ** 32 - 1)
+    elif kind == "constant":  # the k-th key's bucket is one value
+        v[lo:hi] = np.uint32(1 << 21)
+    elif kind == "constant+above":
+        v[lo:hi] = np.uint32(1 << 21)
+        v[rng.integers(0, n, k // 3)] = np.uint32(3 << 20) + rng.integers(0, 1 << 19, k // 3, dtype=np.uint32)
+    else:
+        assert kind == "narrow"  # three values in it, each many times, and keys far above
+        v[lo:hi] = np.uint32(1 << 29) + rng.integers(0, 3, hi - lo, dtype=np.uint32)
+        v[rng.integers(0, n, k // 3)] = np.uint32(1 << 31) + rng.integers(0, 1 << 30, k // 3, dtype=np.uint32)
+    return v
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,k", [((1 << 20) + 3, 4096), ((1 << 22) + 1, 6000), ((1 << 24) + 5, 4096)])
+@pytest.mark.parametrize("kind", ["scatter", "ascending", "saw", "block", "block+outlier", "constant", "constant+above",
+                                  "narrow"])
+def test_long_concatenations(orc, dt, kind, n, k, f32):  # noqa: F811
+    assert dt.select_route(n, k)["pipeline"] == "short"
+    v = clustered(kind, n, k, n)
+    print(f"[case] concatenation {kind} n={n} k={k} f32={f32}", flush=True)
+    check(orc, dt, as_keys(orc, v, f32), f32, k, dt.ALGO_RADIX)
 
 
 @pytest.mark.parametrize("n,k", [(257, 100), (4096, 1000), (36_864, 30_000), (300_001, 2_000)])
