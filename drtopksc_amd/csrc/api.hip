@@ -353,6 +353,11 @@ int pick_pipeline(const Plan& pl, char* ws, ShortPlan* sp, FilterArgs* fa) {
     if (!pl.own_config || pl.algo == DRTOPK_ALGO_BITONIC || g_test_segcap.load(std::memory_order_relaxed) != 0)
         return DRTOPK_PIPELINE_GENERAL;
     if (pl.n <= SMALL_N) return DRTOPK_PIPELINE_SMALL;
+    // Where both fit, the filter pipeline takes k above 7168 of 2^24 keys and more (short -> filter, us, random
+    // uint32; ascending; a sixteenth of the keys large in one block): 2^24, 8192: 74 -> 62; 97 -> 69; 106 -> 57.
+    // 2^26, 8192: 114 -> 112; 152 -> 129; 136 -> 104.  Random keys are quicker with the short one at smaller k
+    // (2^26, 6200: 101 and 112) and below 2^24 keys (2^21, 7000: 41 and 52; 2^20, 6200: 40 and 45).
+    if (pl.k > 7168 && pl.n >= (1ull << 24) && filter_plan(pl, fa, ws)) return DRTOPK_PIPELINE_FILTER;
     if (short_plan(pl, sp)) return DRTOPK_PIPELINE_SHORT;
     return filter_plan(pl, fa, ws) ? DRTOPK_PIPELINE_FILTER : DRTOPK_PIPELINE_GENERAL;
 }

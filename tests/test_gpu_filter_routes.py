@@ -25,7 +25,7 @@ def filtered(dt, v, f32, k):  # noqa: F811
 
 
 @pytest.mark.parametrize("n,k,lm", [(65_537, 8_192, 13), (73_737, 9_217, 13), (1_000_003, 125_000, 13),
-                                    (2_400_003, 8_500, 15), ((1 << 24) + 5, 1 << 22, 13), (40_000_003, 9_300, 17)])
+                                    ((1 << 24) + 3, 8_000, 17), ((1 << 25) + 1, 7_169, 19), (2_400_003, 8_500, 15), ((1 << 24) + 5, 1 << 22, 13), (40_000_003, 9_300, 17)])
 @pytest.mark.parametrize("dist", ["uniform", "f32"])
 def test_edges_in_k(orc, dt, dist, n, k, lm):  # noqa: F811
     v, f32 = make(orc, dist, n, 61)

@@ -24,6 +24,8 @@ ROUTES = [
     (2_400_003, 8_500, -1, "filter", 15), (2_400_003, 9_000, -1, "filter", 13),
     (1 << 24, 1 << 22, -1, "filter", 13), (1 << 24, (1 << 22) + 1, -1, "general", 0),  # k = n / 4, above
     (40_000_003, 9_000, -1, "filter", 19), (40_000_003, 9_300, -1, "filter", 17), (1 << 28, 1 << 16, -1, "filter", 17), (1 << 30, 1 << 16, -1, "filter", 19),
+    (1 << 26, 7168, -1, "short", 0), (1 << 26, 7169, -1, "filter", 19), ((1 << 24) - 1, 8192, -1, "short", 0),
+    (1 << 20, 8192, -1, "short", 0), (1 << 24, 8192, -1, "filter", 17),
     (1 << 30, 1 << 28, -1, "filter", 15), ((1 << 30) + 1, 1 << 20, -1, "general", 0),
 ]
 
