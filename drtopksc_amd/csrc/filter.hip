@@ -47,7 +47,9 @@ constexpr u32 F_BATCH = WG * 8; // kept keys a workgroup takes at a time in k_fp
 // (2^28 keys, the top ones 1 in 256 of a sixteenth: 380 us for the call, 219 in batches).
 constexpr u32 DENSE_UNIT = 256, DENSE_RANGE = 2 * F_BATCH;
 constexpr u32 DENSE_ENTRY = 0x80000000u;  // a class entry of a dense range names its unit, others their range
-constexpr u32 F_SORT = 512;       // samples above the bound that are put in order at once
+// Samples above the bound that are put in order at once, each compared with all.  482 of them (k = n / 24 below 2^26
+// keys) took the kernel 21 us, the selections and the sort of the splitters alone 14; 353 of them 16 and 15.
+constexpr u32 F_SORT = 320;
 constexpr u32 F_STAGE = 512;    // kept keys a wave stages in LDS
 constexpr u32 F_LISTS = 64;     // sublists of the class, so that their cursors do not serialise
 
