@@ -268,25 +268,25 @@ __global__ __launch_bounds__(WG) void k_collect(const u32* __restrict__ keys, u3
     u32 tot;  // survivors | keys equal to T << 16, at most 4096 each
     u32 slot = block_excl_scan_u32<WG>((u32)__popc(take) | (eq << 16), scratch, &tot) & 0xFFFFu;
     const u32 base = blockIdx.x * COLLECT_TILE;
-    u32 cur = 0, run = 0;  // sorted keys: a thread's run in one bucket with one atomic
+    bool one = false;  // sorted or tied keys: the thread's are all in one bucket
+    if (take == 0xFFFFu) {
+        u32 mn = r[0][0];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) mn = min(min(mn, min(r[q][0], r[q][1])), min(r[q][2], r[q][3]));
+        const u32 b = mn != T ? bk.of(mn - T) : 0u;
+        one = b ? b == bk.of(mx - T) : mx == T;
+        if (one && b) atomicAdd(&lh[b], 16u);
+    }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         if (take & (1u << j)) {
             const u32 o = r[j >> 2][j & 3];
             skeys[base + slot] = o;
             if (IDX) sidx[base + slot] = g[j >> 2] + (u32)(j & 3);
+            if (!one && o != T) atomicAdd(&lh[bk.of(o - T)], 1u);
             ++slot;
-            if (o == T) continue;
-            const u32 b = bk.of(o - T);
-            if (b != cur) {
-                if (cur) atomicAdd(&lh[cur], run);
-                cur = b;
-                run = 0;
-            }
-            ++run;
         }
     }
-    if (cur) atomicAdd(&lh[cur], run);
     mx = wave_max_last(mx);
     if ((threadIdx.x & (WAVE - 1)) == WAVE - 1) wmax[threadIdx.x / WAVE] = mx;
     __syncthreads();
