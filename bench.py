@@ -6,9 +6,9 @@ reference's final configuration (FILTER|BETA|SHUFFLE, 8-bit digits, beta 2, auto
 each call returning the k-th key, the top-k keys and their int64 indices.
 value = keys examined per second over the sweep (25 * 2^30 / step time), in Gelem/s.
 
-Printed as one JSON line; besides the headline it carries the per-k times with two %HBM
-figures, the HBM roofline of the dominant kernel (the delegate pass), the other single-vector
-workloads (bucket family, normal and log-normal keys, float32 2^28 with the bitonic family,
+Printed as one JSON line; besides the headline it carries the per-k times with the pipeline each call
+takes and the fraction of the HBM peak its bytes come to, the HBM roofline of the dominant kernel (the
+delegate pass), the other single-vector workloads (bucket family, normal and log-normal keys, float32 2^28 with the bitonic family,
 the plain radix select, the option ablation, the bitonic reference points), the batched and
 served forms, and the OpenMP CPU baseline timed on this host for each key distribution.
 """
@@ -46,10 +46,8 @@ REF_ABLATION_2P29_K2P24_MS = {  # baseline{,+filter,+filter+shuffle}/U_OptimumFI
     "baseline": 53.29, "filter": 36.81, "filter+shuffle": 28.46}
 
 
-def bytes_build(st: dict, n: int, k: int) -> int:
-    """The general pipeline's algorithmic bytes for one top-k: what each pass must move at least.  (The
-    statistics are that pipeline's; a timed call asks for none and may take a shorter pipeline, which
-    moves fewer bytes for the same result.)
+def bytes_general(st: dict, n: int, k: int) -> int:
+    """The general pipeline's algorithmic bytes for one top-k: what each pass must move at least.
     - 4n: the delegate pass reads V once;
     - 4D: the delegate write;
     - 4D per first-top-k pass that reads the delegates (digit passes after the first, whose
@@ -64,8 +62,25 @@ def bytes_build(st: dict, n: int, k: int) -> int:
     return 4 * n + 4 * D + 4 * D * p1 + 4 * st["selected_subranges"] * L + 8 * C + 4 * C * p2 + 12 * k
 
 
+def bytes_moved(route: dict, st: dict, n: int, k: int) -> int:
+    """Bytes that the pipeline of a call without statistics (drtopk_select_route) must move at least.  `st` holds
+    the statistics of another call on the same keys, which always takes the general pipeline.
+    - small: the keys and the outputs;
+    - short: 4n, the delegates written and read (8D), the selected subranges' keys read, their concatenation
+      (k entries at least) written and read with its indices (16k), 12k out;
+    - filter: 4n, 12k out, and for every key above the k-th (all of them are kept) 8 bytes written, 4 read to
+      pick the k-th key's class and 8 read for the outputs."""
+    if route["pipeline"] == "general":
+        return bytes_general(st, n, k)
+    if route["pipeline"] == "short":
+        return 4 * n + 8 * route["delegates"] + 4 * min(route["slots"], n) + 16 * k + 12 * k
+    if route["pipeline"] == "filter":
+        return 4 * n + 20 * st["count_greater"] + 12 * k
+    return 4 * n + 12 * k
+
+
 def bytes_survey(st: dict, n: int, k: int) -> int:
-    """The byte formula as the hot-path scope states it: 4n + 4D + 4D*p1 (p1 = digit passes
+    """The byte formula as the hot-path scope states it, for calls that take the general pipeline: 4n + 4D + 4D*p1 (p1 = digit passes
     + 1 selection pass) + 4*S_sel*2^alpha + 4C + 4C*p2 (p2 = second-top-k passes) + 12k."""
     D, C, L = st["num_delegates"], st["concat_size"], 1 << st["alpha"]
     p1 = st["first_passes"] + 1
@@ -84,6 +99,32 @@ def checks_clean(dt, ws) -> bool:
 
 def frac(nbytes: float, ms: float) -> float:
     return round(nbytes / (ms * 1e-3) / (HBM_PEAK_GBS * 1e9), 4)
+
+
+def row(route: dict, st: dict, n: int, k: int, ms: float, ref=None) -> dict:
+    """One timed call: its pipeline, the fraction of the HBM peak that its bytes and the keys alone come to, and
+    under "stats_call" what the call with statistics, on the general pipeline, reports."""
+    r = {"k": k, "pipeline": route["pipeline"], "ms": round(ms, 4), "gelem_s": round(n / (ms * 1e-3) / 1e9, 1),
+         "hbm_frac": frac(bytes_moved(route, st, n, k), ms), "hbm_frac_4n": frac(4 * n, ms)}
+    if route["pipeline"] == "general":
+        r["hbm_frac_survey"] = frac(bytes_survey(st, n, k), ms)
+    if ref and k in ref:
+        r["ref_v100s_ms"] = ref[k]
+    r["stats_call"] = {"alpha": st["alpha"], "path": st["path"], "concat": st["concat_size"],
+                       "phase_ms": [round(x, 4) for x in st["phase_ms"]]}
+    return r
+
+
+def brief(x):
+    """A record for the printed line: a list of rows becomes [k, ms] pairs, of a sweep over the powers of two ms
+    alone (the full record goes to --detail)."""
+    if isinstance(x, list) and x and isinstance(x[0], dict) and "ms" in x[0]:
+        if len(x) > 8 and all(r["k"] == x[0]["k"] << i for i, r in enumerate(x)):
+            return [round(r["ms"], 3) for r in x]
+        return [[r["k"], round(r["ms"], 3)] for r in x]
+    if isinstance(x, dict):
+        return {k: brief(v) for k, v in x.items()}
+    return x
 
 
 class Runner:
@@ -124,24 +165,18 @@ class Runner:
         return e0.elapsed_time(e1) / reps
 
     def sweep(self, dev, ks, algo=0, p=None, reps=5, ref=None):
-        """Per-k stats (one synchronised call) and event-timed ms (reps calls), with both %HBM
-        figures and the conservative 4n one."""
+        """Event-timed ms per k (reps calls without statistics), the pipeline those calls take, and the
+        statistics of one more call."""
         dt = self.dt
         n = dev.numel()
         p = p or dt.params()
-        self.reserve(max(dt.workspace_size(n, k, algo, dt.F32 if dev.dtype == self.torch.float32 else dt.U32, p)
-                         for k in ks))
+        dtype = dt.F32 if dev.dtype == self.torch.float32 else dt.U32
+        self.reserve(max(dt.workspace_size(n, k, algo, dtype, p) for k in ks))
         rows = []
         for k in ks:
             _, _, _, st = self.call(dev, k, algo, p, stats=True)
             ms = self.time_ms(lambda: self.call(dev, k, algo, p), reps)
-            r = {"k": k, "alpha": st["alpha"], "path": st["path"], "ms": round(ms, 4),
-                 "gelem_s": round(n / (ms * 1e-3) / 1e9, 1), "hbm_frac": frac(bytes_build(st, n, k), ms),
-                 "hbm_frac_survey": frac(bytes_survey(st, n, k), ms), "hbm_frac_4n": frac(4 * n, ms),
-                 "concat": st["concat_size"]}
-            if ref and k in ref:
-                r["ref_v100s_ms"] = ref[k]
-            rows.append(r)
+            rows.append(row(dt.select_route(n, k, algo, dtype, p), st, n, k, ms, ref))
         return rows
 
     def kth_u32(self) -> int:
@@ -441,6 +476,7 @@ def main():
     ap.add_argument("--legs", default="sweep,configs,batched,served",
                     help="comma list of sweep, configs, batched, served (profiling runs pick one)")
     ap.add_argument("--served-requests", type=int, default=2000)
+    ap.add_argument("--detail", help="also write the full record (every row's statistics and fractions) to this file")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py runs on one GPU only (asked for --gpus {args.gpus}); the multi-GPU exchange is "
@@ -501,16 +537,8 @@ def main():
     value = len(ks) * n / (ms_step * 1e-3) / 1e9
     device_ok = checks_clean(dt, R.ws)  # device-side checks of every call above
 
-    rows = []
-    for k, st, ms in zip(ks, per_k, k_ms):
-        r = {"k": k, "alpha": st["alpha"], "path": st["path"], "ms": round(ms, 4),
-             "gelem_s": round(n / (ms * 1e-3) / 1e9, 1),
-             "hbm_frac": frac(bytes_build(st, n, k), ms), "hbm_frac_survey": frac(bytes_survey(st, n, k), ms),
-             "hbm_frac_4n": frac(4 * n, ms), "concat": st["concat_size"],
-             "phase_ms": [round(x, 4) for x in st["phase_ms"]]}
-        if args.log2n == 30 and k in REF_RADIX_UNIFORM_MS:
-            r["ref_v100s_ms"] = REF_RADIX_UNIFORM_MS[k]
-        rows.append(r)
+    rows = [row(dt.select_route(n, k), st, n, k, ms, REF_RADIX_UNIFORM_MS if args.log2n == 30 else None)
+            for k, st, ms in zip(ks, per_k, k_ms)]
     # roofline of the dominant kernel: the delegate pass (phase 0), k = 2^10 (alpha 11)
     ref_i = ks.index(1 << 10) if (1 << 10) in ks else 0
     st_ref = per_k[ref_i]
@@ -551,12 +579,13 @@ def main():
     batched = None
     if not args.no_batched:
         batched = batched_leg(dt, torch, args.steps, args.warmup, nrows=args.batch_rows)
-        print(f"[bench] batched {batched}", file=sys.stderr, flush=True)
+        print(f"[bench] batched {batched['ms']} ms", file=sys.stderr, flush=True)
     served = None
     if not args.no_served:
         served = served_leg(dt, torch, nreq=args.served_requests)
-        print(f"[bench] served {served}", file=sys.stderr, flush=True)
+        print(f"[bench] served {served['served_saturated']['req_s']} req/s", file=sys.stderr, flush=True)
 
+    survey = [r["hbm_frac_survey"] for r in rows if "hbm_frac_survey" in r]
     out = {
         "metric": METRIC, "value": round(value, 2), "unit": "Gelem/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": round(ms_step, 4), "higher_is_better": True, "scaling": "weak",
@@ -567,10 +596,18 @@ def main():
                    "digit_bits": 8, "beta": 2, "alpha": "auto (reference policy)"},
         "roofline": roofline, "cpu_baseline": cpu, "host": host,
         "min_hbm_frac": min(r["hbm_frac"] for r in rows),
-        "min_hbm_frac_survey": min(r["hbm_frac_survey"] for r in rows),
+        "min_hbm_frac_survey": min(survey) if survey else None,  # calls on the general pipeline
         "device_checks_clean": device_ok,
         "per_k": rows, "configs": configs, "batched": batched, "served": served, "wall_s": round(wall, 3),
     }
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(out, f, indent=1)
+    # the line stays short enough to be kept whole by whatever keeps the end of the output
+    out["per_k"] = [[r["k"], r["pipeline"], r["ms"], r["hbm_frac"]] for r in rows]
+    out["configs"] = brief(configs)
+    if served:
+        out["served"] = {k: v for k, v in served.items() if k != "saturated_by_max_inflight"}
     print(json.dumps(out))
 
 
