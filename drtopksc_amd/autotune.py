@@ -9,8 +9,8 @@ range (n 2^12..2^22, k 1..4096) it builds a batch of `rows` rows of that type wh
 in that cell, times drtopk_select_batched (HIP events on the launch stream, median of `reps`)
 for each candidate, checks that every candidate returns the same outputs, and keeps the fastest.
 Candidates: alpha in policy-2 .. policy+2 (the planner lowers invalid ones), tiles of 2^13 or
-2^15 keys (the digit width no longer matters to the batched kernels and stays 8).  Rows of one cell share a batch, so a cell's time is its
-throughput when batched with its own kind.
+2^15 keys.  Rows of one cell share a batch, so a cell's time is its throughput when batched with its
+own kind.
 
 The result is JSON: {"device": ..., "cells": [[dtype, log2n, log2k, alpha, digit_bits, tile_log2], ...]};
 drtopksc_amd.tuning_from_table() turns it into a drtopk_tuning, and
@@ -31,6 +31,9 @@ import json
 import os
 import sys
 import time
+
+
+DIGIT_BITS = 8  # of every cell: no kernel of the batched form depends on it
 
 
 def policy_alpha(n: int, k: int) -> int:
@@ -91,9 +94,22 @@ SINGLE_JSON = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning",
 SINGLE_INC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "single_tuning.inc")
 
 
+def single_candidates(dt, n: int, k: int):
+    """(alpha, beta, params) to time for one cell of the single-vector table, the reference policy first.  All
+    name their alpha: a call that leaves it to the library takes a pipeline that the table does not steer."""
+    pol = min(policy_alpha(n, k), n.bit_length() - 1)
+    out = [(pol, 2 if 0 < pol <= 5 else 1, dt.params(alpha=pol))]
+    for a in range(max(1, pol - 2), min(n.bit_length() - 1, pol + 2) + 1):
+        for b in ((1, 2, 3, 4) if a <= 5 else (1,)):
+            fl = dt.FLAGS_DEFAULT if b > 1 else (dt.FLAG_FILTER | dt.FLAG_SHUFFLE)
+            if (a, b) != out[0][:2]:
+                out.append((a, b, dt.params(alpha=a, beta=max(b, 2), flags=fl)))
+    return out
+
+
 def tune_single(lns, kmax_log2: int, reps: int, margin: float, out_path: str) -> int:
-    """The single-vector table (DRTOPK_ALPHA_TUNED): for n = 2^ln uniform uint32 keys and every
-    k = 2^lk, time drtopk_select (keys + indices out, HIP events, median of `reps`) for alpha in
+    """The single-vector table (DRTOPK_ALPHA_TUNED), which the general pipeline follows: for n = 2^ln
+    uniform uint32 keys and every k = 2^lk, time drtopk_select (keys + indices out, HIP events, median of `reps`) for alpha in
     policy-2 .. policy+2 and, at alpha <= 5, beta 1 (one delegate) .. 4; every candidate must
     return the reference policy's outputs.  A cell keeps the fastest candidate when it beats the
     policy by more than `margin`, else the policy."""
@@ -114,15 +130,9 @@ def tune_single(lns, kmax_log2: int, reps: int, margin: float, out_path: str) ->
         ws = torch.empty(256, dtype=torch.uint8, device="cuda")
         for lk in range(0, min(kmax_log2, ln - 4) + 1):
             k = 1 << lk
-            pol = policy_alpha(n, k)
-            cands = []
-            for a in range(max(1, pol - 2), min(ln, pol + 2) + 1):
-                for b in ((1, 2, 3, 4) if a <= 5 else (1,)):
-                    fl = dt.FLAGS_DEFAULT if b > 1 else (dt.FLAG_FILTER | dt.FLAG_SHUFFLE)
-                    cands.append((a, b, dt.params(alpha=a, beta=max(b, 2), flags=fl)))
             res = {}
             ref = None
-            for a, b, p in [(-1, 0, dt.params())] + cands:
+            for a, b, p in single_candidates(dt, n, k):
                 try:
                     need = dt.workspace_size(n, k, dt.ALGO_RADIX, dt.U32, p)
                 except dt.DrTopKError:
@@ -132,7 +142,7 @@ def tune_single(lns, kmax_log2: int, reps: int, margin: float, out_path: str) ->
                     torch.cuda.empty_cache()
                     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
                 o = (kth, okeys[:k], oidx[:k])
-                _, _, _, stt = dt.select(dev, k, p=p, workspace=ws, out=o, stats=True)
+                dt.select(dev, k, p=p, workspace=ws, out=o, stats=True)
                 got = [x.clone() for x in o]
                 if ref is None:
                     ref = got
@@ -147,9 +157,8 @@ def tune_single(lns, kmax_log2: int, reps: int, margin: float, out_path: str) ->
                     e1.synchronize()
                     ts.append(e0.elapsed_time(e1))
                 ts.sort()
-                key = (stt["alpha"], stt["beta"]) if a < 0 else (a, b)
-                res[key] = min(res.get(key, 1e9), ts[len(ts) // 2])
-            pol_key = next(iter(res))  # the policy's resolved (alpha, beta) was timed first
+                res[a, b] = ts[len(ts) // 2]
+            pol_key = next(iter(res))  # the policy was timed first
             best = min(res.items(), key=lambda kv: kv[1])
             pick = best[0] if best[1] < res[pol_key] * (1.0 - margin) else pol_key
             cells.append([ln, lk, pick[0], pick[1]])
@@ -249,21 +258,20 @@ def main(argv=None):
                 best = None
                 ref = None
                 for a in range(max(0, a0 - 2), a0 + 3):
-                    for nb in (8,):  # no kernel of the batched form depends on it
-                        for tl in (13, 15):
-                            if a > tl:
-                                continue
-                            t = dt.tuning_default()
-                            t.alpha[dtype][ln][lk] = a
-                            t.digit_bits[dtype][ln][lk] = nb
-                            t.tile_log2[dtype][ln][lk] = tl
-                            ms, out = time_batch(dt, torch, rows, buf, keys_len, out_len, t, args.reps)
-                            if ref is None:
-                                ref = [o.clone() for o in out]
-                            elif not all(torch.equal(x, y) for x, y in zip(out, ref)):
-                                raise RuntimeError(f"cell ({dtype},{ln},{lk}) alpha {a} nb {nb} tile {tl}: outputs differ")
-                            if best is None or ms < best[0]:
-                                best = (ms, a, nb, tl)
+                    for tl in (13, 15):
+                        if a > tl:
+                            continue
+                        t = dt.tuning_default()
+                        t.alpha[dtype][ln][lk] = a
+                        t.digit_bits[dtype][ln][lk] = DIGIT_BITS
+                        t.tile_log2[dtype][ln][lk] = tl
+                        ms, out = time_batch(dt, torch, rows, buf, keys_len, out_len, t, args.reps)
+                        if ref is None:
+                            ref = [o.clone() for o in out]
+                        elif not all(torch.equal(x, y) for x, y in zip(out, ref)):
+                            raise RuntimeError(f"cell ({dtype},{ln},{lk}) alpha {a} tile {tl}: outputs differ")
+                        if best is None or ms < best[0]:
+                            best = (ms, a, DIGIT_BITS, tl)
                 cells.append([dtype, ln, lk, best[1], best[2], best[3]])
                 report.append({"dtype": dtype, "log2n": ln, "log2k": lk, "policy_alpha": a0, "alpha": best[1],
                                "digit_bits": best[2], "tile_log2": best[3], "ms": round(best[0], 4), "rows": len(rows)})

@@ -56,3 +56,17 @@ def test_arguments(dt):
             dt.select_route(n, k)
     p = dt.params()
     assert dt.lib().drtopk_select_route(0, 0, 100, 10, ctypes.byref(p), None, None, None) == 1
+
+
+def test_autotuner_times_the_pipeline_it_tunes(dt):
+    """Every candidate of the single-vector table, the reference policy's too, runs on the general pipeline."""
+    from drtopksc_amd import autotune
+    for n, k in ((1 << 16, 1), (1 << 16, 1 << 12), (1 << 20, 8), (1 << 22, 1 << 10), (1 << 24, 1 << 20), (1 << 30, 1 << 16)):
+        cands = autotune.single_candidates(dt, n, k)
+        assert cands[0][0] == autotune.policy_alpha(n, k) and len({c[:2] for c in cands}) == len(cands)
+        for a, b, p in cands:
+            try:
+                r = dt.select_route(n, k, p=p)
+            except dt.DrTopKError:
+                continue  # fewer delegates than k: the tuner leaves it out too
+            assert r["pipeline"] == "general" and r["alpha"] == a
