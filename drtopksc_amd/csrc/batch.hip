@@ -67,7 +67,7 @@ struct BatchRow {
                     // and as many row indices
     u32 S;          // subranges (0 when alpha == 0)
     u32 chunk_begin, nchunks;
-    u8 alpha, f32, nb, tile_log2;  // nb: as tuned, no kernel depends on it
+    u8 alpha, f32, nb, tile_log2;  // nb: as tuned, part of the plan's layout; no kernel reads it
 };
 static_assert(sizeof(BatchRow) == 64, "row layout");
 
@@ -88,21 +88,6 @@ constexpr int MAX_TILE_LOG2 = 15;
 template <bool F32>
 __device__ __forceinline__ u32 ord(u32 b) {
     return F32 ? KeyF32::to_ord(b) : b;
-}
-
-// Maximum over each aligned group of g lanes (g = 1, 2, 4, .., 64, uniform over the wave),
-// complete in the group's last lane, with DPP moves alone: quad permutes and the half-row / row
-// mirrors give every lane of a 16-lane row its row's maximum, row broadcast 15 then carries row 0
-// into row 1 and row 2 into row 3 (32-lane groups), and row broadcast 31 row 1 into rows 2 and 3
-// (the whole wave).
-__device__ __forceinline__ u32 group_max_last(u32 m, int g) {
-    if (g >= 2) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
-    if (g >= 4) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
-    if (g >= 8) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xF, 0xF, false));  // row_half_mirror
-    if (g >= 16) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x140, 0xF, 0xF, false)); // row_mirror
-    if (g >= 32) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x142, 0xA, 0xF, false));  // row_bcast:15
-    if (g >= 64) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x143, 0xC, 0xF, false));  // row_bcast:31
-    return m;
 }
 
 constexpr u32 BS_WKEYS = BS_UNR * WAVE * 4;  // keys per wave per batch (2048)

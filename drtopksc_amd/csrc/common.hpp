@@ -164,6 +164,26 @@ __device__ __forceinline__ u32 wave_incl_scan_u32(u32 v) {
     return v;
 }
 
+// Maximum over aligned groups of g lanes (g <= 16, uniform) with DPP moves, in every lane of the group: quad
+// permutes, the half-row and the row mirror.
+__device__ __forceinline__ u32 row_max_u32(u32 m, int g) {
+    if (g >= 2) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+    if (g >= 4) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+    if (g >= 8) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    if (g >= 16) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x140, 0xF, 0xF, false)); // row_mirror
+    return m;
+}
+// The same for groups of up to 64 lanes, complete in the group's last lane: row broadcast 15 carries row 0 into
+// row 1 and row 2 into row 3 (32-lane groups), row broadcast 31 row 1 into rows 2 and 3 (the whole wave).
+__device__ __forceinline__ u32 group_max_last(u32 m, int g) {
+    m = row_max_u32(m, g);
+    if (g >= 32) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x142, 0xA, 0xF, false));  // row_bcast:15
+    if (g >= 64) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x143, 0xC, 0xF, false));  // row_bcast:31
+    return m;
+}
+// Maximum over the wave, in lane 63.
+__device__ __forceinline__ u32 wave_max_last(u32 m) { return group_max_last(m, WAVE); }
+
 // u64 sum over the 64 lanes of a wave (result in every lane).
 __device__ __forceinline__ u64 wave_sum_u64(u64 v) {
 #pragma unroll

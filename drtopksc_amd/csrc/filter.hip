@@ -75,7 +75,8 @@ struct FilterState {
 size_t filter_state_bytes() { return sizeof(FilterState) + 4ull * (F_REPS * F_CLASSES + 2 * F_RANGES); }
 
 // ---------------------------------------------------------------- sample
-// Sample i is a key of stratum [i n / m, (i + 1) n / m).
+// Sample i is a key of stratum [i n / m, (i + 1) n / m), at a place mixed from i by xorshifts and multiplications
+// with the shifts of xxHash's 32-bit finaliser and its first three primes.
 __host__ __device__ __forceinline__ u32 sample_pos(u32 i, u64 n, int lm) {
     const u32 b = (u32)(((u64)i * n) >> lm), e = (u32)(((u64)(i + 1) * n) >> lm);
     u32 h = i * 0x9E3779B1u;

@@ -221,20 +221,6 @@ __device__ __forceinline__ u32x4 load4(const u32x4* p) { return __builtin_nontem
 constexpr int GROUP_BATCHES = 8;                      // 16-byte loads in flight per lane
 constexpr int GROUP_CHUNK = GROUP_BATCHES * WG * 4;   // 8192 keys per workgroup chunk
 
-// Maximum over each aligned group of g lanes (g = 1, 2, .., 64, uniform) with DPP moves, complete
-// in the group's last lane: quad permutes and the half-row / row mirrors give every lane of a
-// 16-lane row its row's maximum, row broadcast 15 then carries row 0 into row 1 and row 2 into
-// row 3 (32-lane groups), and row broadcast 31 row 1 into rows 2 and 3 (the whole wave).
-__device__ __forceinline__ u32 group_max_last(u32 m, int g) {
-    if (g >= 2) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
-    if (g >= 4) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
-    if (g >= 8) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xF, 0xF, false));  // row_half_mirror
-    if (g >= 16) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x140, 0xF, 0xF, false)); // row_mirror
-    if (g >= 32) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x142, 0xA, 0xF, false));  // row_bcast:15
-    if (g >= 64) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x143, 0xC, 0xF, false));  // row_bcast:31
-    return m;
-}
-
 template <class K, int BETA, int POSM, int FUSE, class LT>
 __global__ __launch_bounds__(WG) void k_sample_groups(const u32* __restrict__ keys, u64 n, int alpha, int vec_ok,
                                                       u64 nchunks, u32* __restrict__ dvals, void* __restrict__ dpos,

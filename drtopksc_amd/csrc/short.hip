@@ -112,9 +112,7 @@ __global__ __launch_bounds__(WG) void k_super(const u32* __restrict__ dvals, u32
     u32 m = max4(load_padded(dvals, e, S));
     for (int level = 0; level < 2; ++level) {
         const int f = level ? f1 + f2 : f1, g = 1 << (f - 2);  // lanes per range; its last lane gets the maximum
-        m = row_max_u32(m, g);
-        if (g >= 32) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x142, 0xA, 0xF, false));  // row_bcast:15
-        if (g >= 64) m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x143, 0xC, 0xF, false));  // row_bcast:31
+        m = group_max_last(m, g);
         if ((lane & (g - 1)) == g - 1 && ((e >> f) << f) < S) (level ? sup2 : sup1)[e >> f] = m;
         if (f2 == 0) break;
     }

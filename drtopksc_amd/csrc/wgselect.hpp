@@ -33,21 +33,6 @@ struct WgSel {
     u32 hi;            // wg_kth: the largest key
 };
 
-// Maximum over aligned groups of g lanes (g <= 16), in every lane of the group.
-__device__ __forceinline__ u32 row_max_u32(u32 m, int g) {
-    if (g >= 2) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
-    if (g >= 4) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
-    if (g >= 8) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x141, 0xF, 0xF, false));  // row_half_mirror
-    if (g >= 16) m = max(m, (u32)__builtin_amdgcn_mov_dpp((int)m, 0x140, 0xF, 0xF, false)); // row_mirror
-    return m;
-}
-// Maximum over the wave, in lane 63.
-__device__ __forceinline__ u32 wave_max_last(u32 m) {
-    m = row_max_u32(m, 16);
-    m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x142, 0xA, 0xF, false));  // row_bcast:15
-    m = max(m, (u32)__builtin_amdgcn_update_dpp(0, (int)m, 0x143, 0xC, 0xF, false));  // row_bcast:31
-    return m;
-}
 __device__ __forceinline__ u32 max4(const u32x4& v) { return max(max(v[0], v[1]), max(v[2], v[3])); }
 
 // Exclusive prefix over the wave totals a[0..NT/64) (NT/64 <= 16) at wave w, and their sum, without
