@@ -104,3 +104,31 @@ def test_heavy_value(orc, dt, share, n, k):  # noqa: F811
     v[n // 2:n // 2 + 16] = 5
     print(f"[case] heavy value n={n} k={k} share={share}", flush=True)
     check(orc, dt, v, False, k, dt.ALGO_RADIX)
+
+
+def test_long_concatenations_in_a_graph(orc, dt):  # noqa: F811
+    """A captured call, replayed on keys that go through the several workgroups, through one and back: the
+    arrivals are counted anew in each replay."""
+    n, k = (1 << 22) + 1, 6000
+    vs = [clustered(kind, n, k, 3) for kind in ("block", "ascending", "scatter", "constant")]
+    dev = torch.from_numpy(vs[0].view(np.int32)).cuda()
+    ws = torch.empty(dt.workspace_size(n, k), dtype=torch.uint8, device="cuda")
+    out = (torch.empty(1, dtype=torch.int32, device="cuda"), torch.empty(k, dtype=torch.int32, device="cuda"),
+           torch.empty(k, dtype=torch.int64, device="cuda"))
+    print(f"[case] concatenation graph n={n} k={k}", flush=True)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        dt.select(dev, k, workspace=ws, out=out)
+    torch.cuda.current_stream().wait_stream(s)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        dt.select(dev, k, workspace=ws, out=out, stream=torch.cuda.current_stream())
+    for v in vs * 2:
+        dev.copy_(torch.from_numpy(v.view(np.int32)))
+        g.replay()
+        torch.cuda.synchronize()
+        K, keys, idx = orc.topk_reference(v, k)
+        assert int(out[0].cpu().numpy().view(np.uint32)[0]) == K
+        assert np.array_equal(out[1].cpu().numpy().view(np.uint32), keys)
+        assert np.array_equal(out[2].cpu().numpy(), idx)
