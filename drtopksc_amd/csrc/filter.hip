@@ -17,13 +17,14 @@
 //  k_fkth     the k-th key, and where each range's outputs start.
 //  k_fwrite   the outputs in index order; ties at t are read from the keys again.
 //
-// At 2^30 keys, k = 2^22, the six take 6 + 30 + 738 + 25 + 17 + 29 us (1028 us for the general
-// pipeline, 856 for the call); the read alone takes 630.  At 2^24 keys, k = 2^16: 3 + 9 + 21 + 8 + 14 + 5 us
-// (67 and 63 for the calls): there the launches, and the chains of round trips in the two
+// At 2^30 keys, k = 2^22, the six take 7 + 29 + 735 + 22 + 20 .. 38 + 27 us (1028 us for the general
+// pipeline, 855 for the call); the read alone takes 630.  At 2^24 keys, k = 2^16: 3 + 9 + 21 + 8 + 16 + 6 us
+// (67 and 61 for the calls): there the launches, and the chains of round trips in the two
 // one-workgroup kernels, are most of it.
 //
 // Should the bound fail after all, or a buffer not hold what it was sized for, k_fkth selects from
-// the keys themselves with its one workgroup: slow, but exact.
+// the keys themselves with its one workgroup: slow (25 ms at 2^25 keys, 438 at 2^28), but exact.
+// drtopk_select_route tells from the workspace that a call ended there.
 #include <algorithm>
 #include <cstddef>
 #include <type_traits>
